@@ -743,6 +743,13 @@ hipError_t launch_project_tile(const ProjCommon& c, const CullParams& cp, const 
                                hipStream_t stream) {
     if (nchunks == 0) return hipSuccess;
     float* bins = static_cast<float*>(bins_v);
+    if (cfg.range.recs) {
+        if (cfg.range.sort) {
+            const hipError_t e = launch_range_sort(c, *fixed, cfg.range, stream);
+            if (e != hipSuccess || cfg.range.sort == 2) return e;
+        }
+        return launch_project_range(c, cp, cfg.range, bins, phase, lut, cfg.atomic, cfg.stats, stream);
+    }
 #define BCSIM_TILE(A, P, U) \
     return launch_tile_kind<A, P, U>(c, cp, fixed, spline, boxes, nchunks, bins, shared_origin, cfg, stream)
     if (arc) {

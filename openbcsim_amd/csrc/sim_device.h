@@ -193,6 +193,51 @@ struct CullParams {
     float lut_dl, lut_de;     // LUT grid spacing, 0 for a degenerate table (weight cutoff: records to metres)
 };
 
+// ---- projection in range order (project_range.hip) ----
+
+constexpr int kRangeBins = kMaxFftLen;  // bins a sorted set covers: those of the longest line
+constexpr int kRangePatch = 64;         // lines of a patch: one per lane of a wave
+
+// One point of a sorted set: its position from the common origin, its distance and
+// bin, and the phase rotation of its sub-sample delay.
+struct alignas(32) RangeRec {
+    float dx, dy, dz, amp;
+    float absd;
+    int bin;
+    float co, si;
+};
+
+// Up to kRangePatch lines near one another in direction, and the axes about which
+// their directions differ by at most (dr, dl, de) in norm.
+struct alignas(16) RangePatch {
+    float rx, ry, rz, dr;
+    float lx, ly, lz, dl;
+    float ex, ey, ez, de;
+    int n;                    // lines; k >= n repeats line[0]
+    int pad[3];
+    int line[kRangePatch];
+    float axes[6][kRangePatch];  // lateral x, y, z and elevational x, y, z of each line
+};
+
+struct RangeLaunch {
+    RangeRec* recs;           // points sorted by bin, or null: the tile kernel runs
+    int* start;               // [kRangeBins + 1]: first record of each bin
+    int* rank;                // [n] scratch of the sort
+    const RangePatch* patches;
+    int n_patches;
+    const float* table;       // the lookup table as [r][e][l], or null
+    int max_slices;           // radial slices of it that a window can need
+    int cell_floats;          // LDS floats of one staged radial cell
+    int run_bins;             // bins of a wave's run (a multiple of 4)
+    int window_bins;          // bins of a workgroup's window (a multiple of run_bins)
+    int group;                // patches of a workgroup
+    int block;                // threads per workgroup
+    int sort;                 // 1: sort the points into recs, start first; 2: sort only
+};
+
+// LDS of a projection workgroup with a lookup table: the staged radial cells.
+inline size_t range_lds_bytes(const RangeLaunch& R) { return (size_t)(R.max_slices - 1) * R.cell_floats * 4; }
+
 struct TileLaunch {
     int tile_lines;           // lines whose bins one workgroup keeps in LDS (<= 32)
     int windows;              // radial windows per line; workgroup = tile * windows + window
@@ -217,6 +262,9 @@ struct TileLaunch {
     // Gaussian exponentials), [1] LDS bin additions and [2] (chunk, line) pairs
     // the cull kept (each evaluated by a wave of 64 lanes), added up by the launch
     unsigned long long* stats;
+    // with recs set, launch_project_tile runs the points in range order instead (the
+    // shape above is then not used)
+    RangeLaunch range;
 };
 
 // Blocks one order_tiles launch orders (one workgroup walks them three times).
@@ -288,6 +336,11 @@ hipError_t launch_project_tile(const ProjCommon& c, const CullParams& cp, const 
                                const SplineSet* spline, const ChunkBox* boxes, int nchunks, void* bins,
                                bool arc, bool phase, bool lut, bool shared_origin, const TileLaunch& cfg,
                                hipStream_t stream);
+// project_range.hip: sorts the points s (lines[0]'s origin) into R's buffers; projects
+// them, storing every bin of every line or, with `accumulate`, adding to it.
+hipError_t launch_range_sort(const ProjCommon& c, const FixedSet& s, const RangeLaunch& R, hipStream_t stream);
+hipError_t launch_project_range(const ProjCommon& c, const CullParams& cp, const RangeLaunch& R, float* out,
+                                bool phase, bool lut, int accumulate, unsigned long long* stats, hipStream_t stream);
 // Bytes of one LDS bin of the tile kernel: float or 64-bit fixed point, real or complex.
 inline size_t tile_bin_bytes(bool complex_bins, bool fixed) { return (fixed ? 8 : 4) * (complex_bins ? 2 : 1); }
 size_t tile_lds_bytes(int window_bins, size_t bin_bytes, int tile_lines, int list_cap, int list_packed);

@@ -153,6 +153,52 @@ struct ChunkOrders {
     }
 };
 
+// A dataset's points sorted by radial bin from a scan origin (project_range.hip), one
+// copy (32 bytes a point) per origin, bin rule and demodulation phase.  Like the chunk
+// orders they live as long as the dataset; further origins run the tile kernel.
+struct RangeOrders {
+    struct Key {
+        float ox, oy, oz, phase;
+        double scale, denom;
+        bool operator==(const Key& k) const {
+            return ox == k.ox && oy == k.oy && oz == k.oz && phase == k.phase && scale == k.scale && denom == k.denom;
+        }
+    };
+    struct Order {
+        Key key;
+        DevBuf recs, start;
+    };
+    static constexpr size_t kMaxOrders = 4;
+    std::mutex mu;
+    std::vector<std::unique_ptr<Order>> orders;
+
+    // The order of `key`, or null.  `sort` fills a new order's buffers and waits for
+    // them (other simulators may read them next, on streams of their own); null: only
+    // an order built earlier.  Without memory for another copy there is no order.
+    template <class Sort>
+    const Order* get(const Key& key, size_t n, const Sort* sort) {
+        std::lock_guard<std::mutex> g(mu);
+        for (auto& o : orders)
+            if (o->key == key) return o.get();
+        if (!sort || orders.size() >= kMaxOrders) return nullptr;
+        auto o = std::make_unique<Order>();
+        o->key = key;
+        try {
+            DevBuf rank;
+            o->recs.ensure(n * sizeof(RangeRec));
+            o->start.ensure((kRangeBins + 1) * sizeof(int));
+            rank.ensure(n * sizeof(int));
+            (*sort)(o->recs.as<RangeRec>(), o->start.as<int>(), rank.as<int>());
+        } catch (const BcsimError& e) {
+            if (e.code != BCSIM_ERR_OUT_OF_MEMORY) throw;
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        orders.push_back(std::move(o));
+        return orders.back().get();
+    }
+};
+
 struct FixedDataset {
     DevBuf pts;    // float4[n] (x, y, z, amplitude), Morton order
     DevBuf boxes;  // ChunkBox[nchunks]
@@ -161,6 +207,7 @@ struct FixedDataset {
     double peak_amp = 0.0;  // largest |amplitude| (infinite if any is not finite)
     double typ_amp = 0.0;   // median |amplitude| of the non-zero amplitudes
     mutable ChunkOrders visit;
+    mutable RangeOrders by_range;
 };
 
 struct SplineDataset {
@@ -450,6 +497,7 @@ struct bcsim_sim {
     int profile = -1;
     float sigma_l = 0.f, sigma_e = 0.f;
     std::shared_ptr<DevBuf> lut;  // float4 quad pairs [n_rad][n_ele][n_lat][2]; replaced, never rewritten
+    std::shared_ptr<DevBuf> lut_rel;  // the samples as [n_rad][n_ele][n_lat] (project_range.hip); null if one is not finite
     std::shared_ptr<const std::vector<float>> lut_samples;  // the table as given, for the cutoff's boxes
     float lut_peak = 0.0f;                                   // largest |sample|
     std::shared_ptr<DevBuf> lut_boxes;                       // ProfileParams::slice_box for lut_boxes_cut
@@ -462,6 +510,9 @@ struct bcsim_sim {
     int num_rf = 0, fft_len = 0, log2_len = 0, n_out = 0;
     int tables_fft = 0, tables_out = 0;  // frame shape the convolution tables were built for
     DevBuf d_lines, d_H, d_demod, d_tw, d_bins, d_iq;
+    DevBuf d_patches;  // RangePatch[n_patches] of the lines' directions
+    int n_patches = 0;
+    bool dirty_patches = true;
     DevBuf d_stats;  // with store_kernel_details: per projection launch, weight evaluations and LDS additions
 
     std::map<std::string, std::vector<double>> debug;
@@ -671,6 +722,13 @@ struct bcsim_sim {
             if (!ok) fail(BCSIM_ERR_INVALID_ARGUMENT, "Invalid Scanline: Not orthogonal unit vectors (line " +
                                                            std::to_string(i) + ")");
         }
+        // the patches follow the directions alone: a new time or origin keeps them
+        const auto turned = [](const LineGeom& a, const LineGeom& b) {
+            return a.rx != b.rx || a.ry != b.ry || a.rz != b.rz || a.lx != b.lx || a.ly != b.ly || a.lz != b.lz;
+        };
+        dirty_patches = dirty_patches || g.size() != lines.size() ||
+                        !std::equal(g.begin(), g.end(), lines.begin(),
+                                    [&](const LineGeom& a, const LineGeom& b) { return !turned(a, b); });
         lines.swap(g);
         line_length = length;
         all_equal = equal;
@@ -717,6 +775,7 @@ struct bcsim_sim {
         sigma_l = src.sigma_l;
         sigma_e = src.sigma_e;
         lut = src.lut;
+        lut_rel = src.lut_rel;
         lut_samples = src.lut_samples;
         lut_peak = src.lut_peak;
         lut_boxes = src.lut_boxes;
@@ -725,7 +784,7 @@ struct bcsim_sim {
         lut_r0 = src.lut_r0, lut_r1 = src.lut_r1, lut_l0 = src.lut_l0;
         lut_l1 = src.lut_l1, lut_e0 = src.lut_e0, lut_e1 = src.lut_e1;
         can_change_device = false;
-        dirty_scan = dirty_conv = dirty_basis = true;
+        dirty_scan = dirty_conv = dirty_basis = dirty_patches = true;
     }
 
     // Give every line the time t (a frame of a dynamic phantom at one instant):
@@ -755,7 +814,7 @@ struct bcsim_sim {
 
     // Device bytes of the datasets and LUT (shared by views).
     size_t resident_bytes() const {
-        size_t b = lut ? lut->bytes : 0;
+        size_t b = (lut ? lut->bytes : 0) + (lut_rel ? lut_rel->bytes : 0);
         for (auto& f : fixed) b += f->pts.bytes + f->boxes.bytes;
         for (auto& sp : splines)
             b += sp->cx.bytes + sp->cy.bytes + sp->cz.bytes + sp->amp.bytes + sp->boxes.bytes + sp->iboxes.bytes;
@@ -935,6 +994,22 @@ struct bcsim_sim {
         table->ensure(quad.size() * sizeof(float4));
         hip_check(hipMemcpy(table->p, quad.data(), quad.size() * sizeof(float4), hipMemcpyHostToDevice),
                   "hipMemcpy");
+        // the samples themselves, lateral fastest
+        bool finite = true;
+        std::vector<float> rel(cells);
+        for (int r = 0; r < nr; r++)
+            for (int l = 0; l < nl; l++)
+                for (int e = 0; e < ne; e++) {
+                    const float v = at(r, l, e);
+                    finite = finite && std::isfinite(v);
+                    rel[((size_t)r * ne + e) * nl + l] = v;
+                }
+        lut_rel.reset();
+        if (finite) {
+            lut_rel = std::make_shared<DevBuf>();
+            lut_rel->ensure(cells * sizeof(float));
+            hip_check(hipMemcpy(lut_rel->p, rel.data(), cells * sizeof(float), hipMemcpyHostToDevice), "hipMemcpy");
+        }
         lut = std::move(table);
         lut_samples = std::make_shared<const std::vector<float>>(samples, samples + cells);
         lut_peak = 0.0f;
@@ -1397,6 +1472,7 @@ struct bcsim_sim {
         const ChunkBox* boxes = nullptr;
         int nchunks = 0;
         size_t n = 0;
+        const FixedDataset* fixed = nullptr;  // the fixed kind
         const SplineDataset* sp = nullptr;  // spline kinds
         SplineScan* scan = nullptr;
         const int* chunk_order = nullptr;   // visiting order of the chunks (ChunkOrders), or null
@@ -1463,6 +1539,7 @@ struct bcsim_sim {
             t.boxes = f->boxes.as<ChunkBox>();
             t.nchunks = f->nchunks;
             t.n = f->n;
+            t.fixed = f.get();
             if (chunk_order) {
                 t.chunk_order = f->visit.get(okey, create);
                 t.chunk_dist = ChunkOrders::distances(okey, t.chunk_order, t.nchunks);
@@ -1524,6 +1601,9 @@ struct bcsim_sim {
     int tile_blocks(const TileLaunch& cfg) const {
         return (((int)lines.size() + cfg.tile_lines - 1) / cfg.tile_lines) * cfg.windows;
     }
+
+    // Fewer lines than this leave most lanes of the range order's one patch idle.
+    static constexpr int kRangeMinLines = 16;
 
     // Fewer blocks than this start together on the 256 CUs: no order to choose.
     static constexpr int kMinOrderedBlocks = 512;
@@ -1703,6 +1783,138 @@ struct bcsim_sim {
         return r;
     }
 
+    // Patches of up to kRangePatch lines for the projection in range order: the lines
+    // split at the median of the direction component that spreads most, at a multiple
+    // of the patch size, until a patch's worth is left (8 x 8 lines on a 64 x 64 grid).
+    void build_patches() {
+        std::vector<int> order(lines.size());
+        for (size_t i = 0; i < order.size(); i++) order[i] = (int)i;
+        std::vector<RangePatch> patches;
+        // mean of an axis of the lines [first, last), and how far theirs lie from it (rounded up)
+        const auto bound = [&](const int* first, const int* last, float LineGeom::*x, float* axis) {
+            const auto at = [&](int i) { return &(lines[i].*x); };
+            double m[3] = {0, 0, 0}, far = 0.0;
+            for (const int* p = first; p < last; p++)
+                for (int a = 0; a < 3; a++) m[a] += at(*p)[a];
+            for (int a = 0; a < 3; a++) axis[a] = (float)(m[a] / (double)(last - first));
+            for (const int* p = first; p < last; p++) {
+                double d = 0.0;
+                for (int a = 0; a < 3; a++) d += ((double)at(*p)[a] - axis[a]) * ((double)at(*p)[a] - axis[a]);
+                far = std::max(far, std::sqrt(d));
+            }
+            axis[3] = (float)(far * (1.0 + 1e-6));
+        };
+        // A patch of up to about +-35 degrees sees every point that its beams reach in front of
+        // the origin; wider ones would leave points to the kernel's slow rule for the far side.
+        const auto narrow = [&](const int* first, const int* last) {
+            float axis[4];
+            bound(first, last, &LineGeom::rx, axis);
+            return axis[3] <= 0.62f;
+        };
+        const auto split = [&](auto&& self, int* first, int* last) -> void {
+            const int n = (int)(last - first);
+            if (n > kRangePatch || (n > 1 && !narrow(first, last))) {
+                const auto dir = [&](int i, int a) { return (&lines[i].rx)[a]; };
+                int axis = 0;
+                float widest = -1.0f;
+                for (int a = 0; a < 3; a++) {
+                    float lo = INFINITY, hi = -INFINITY;
+                    for (int* p = first; p < last; p++) lo = std::min(lo, dir(*p, a)), hi = std::max(hi, dir(*p, a));
+                    if (hi - lo > widest) widest = hi - lo, axis = a;
+                }
+                int* mid = first + (n > kRangePatch ? ((n + kRangePatch - 1) / kRangePatch / 2) * kRangePatch : n / 2);
+                std::nth_element(first, mid, last, [&](int i, int j) {
+                    return dir(i, axis) != dir(j, axis) ? dir(i, axis) < dir(j, axis) : i < j;
+                });
+                self(self, first, mid);
+                self(self, mid, last);
+                return;
+            }
+            std::sort(first, last);
+            RangePatch q{};
+            q.n = n;
+            for (int k = 0; k < kRangePatch; k++) {
+                const LineGeom& g = lines[q.line[k] = first[k < n ? k : 0]];
+                const float axes[6] = {g.lx, g.ly, g.lz, g.ex, g.ey, g.ez};
+                for (int a = 0; a < 6; a++) q.axes[a][k] = axes[a];
+            }
+            bound(first, last, &LineGeom::rx, &q.rx);
+            bound(first, last, &LineGeom::lx, &q.lx);
+            bound(first, last, &LineGeom::ex, &q.ex);
+            patches.push_back(q);
+        };
+        split(split, order.data(), order.data() + order.size());
+        quiesce();
+        d_patches.ensure(patches.size() * sizeof(RangePatch));
+        hip_check(hipMemcpy(d_patches.p, patches.data(), patches.size() * sizeof(RangePatch), hipMemcpyHostToDevice),
+                  "hipMemcpy");
+        n_patches = (int)patches.size();
+        dirty_patches = false;
+    }
+
+    // Projection of target t in range order (project_range.hip), or a launch without
+    // records: the tile kernel runs.  It takes arc projection of fixed points onto
+    // lines of one origin, when nothing in the tile kernel's shape was set by hand,
+    // the amplitudes and the table are finite (its skipped pairs then add exactly 0)
+    // and the slices of a window fit LDS.
+    RangeLaunch range_launch(const ProjTarget& t, const FixedDataset* ds, const TileLaunch& shape, float* bins,
+                             bool create) {
+        RangeLaunch R{};
+        const bool lut_profile = profile == kProfileLut;
+        const bool by_hand = tune.windows || tune.lines || tune.block || tune.slices || bin_mode;
+        if (!ds || direct_mode || !arc || by_hand || (int)lines.size() < kRangeMinLines || !std::isfinite(t.c.prof.w_cut) ||
+            !std::isfinite(ds->peak_amp) || !shared_origin())
+            return R;
+        const CullParams cp = cull_params(t.c);
+        if (lut_profile) {
+            if (!lut_rel || !(cp.lut_dl > 0.0f)) return R;
+            R.table = lut_rel->as<float>();
+            R.cell_floats = 2 * (lut_nl | 1) * lut_ne;
+        }
+        if (dirty_patches) {
+            if (!create) return R;
+            build_patches();
+        }
+        R.n_patches = n_patches;
+        R.run_bins = 4;  // one store of four bins; longer runs leave too few waves at the sizes of a 2D sector
+        if (lut_profile) {
+            // A window spans less than two radial cells, so that the staged cells leave room
+            // for two workgroups of 16 waves on a CU; 16 patches share them.  (1M points, 4096
+            // lines, frames one after another: windows of 24 / 32 / 36 bins 0.852 / 0.874 /
+            // 0.876 ms, 8 or 32 patches 0.955 / 1.007.)
+            R.block = 1024;
+            R.group = 16;
+            for (R.window_bins = 24;; R.window_bins -= R.run_bins) {
+                const double radial = (double)R.window_bins * (double)cp.r_per_bin * (double)t.c.prof.inv_dr;
+                R.max_slices = (int)std::min<double>(lut_nr, std::floor(radial + 2.0 * (1e-3 + 2e-6 * lut_nr)) + 3.0);
+                if (R.window_bins == R.run_bins || range_lds_bytes(R) <= (size_t)kLdsBytes / 2 - 512) break;
+            }
+            if (range_lds_bytes(R) > (size_t)kLdsBytes - 512) return R;
+        } else {
+            // nothing to share: small workgroups of four waves, a patch and a run each
+            R.block = 256;
+            R.group = std::min(R.n_patches, 4);
+            R.window_bins = R.run_bins * (4 / R.group);
+        }
+        const RangeOrders::Key key{lines[0].ox, lines[0].oy, lines[0].oz, t.c.phase_per_sample, t.c.bin_scale, t.c.bin_denom};
+        const auto sort = [&](RangeRec* recs, int* start, int* rank) {
+            TileLaunch g = shape;
+            g.range = R;
+            g.range.recs = recs;
+            g.range.start = start;
+            g.range.rank = rank;
+            g.range.sort = 2;
+            launch_target(t, g, bins);
+            hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
+        };
+        const RangeOrders::Order* o = ds->by_range.get(key, ds->n, create ? &sort : nullptr);
+        if (!o) return R;
+        R.patches = d_patches.as<RangePatch>();
+        R.start = o->start.as<int>();
+        R.recs = o->recs.as<RangeRec>();
+        return R;
+    }
+
     // Debug data keys the reference records on every frame with
     // store_kernel_details (GpuAlgorithm.cpp:193-358) that have no kernel of their
     // own here: one stream per frame (stream number 0 for every line), and the
@@ -1739,12 +1951,17 @@ struct bcsim_sim {
                 direct_plans.push_back(proj_launch(t.n));
             } else {
                 plans.push_back(plan_tile(t, autotune && !fm));
-                const TileLaunch& g = plans.back();
+                TileLaunch& g = plans.back();
+                g.range = range_launch(t, t.fixed, g, bins, fm == nullptr);
                 last_plan += std::string(t.kind) + (t.ss.iboxes ? " (interval boxes)" : "") +
                              ": lines=" + std::to_string(g.tile_lines) +
                              " block=" + std::to_string(g.block) + " slices=" + std::to_string(g.slices) +
                              " windows=" + std::to_string(g.windows) + " bins=" + (g.fixed ? "fixed" : "float") +
-                             " list=" + std::to_string(g.list_cap) + (g.list_packed ? " packed" : "") + "\n";
+                             " list=" + std::to_string(g.list_cap) + (g.list_packed ? " packed" : "") +
+                             (g.range.recs ? " (replaced by range order: patches of " + std::to_string(kRangePatch) +
+                                                 " lines, windows of " + std::to_string(g.range.window_bins) + " bins)"
+                                           : "") +
+                             "\n";
             }
         }
         const int frame_radix = plan_radix(autotune && !fm);
@@ -1752,7 +1969,7 @@ struct bcsim_sim {
 
         // The bins are zeroed first unless a single launch writes every bin with plain stores.
         const bool single = targets.size() == 1;
-        const bool need_zero = !single || (direct_mode ? direct_plans[0].slices > 1 : plans[0].slices > 1);
+        const bool need_zero = !single || (direct_mode ? direct_plans[0].slices > 1 : plans[0].slices > 1 && !plans[0].range.recs);
         if (need_zero) {
             Timed t(this, "kernel_memset_ms");
             hip_check(launch_fill_zero(bins, bin_floats, stream), "fill kernel");
@@ -1783,10 +2000,11 @@ struct bcsim_sim {
                 tm.stop();
             } else {
                 TileLaunch cfg = plans[i];
+                if (cfg.range.recs) cfg.atomic = 0;  // no slices: each bin is stored, or added to, once
                 cfg.atomic |= single ? 0 : 1;
                 if (stats_launches) cfg.stats = d_stats.as<unsigned long long>() + kStatsPerLaunch * i;
                 const int blocks = tile_blocks(cfg);
-                if (!fm && tile_order && blocks >= kMinOrderedBlocks && blocks <= kMaxOrderedTiles) {
+                if (!fm && !cfg.range.recs && tile_order && blocks >= kMinOrderedBlocks && blocks <= kMaxOrderedTiles) {
                     int* wo = order_buffer(i, blocks);
                     cfg.work = wo;
                     cfg.order = wo + blocks;
