@@ -9,6 +9,32 @@
 
 namespace bcsim_hip {
 
+constexpr float kExpMinusMax = 80.0f;  // largest argument of exp_minus
+
+// Correctly rounded square root of a squared distance: the hardware root (within an
+// ulp) and the neighbour whose rounding interval holds x.  Residuals below 2^-96
+// (distances below 4e-15 m, bin 0 whatever their last bit) may be an ulp off; the
+// compiler's form rescales those, at twice the instructions.
+__device__ __forceinline__ float sqrt_distance(float x) {
+    const float s = __builtin_amdgcn_sqrtf(x);
+    const float dn = __int_as_float(__float_as_int(s) - 1), up = __int_as_float(__float_as_int(s) + 1);
+    float r = __builtin_fmaf(-dn, s, x) <= 0.0f ? dn : s;
+    return __builtin_fmaf(-up, s, x) > 0.0f ? up : r;
+}
+
+// exp(-x) for 0 <= x <= 80, where it neither under- nor overflows: 2^y, y = -x log2(e)
+// kept as a whole number n, a remainder and the rounding error of y, scaled by adding n
+// to the exponent: expf without its range checks, with the same error (8.2e-8 at most,
+// 2.6e-8 rms over [0, 80]).
+__device__ __forceinline__ float exp_minus(float x) {
+    constexpr float c = -1.44269502f, c_lo = -1.92596303e-8f;  // -log2(e)
+    const float y = x * c;
+    const float d = __builtin_fmaf(x, c_lo, __builtin_fmaf(x, c, -y));
+    const float n = __builtin_rintf(y);
+    const float t = __builtin_amdgcn_exp2f((y - n) + d);  // in [0.7, 1.42]
+    return __int_as_float(__float_as_int(t) + ((int)n << 23));
+}
+
 // Beam-local coordinates, float, left-to-right dot products (CpuAlgorithm.cpp:58-72).
 struct Local {
     float r, l, e;
@@ -23,7 +49,7 @@ __device__ __forceinline__ Local local_coords(const LineGeom& L, float px, float
     o.r = dx * L.rx + dy * L.ry + dz * L.rz;
     o.l = dx * L.lx + dy * L.ly + dz * L.lz;
     o.e = dx * L.ex + dy * L.ey + dz * L.ez;
-    if (ARC) o.r = copysignf(__builtin_sqrtf(dx * dx + dy * dy + dz * dz), o.r);
+    if (ARC) o.r = copysignf(sqrt_distance(dx * dx + dy * dy + dz * dz), o.r);
     return o;
 }
 
@@ -40,7 +66,7 @@ __device__ __forceinline__ float gauss_weight(const ProfileParams& P, float l, f
     const float x = l * l * P.inv_tsl + e * e * P.inv_tse;
     if (x > P.g_cut) return 0.0f;
     t.evals++;
-    return expf(-x);
+    return P.g_cut <= kExpMinusMax ? exp_minus(x) : expf(-x);
 }
 
 // LUTBeamProfile::sampleProfile (BeamProfile.cpp:79-130): truncating indices, zero
@@ -120,22 +146,21 @@ __device__ __forceinline__ float lut_weight(const ProfileParams& P, float r, flo
 }
 
 // Bin of radial distance r: floor(r*scale/denom + 0.5) evaluated in double as the
-// reference writes it (CpuAlgorithm.cpp:75 fixed, :161-162 spline).  The quotient is
-// first formed with the reciprocal; only when the result lies within 1e-9 of a
-// bin boundary (where the two could round differently) is the exact division
-// done.  Returns -1 for bins outside [0, num_rf) and for non-finite r.
+// reference writes it (CpuAlgorithm.cpp:75 fixed, :161-162 spline).  The sum is
+// first formed as one multiply-add by bins per metre; only when the result lies
+// within 1e-9 of a bin boundary (where the two could round differently) is the
+// exact division done.  Returns -1 for bins outside [0, num_rf) and for non-finite r.
+__device__ __forceinline__ double radial_sum(const ProjCommon& c, float r) {
+    double t = __builtin_fma((double)r, c.bins_per_metre, 0.5);
+    const double fr = __builtin_amdgcn_fract(t);
+    if (fr < 1e-9 || fr > 1.0 - 1e-9) t = (double)r * c.bin_scale / c.bin_denom + 0.5;
+    return t;
+}
+
 __device__ __forceinline__ int radial_bin(const ProjCommon& c, float r, double& true_index) {
-    const double q = (double)r * c.bin_scale;
-    true_index = q * c.bin_inv_denom;
-    double t = true_index + 0.5;
-    double fl = floor(t);
-    const double fr = t - fl;
-    if (fr < 1e-9 || fr > 1.0 - 1e-9) {
-        t = q / c.bin_denom + 0.5;
-        fl = floor(t);
-    }
-    if (!(t >= 0.0 && t < (double)c.num_rf)) return -1;
-    return (int)fl;
+    const double t = radial_sum(c, r);
+    true_index = t - 0.5;
+    return t >= 0.0 && t < (double)c.num_rf ? (int)t : -1;
 }
 
 // Add one scatterer's contribution to its bin in LDS (CpuAlgorithm.cpp:77-95).

@@ -55,7 +55,7 @@ __global__ __launch_bounds__(256) void range_clear_kernel(int* __restrict__ star
 __device__ __forceinline__ int range_bin(const ProjCommon& c, const float4& p, float ox, float oy, float oz, float3& d,
                                          float& absd, double& ti) {
     d = make_float3(p.x - ox, p.y - oy, p.z - oz);
-    absd = __builtin_sqrtf(d.x * d.x + d.y * d.y + d.z * d.z);
+    absd = sqrt_distance(d.x * d.x + d.y * d.y + d.z * d.z);
     return radial_bin(c, absd, ti);
 }
 
@@ -124,19 +124,6 @@ __device__ __forceinline__ float dot_fused(float x, float y, float z, float a, f
 
 // max(x, 0) of a number as one integer instruction (fmaxf also quiets NaNs).
 __device__ __forceinline__ float at_least_0(float x) { return __int_as_float(max(__float_as_int(x), 0)); }
-
-// exp(-x) for 0 <= x <= 80, where it neither under- nor overflows: 2^y, y = -x log2(e)
-// kept as a whole number n, a remainder and the rounding error of y, scaled by adding n
-// to the exponent.  (expf without its range checks: the same error, 4.5 against 13
-// instructions a weight over the common part of both.)
-__device__ __forceinline__ float exp_minus(float x) {
-    constexpr float c = -1.44269502f, c_lo = -1.92596303e-8f;  // -log2(e)
-    const float y = x * c;
-    const float d = __builtin_fmaf(x, c_lo, __builtin_fmaf(x, c, -y));
-    const float n = __builtin_rintf(y);
-    const float t = __builtin_amdgcn_exp2f((y - n) + d);  // in [0.7, 1.42]
-    return __int_as_float(__float_as_int(t) + ((int)n << 23));
-}
 
 // Records (r, l, e) of the table that a window can look up, and the slices it holds.
 struct RangeRegion {
@@ -249,7 +236,7 @@ __global__ __launch_bounds__(1024, 8) void project_range_kernel(ProjCommon c, Cu
         return __builtin_amdgcn_readfirstlane(u);
     };
     const char* cell_bytes = reinterpret_cast<const char*>(cells);
-    const bool small_x = P.g_cut <= 80.0f;
+    const bool small_x = P.g_cut <= kExpMinusMax;
     for (int u = wave; u < units; u = claim()) {
         const RangePatch& patch = R.patches[patch0 + u / runs];
         const int w0 = (u % runs) * R.run_bins;       // the run's first bin in the window

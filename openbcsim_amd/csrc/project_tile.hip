@@ -198,6 +198,31 @@ __device__ __forceinline__ bool narrow_support(const ProfileParams& P, CullParam
     return true;
 }
 
+// Adds up a block's counts: its listed (chunk, line) pairs for the next launch's order,
+// and the launch statistics (into the workgroup's wg_stats).
+__device__ __forceinline__ void count_work(const TileLaunch& g, int wg, int hits, const Tally& tally,
+                                           unsigned long long* wg_stats) {
+    const int lane = threadIdx.x & 63;
+    if (g.work) {
+        // the block's work, for the order of the next launch: one atomic per wave
+        for (int off = 32; off > 0; off >>= 1) hits += __shfl_xor(hits, off);
+        if (lane == 0 && hits) atomicAdd(&g.work[wg], hits);
+    }
+    if (g.stats) {
+        unsigned long long ev = (unsigned)tally.evals, ad = (unsigned)tally.adds, hc = (unsigned)hits;
+        for (int off = 32; off > 0; off >>= 1) {
+            ev += __shfl_xor(ev, off);
+            ad += __shfl_xor(ad, off);
+            if (!g.work) hc += __shfl_xor(hc, off);  // (already summed over the wave for the block order)
+        }
+        if (lane == 0) {
+            atomicAdd(&wg_stats[0], ev);
+            atomicAdd(&wg_stats[1], ad);
+            atomicAdd(&wg_stats[2], hc);
+        }
+    }
+}
+
 // One (tile, window, slice) block of work: everything a workgroup of the tile
 // kernel does.  `wg` = tile * windows + window; `lds` is the dynamic LDS and
 // `list_n` a workgroup-shared counter.  FIXED: 64-bit fixed-point LDS bins.
@@ -434,7 +459,7 @@ __device__ __forceinline__ void tile_block(const ProjCommon& c, const CullParams
                 const float4 p = fs.pts[s];
                 const float amp = FIXED ? p.w * c.amp_scale : p.w;
                 const float dx = p.x - org_x, dy = p.y - org_y, dz = p.z - org_z;
-                const float absd = __builtin_sqrtf(dx * dx + dy * dy + dz * dz);
+                const float absd = sqrt_distance(dx * dx + dy * dy + dz * dz);
                 double ti_pos;
                 const int bin_pos = radial_bin(c, absd, ti_pos);
                 const int lb_pos = bin_pos - b0;
@@ -494,24 +519,7 @@ __device__ __forceinline__ void tile_block(const ProjCommon& c, const CullParams
         if (threadIdx.x == 0) list_n = 0;
         __syncthreads();
     }
-    if (g.work) {
-        // the block's work, for the order of the next launch: one atomic per wave
-        for (int off = 32; off > 0; off >>= 1) hits += __shfl_xor(hits, off);
-        if (lane == 0 && hits) atomicAdd(&g.work[wg], hits);
-    }
-    if (g.stats) {
-        unsigned long long ev = (unsigned)tally.evals, ad = (unsigned)tally.adds, hc = (unsigned)hits;
-        for (int off = 32; off > 0; off >>= 1) {
-            ev += __shfl_xor(ev, off);
-            ad += __shfl_xor(ad, off);
-            if (!g.work) hc += __shfl_xor(hc, off);  // (already summed over the wave for the block order)
-        }
-        if (lane == 0) {
-            atomicAdd(&wg_stats[0], ev);
-            atomicAdd(&wg_stats[1], ad);
-            atomicAdd(&wg_stats[2], hc);
-        }
-    }
+    count_work(g, wg, hits, tally, wg_stats);
     __syncthreads();
     if (g.stats && threadIdx.x < 3) atomicAdd(&g.stats[threadIdx.x], wg_stats[threadIdx.x]);  // one per block
     // flush: line k's window [b0, b0 + nb) of the global bins [line][num_rf]
@@ -528,6 +536,200 @@ __device__ __forceinline__ void tile_block(const ProjCommon& c, const CullParams
     }
 }
 
+// Work of a wave (Tally, counted in scalar registers).
+struct LineTally {
+    int evals = 0;
+    int adds = 0;
+};
+
+// A value that is the same in every lane, in a scalar register.
+__device__ __forceinline__ float uniform(float v) {
+    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+}
+// The scatterers of one chunk, one per lane: for splines the CP control points active
+// at the line's time, for points the position itself.  The chunk's address is uniform
+// and the lane's offset 32 bits, so that an address costs no vector instructions.
+template <bool SPLINE, int CP>
+struct ChunkLoad {
+    float x[CP], y[CP], z[CP], amp;
+    bool in;
+    __device__ __forceinline__ void load(const FixedSet& fs, const SplineSet& ss, int lo, int chunk, unsigned lane) {
+        const int first = chunk * kChunk;
+        const unsigned n = SPLINE ? ss.n : fs.n;
+        in = lane < n - first;
+        const unsigned at = min(lane, n - first - 1);
+        if (SPLINE) {
+            const size_t base = (size_t)lo * n + first;
+#pragma unroll
+            for (int i = 0; i < CP; i++) {
+                x[i] = (ss.cx + base + (size_t)i * n)[at];
+                y[i] = (ss.cy + base + (size_t)i * n)[at];
+                z[i] = (ss.cz + base + (size_t)i * n)[at];
+            }
+            amp = (ss.amp + first)[at];
+        } else {
+            const float4 p = (fs.pts + first)[at];
+            x[0] = p.x, y[0] = p.y, z[0] = p.z, amp = p.w;
+        }
+    }
+};
+
+// Projects the listed chunks list[0, n) onto one line, a chunk per wave at a time, the
+// next chunk's loads under way meanwhile.
+template <bool ARC, bool PHASE, bool LUT, bool SPLINE, int CP, class Acc>
+__device__ __forceinline__ void project_list(const ProjCommon& c, const FixedSet& fs, const SplineSet& ss,
+                                             const LineGeom& L, int lo, const float* basis, const int* list, int n,
+                                             Acc* bins, int b0, int nb, float scale, LineTally& tally) {
+    const unsigned lane = threadIdx.x & 63;
+    const int nwaves = blockDim.x >> 6;
+    int j = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const ProfileParams& P = c.prof;
+    const bool small_x = P.g_cut <= kExpMinusMax;
+    if (j >= n) return;
+    ChunkLoad<SPLINE, CP> q;
+    q.load(fs, ss, lo, __builtin_amdgcn_readfirstlane(list[j]), lane);
+    for (;;) {
+        float px = q.x[0], py = q.y[0], pz = q.z[0];
+        if (SPLINE) {
+            // CpuAlgorithm.cpp:137-140: float sum from zero, in control-point order
+            px = py = pz = 0.0f;
+#pragma unroll
+            for (int i = 0; i < CP; i++) {
+                px = px + q.x[i] * basis[i];
+                py = py + q.y[i] * basis[i];
+                pz = pz + q.z[i] * basis[i];
+            }
+        }
+        const float amp = q.amp * scale;
+        const bool in = q.in;
+        j += nwaves;
+        if (j < n) q.load(fs, ss, lo, __builtin_amdgcn_readfirstlane(list[j]), lane);
+        const Local p = local_coords<ARC>(L, px, py, pz);
+        const double t = radial_sum(c, p.r);
+        const int lb = (int)t - b0;  // below the window, or huge: fails the unsigned test
+        bool ok = in && t >= 0.0 && (unsigned)lb < (unsigned)nb;
+        float x = 0.0f;
+        if (!LUT) {
+            x = p.l * p.l * P.inv_tsl + p.e * p.e * P.inv_tse;
+            ok = ok && !(x > P.g_cut);
+        }
+        Tally lut;
+        float w = 0.0f;
+        if (ok) {
+            w = (LUT ? lut_weight(P, p.r, p.l, p.e, lut) : small_x ? exp_minus(x) : expf(-x)) * amp;
+            if (w != 0.0f) {  // adding +-0 leaves the bin unchanged
+                if (PHASE) {
+                    float si, co;
+                    sincosf((float)((double)(lb + b0) - (t - 0.5)) * c.phase_per_sample, &si, &co);
+                    lds_add(&bins[2 * lb], w * co);
+                    lds_add(&bins[2 * lb + 1], w * si);
+                } else {
+                    lds_add(&bins[lb], w);
+                }
+            }
+        }
+        tally.evals += __popcll(__ballot(LUT ? lut.evals != 0 : ok));
+        tally.adds += (PHASE ? 2 : 1) * __popcll(__ballot(w != 0.0f));
+        if (j >= n) return;
+    }
+}
+
+// tile_block for a tile of one line (any origin; splines at the line's time): the
+// line's geometry and spline basis stay in registers, the list needs no masks, and a
+// chunk's scatterers are loaded while the previous chunk's are projected.
+template <bool ARC, bool PHASE, bool LUT, bool SPLINE, bool FIXED>
+__device__ __forceinline__ void line_block(const ProjCommon& c, const CullParams& cp, const FixedSet& fs,
+                                           const SplineSet& ss, const ChunkBox* __restrict__ boxes, int nchunks,
+                                           float* __restrict__ out, const TileLaunch& g, int wg, int slice,
+                                           float* lds, int& list_n) {
+    constexpr int E = PHASE ? 2 : 1;
+    using Acc = typename std::conditional<FIXED, long long, float>::type;
+    const int window = wg % g.windows;
+    const int line = wg / g.windows;
+    const int b0 = window * g.window_bins;
+    const int nb = min(g.window_bins, c.num_rf - b0);
+    Acc* bins = reinterpret_cast<Acc*>(lds + kTileLineLds / sizeof(float));  // as tile_lds_bytes lays it out
+    int* list = reinterpret_cast<int*>(bins + (size_t)g.window_bins * E);
+    if (threadIdx.x < 4)
+        reinterpret_cast<float4*>(lds)[threadIdx.x] = reinterpret_cast<const float4*>(c.lines + line)[threadIdx.x];
+    int lo = 0, count = 0;
+    float basis[kMaxSplineDegree + 1] = {};
+    if (SPLINE) {
+        const SplineLineBasis& B = ss.basis[line];
+        lo = __builtin_amdgcn_readfirstlane(B.lo);
+        count = __builtin_amdgcn_readfirstlane(B.count);
+#pragma unroll
+        for (int i = 0; i <= kMaxSplineDegree; i++) basis[i] = uniform(B.b[i]);
+    }
+    for (int i = threadIdx.x; i < nb * E; i += blockDim.x) bins[i] = Acc(0);
+    __shared__ unsigned long long wg_stats[3];  // the block's launch statistics (TileLaunch::stats)
+    if (threadIdx.x == 0) list_n = 0;
+    if (g.stats && threadIdx.x < 3) wg_stats[threadIdx.x] = 0;
+    const float r_lo = fmaxf(cp.r_lo, ((float)b0 - 0.5f) * cp.r_per_bin);
+    const float r_hi = fminf(cp.r_hi, ((float)(b0 + nb) - 0.5f) * cp.r_per_bin);
+    const int lane = threadIdx.x & 63;
+    const int cbeg = slice * g.chunks_per_slice;
+    const int cend = min(nchunks, cbeg + g.chunks_per_slice);
+    const int step = min((int)blockDim.x, g.list_cap);
+    int hits = 0;  // chunks this thread listed
+    LineTally tally;
+    __syncthreads();
+    // through LDS into vector registers: there are not enough scalar ones for it as well
+    const LineGeom L = *reinterpret_cast<const LineGeom*>(lds);
+    for (int next = cbeg; next < cend;) {
+        const int pos = next + (int)threadIdx.x;
+        bool hit = false;
+        int ci = 0;
+        if ((int)threadIdx.x < step && pos < cend) {
+            ci = g.chunks ? g.chunks[pos] : pos;
+            hit = chunk_hits<ARC, LUT>(cp, r_lo, r_hi, L,
+                                       SPLINE && ss.iboxes ? ss.iboxes[(size_t)ci * ss.n_iv + lo] : boxes[ci]);
+        }
+        const unsigned long long m = __ballot(hit);
+        if (m) {  // one addition to the list's length per wave
+            int at = 0;
+            if (lane == 0) at = atomicAdd(&list_n, __popcll(m));
+            at = __builtin_amdgcn_readfirstlane(at);
+            if (hit) {
+                list[at + __popcll(m & ((1ull << lane) - 1))] = ci;
+                hits++;
+            }
+        }
+        next += step;
+        __syncthreads();
+        const int n = __builtin_amdgcn_readfirstlane(list_n);
+        __syncthreads();
+        if (next < cend && n <= g.list_cap - step) continue;
+        const float scale = FIXED ? c.amp_scale : 1.0f;
+        if (!SPLINE)
+            project_list<ARC, PHASE, LUT, false, 1>(c, fs, ss, L, 0, basis, list, n, bins, b0, nb, scale, tally);
+        else if (count == 4)
+            project_list<ARC, PHASE, LUT, true, 4>(c, fs, ss, L, lo, basis, list, n, bins, b0, nb, scale, tally);
+        else if (count == 3)
+            project_list<ARC, PHASE, LUT, true, 3>(c, fs, ss, L, lo, basis, list, n, bins, b0, nb, scale, tally);
+        else if (count == 2)
+            project_list<ARC, PHASE, LUT, true, 2>(c, fs, ss, L, lo, basis, list, n, bins, b0, nb, scale, tally);
+        else if (count == 1)
+            project_list<ARC, PHASE, LUT, true, 1>(c, fs, ss, L, lo, basis, list, n, bins, b0, nb, scale, tally);
+        else
+            project_list<ARC, PHASE, LUT, true, 5>(c, fs, ss, L, lo, basis, list, n, bins, b0, nb, scale, tally);
+        __syncthreads();
+        if (threadIdx.x == 0) list_n = 0;
+        __syncthreads();
+    }
+    Tally all;  // the wave's counts, in its first lane
+    if (lane == 0) all.evals = tally.evals, all.adds = tally.adds;
+    count_work(g, wg, hits, all, wg_stats);
+    __syncthreads();
+    if (g.stats && threadIdx.x < 3) atomicAdd(&g.stats[threadIdx.x], wg_stats[threadIdx.x]);  // one per block
+    float* dst = out + ((size_t)line * c.num_rf + b0) * E;
+    for (int i = threadIdx.x; i < nb * E; i += blockDim.x) {
+        const float v = bin_value(bins[i], c);
+        if (!g.atomic) dst[i] = v;
+        else if (v != 0.0f) unsafeAtomicAdd(dst + i, v);
+    }
+}
+
 template <bool ARC, bool PHASE, bool LUT, bool SPLINE, bool SHARED, bool FIXED>
 __global__ __launch_bounds__(1024) void project_tile_kernel(ProjCommon c, CullParams cp, FixedSet fs, SplineSet ss,
                                                             const ChunkBox* __restrict__ boxes, int nchunks,
@@ -537,6 +739,16 @@ __global__ __launch_bounds__(1024) void project_tile_kernel(ProjCommon c, CullPa
     const int wg = g.order ? g.order[blockIdx.x] : (int)blockIdx.x;
     tile_block<ARC, PHASE, LUT, SPLINE, SHARED, FIXED>(c, cp, fs, ss, boxes, nchunks, out, g, wg, blockIdx.y, lds,
                                                        list_n);
+}
+
+template <bool ARC, bool PHASE, bool LUT, bool SPLINE, bool FIXED>
+__global__ __launch_bounds__(1024, 8) void project_line_kernel(ProjCommon c, CullParams cp, FixedSet fs, SplineSet ss,
+                                                            const ChunkBox* __restrict__ boxes, int nchunks,
+                                                            float* __restrict__ out, TileLaunch g) {
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    __shared__ int list_n;
+    const int wg = __builtin_amdgcn_readfirstlane(g.order ? g.order[blockIdx.x] : (int)blockIdx.x);
+    line_block<ARC, PHASE, LUT, SPLINE, FIXED>(c, cp, fs, ss, boxes, nchunks, out, g, wg, blockIdx.y, lds, list_n);
 }
 
 // Order of the next tile launch's blocks: by the (chunk, line) pairs each listed
@@ -643,8 +855,12 @@ __global__ __launch_bounds__(1024) void project_batch_kernel(const ProjJob* __re
         const int blk = __builtin_amdgcn_readfirstlane(w.y);
         const int per_slice = J.blocks_per_slice;
         const int wg = blk % per_slice, slice = blk / per_slice;
-        tile_block<ARC, PHASE, LUT, KIND == 2, KIND == 1, FIXED>(J.c, J.cp, J.fs, J.ss, J.boxes, J.nchunks, J.bins,
-                                                                 J.g, wg, slice, lds, list_n);
+        if (KIND != 1 && J.g.tile_lines == 1)
+            line_block<ARC, PHASE, LUT, KIND == 2, FIXED>(J.c, J.cp, J.fs, J.ss, J.boxes, J.nchunks, J.bins, J.g, wg,
+                                                          slice, lds, list_n);
+        else
+            tile_block<ARC, PHASE, LUT, KIND == 2, KIND == 1, FIXED>(J.c, J.cp, J.fs, J.ss, J.boxes, J.nchunks, J.bins,
+                                                                     J.g, wg, slice, lds, list_n);
         __syncthreads();  // the next item reuses the LDS
     }
 }
@@ -709,6 +925,8 @@ static hipError_t launch_tile_f(const ProjCommon& c, const CullParams& cp, const
     const size_t lds =
         tile_lds_bytes(cfg.window_bins, tile_bin_bytes(PHASE, FIXED), cfg.tile_lines, cfg.list_cap, cfg.list_packed);
     auto k = project_tile_kernel<ARC, PHASE, LUT, SPLINE, SHARED, FIXED>;
+    if constexpr (!SHARED)
+        if (cfg.tile_lines == 1) k = project_line_kernel<ARC, PHASE, LUT, SPLINE, FIXED>;
     hipError_t e = allow_lds((const void*)k, lds);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k, dim3(tiles * cfg.windows, cfg.slices), dim3(cfg.block), lds, stream, c, cp, fs, ss, boxes,

@@ -75,10 +75,10 @@ struct ProjCommon {
     int num_lines;
     int num_rf;
     // radial bin = floor(r * scale / denom + 0.5) in double (CpuAlgorithm.cpp:75, :161-162);
-    // evaluated as r*scale*inv_denom with an exact-division fallback near half-samples.
+    // evaluated as r*bins_per_metre with an exact-division fallback near half-samples.
     double bin_scale;
     double bin_denom;
-    double bin_inv_denom;
+    double bins_per_metre;
     // sub-sample phase: phase = (bin - true_index) * phase_per_sample, true_index = r*scale/denom
     float phase_per_sample;
     ProfileParams prof;

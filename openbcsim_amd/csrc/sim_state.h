@@ -1252,7 +1252,7 @@ struct bcsim_sim {
             c.bin_scale = 2.0 * (double)fs;
             c.bin_denom = (double)sound_speed;
         }
-        c.bin_inv_denom = 1.0 / c.bin_denom;
+        c.bins_per_metre = c.bin_scale / c.bin_denom;
         c.phase_per_sample = (float)(2.0 * M_PI * (double)f_demod / (double)fs);
         ProfileParams& P = c.prof;
         if (profile == kProfileGaussian) {
@@ -1411,9 +1411,7 @@ struct bcsim_sim {
     // Launch shape of the tile kernel for `tune` (0 fields: heuristic): one
     // radial window unless a line's bins overflow LDS, up to 16 lines per
     // workgroup (while at least ~1024 workgroups remain), and enough chunk
-    // slices for about 256 workgroups (1024 for splines with a time per line,
-    // whose hits cost more: the tuner's choices on the 2D sector and the spline
-    // M-mode, 6 % and 13 % faster than 512 workgroups).
+    // slices to fill the chip.
     TileLaunch tile_launch(int nchunks, const TileTune& tune, bool per_line_splines, bool fixed_bins) const {
         TileLaunch cfg{};
         const int L = (int)lines.size();
@@ -1439,8 +1437,17 @@ struct bcsim_sim {
         }
         T = std::max(1, std::min(T, L));
         const int blocks = ((L + T - 1) / T) * K;
-        const int target = per_line_splines ? 1024 : 256;
-        int slices = tune.slices > 0 ? tune.slices : std::max(1, (target + blocks - 1) / blocks);
+        // Points of one origin: 256 workgroups.  Other targets' hits cost more: 512, and 1024
+        // for splines with a time per line, but no slice of fewer than 400 chunks beyond 256
+        // workgroups, whose flush then costs more than its balance gives.  (Frames of three
+        // simulators in flight by slices 1 / 2 / 3 / 4 / 8: 191 lines x 2344 chunks of a
+        // straight scan 46 / 44 / 44 / 45 / 52 us, 256 spline lines x 3125 chunks 76 / 71 /
+        // 66 / 62 / 66, 131 spline lines x 1216 chunks with phase delay 50 / 43 / 41 / 41 / 47.)
+        const auto per = [&](int workgroups) { return (workgroups + blocks - 1) / blocks; };
+        int slices = per(256);
+        if (per_line_splines || !(arc && shared_origin()))
+            slices = std::max(slices, std::min(per(per_line_splines ? 1024 : 512), nchunks / 400));
+        if (tune.slices > 0) slices = tune.slices;
         slices = std::max(1, std::min(slices, std::max(1, nchunks / 16)));
         cfg.tile_lines = T;
         cfg.windows = K;
@@ -1485,13 +1492,21 @@ struct bcsim_sim {
     // Does this target's launch use fixed-point bins?  Not where its amplitudes do
     // not allow it (amp_scale 0); else the parameter if set, then `tuned` (a
     // TileTune::bins), then the default: fixed for the Gaussian profile, whose LDS
-    // additions weigh on the kernel (fixed-point ones are ~10x cheaper), float for
-    // a LUT, whose table gathers bound it and where the wider bins only halve the
-    // lines a tile holds (measured on the 1M-point volume: 1.91 against 1.65 ms).
+    // additions weigh on the kernel (fixed-point ones are ~10x cheaper).  For a LUT
+    // float on tiles of several lines, which the wider bins would halve (1M-point
+    // volume: 1.91 against 1.65 ms of projection) and for points of one origin; fixed
+    // where a tile is one line anyway (project_line_kernel: 191 lines against 150k
+    // points in a straight scan 79 -> 66 us a frame, 131 spline lines with phase delay
+    // 80 -> 69).
     bool target_fixed(const ProjTarget& t, int tuned = 0) const {
         if (!(t.c.amp_scale > 0.0f)) return false;
-        const int m = bin_mode ? bin_mode : tuned ? tuned : (profile == kProfileLut ? 2 : 1);
-        return m == 1;
+        const int m = bin_mode ? bin_mode : tuned;
+        if (m) return m == 1;
+        if (profile != kProfileLut) return true;
+        const bool spline = std::strcmp(t.kind, "spline") == 0;
+        if (!spline && arc && shared_origin()) return false;
+        return tile_launch(t.nchunks, tune, spline, true).tile_lines == 1 &&
+               tile_launch(t.nchunks, tune, spline, false).tile_lines == 1;
     }
 
     // Key of this scan's chunk visiting order (see ChunkOrders).
