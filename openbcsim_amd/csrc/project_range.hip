@@ -250,10 +250,35 @@ __global__ __launch_bounds__(1024, 8) void project_range_kernel(ProjCommon c, Cu
         // the patch's bounds: a line's coordinate differs from the patch axis's by at most
         // the distance times the largest difference of the axes (a relative 1e-5 for rounding)
         const float m_r = r_far * (patch.dr + 1e-5f), m_l = r_far * (patch.dl + 1e-5f), m_e = r_far * (patch.de + 1e-5f);
-        const float l_lo = P.l_min + ((float)G.l0 - 1.01f) * cp.lut_dl - m_l;
-        const float l_hi = P.l_min + ((float)G.l1 + 1.01f) * cp.lut_dl + m_l;
-        const float e_lo = P.e_min + ((float)G.e0 - 1.01f) * cp.lut_de - m_e;
-        const float e_hi = P.e_min + ((float)G.e1 + 1.01f) * cp.lut_de + m_e;
+        // the window's beam support, and the square of its largest distance from a beam's axis
+        const float l_lo = P.l_min + ((float)G.l0 - 1.01f) * cp.lut_dl, l_hi = P.l_min + ((float)G.l1 + 1.01f) * cp.lut_dl;
+        const float e_lo = P.e_min + ((float)G.e0 - 1.01f) * cp.lut_de, e_hi = P.e_min + ((float)G.e1 + 1.01f) * cp.lut_de;
+        const float l_far = fmaxf(fabsf(l_lo), fabsf(l_hi)), e_far = fmaxf(fabsf(e_lo), fabsf(e_hi));
+        const float reach2 = LUT ? l_far * l_far + e_far * e_far : cp.g_max / fminf(cp.g_a, cp.g_b);
+        // (A) One point per lane: can it reach a line of the patch (hit), and could one that it
+        // reaches see it behind the origin (behind)?  A line that sees a point within its support
+        // sees it at least sqrt(distance^2 - reach^2) before or behind the origin.
+        struct Seen {
+            bool hit, behind;
+        };
+        const auto test = [&](const float4& p, const float4& q) {
+            const float rc = dot_fused(p.x, p.y, p.z, patch.rx, patch.ry, patch.rz);
+            const float lc = dot_fused(p.x, p.y, p.z, patch.lx, patch.ly, patch.lz);
+            const float ec = dot_fused(p.x, p.y, p.z, patch.ex, patch.ey, patch.ez);
+            const float along = 0.9999f * __builtin_amdgcn_sqrtf(fmaxf(0.0f, q.x * q.x - 1.001f * reach2));
+            bool hit = rc > -m_r;
+            if (LUT) {
+                const float tr = (q.x - P.r_min) * P.inv_dr;
+                hit = hit && lc > l_lo - m_l && lc < l_hi + m_l && ec > e_lo - m_e && ec < e_hi + m_e &&
+                      G.l1 >= G.l0 && tr > -1.0f && tr < (float)(P.nr - 1);
+            } else {
+                const float dl = fmaxf(0.0f, fabsf(lc) - m_l), de = fmaxf(0.0f, fabsf(ec) - m_e);
+                hit = hit && !(cp.g_a * dl * dl + cp.g_b * de * de >= cp.g_max);
+            }
+            // points within about a sample of the origin may fall into bin 0 on the far side of it
+            const bool at_origin = __float_as_int(q.y) <= 1;
+            return Seen{hit || at_origin, at_origin || !(rc > m_r - along)};
+        };
         // The sums of the bin at hand of this lane's line, and its four bins finished last:
         // scalars of their own (a struct of them ends up in scratch memory).
         Acc re = Acc(0), im = Acc(0);
@@ -285,31 +310,18 @@ __global__ __launch_bounds__(1024, 8) void project_range_kernel(ProjCommon c, Cu
                 a = recs[2 * (size_t)i];
                 b = recs[2 * (size_t)i + 1];
             }
-            // (A) one point per lane: can it reach a line of the patch?
-            const float rc = dot_fused(p.x, p.y, p.z, patch.rx, patch.ry, patch.rz);
-            const float lc = dot_fused(p.x, p.y, p.z, patch.lx, patch.ly, patch.lz);
-            const float ec = dot_fused(p.x, p.y, p.z, patch.ex, patch.ey, patch.ez);
             const int bin = __float_as_int(q.y) - (b0 + w0);
-            // Points within about a sample of the origin may fall into bin 0 on the far side of it.
-            const bool at_origin = __float_as_int(q.y) <= 1;
-            bool hit = rc > -m_r;
+            const Seen seen = test(p, q);
             float fr = 0.0f;
             int off = 0;
             if (LUT) {
-                hit = hit && lc > l_lo && lc < l_hi && ec > e_lo && ec < e_hi && G.l1 >= G.l0;
                 const float tr = (q.x - P.r_min) * P.inv_dr;
-                hit = hit && tr > -1.0f && tr < (float)(P.nr - 1);
                 const int r0 = (int)tr;  // truncates: a coordinate in (-1, 0) reads slice 0 alone
                 fr = fmaxf(tr - (float)r0, 0.0f);
                 off = 8 * min(max(r0 - G.s0, 0), G.ns - 2) * plane;  // bytes
-            } else {
-                const float dl = fmaxf(0.0f, fabsf(lc) - m_l), de = fmaxf(0.0f, fabsf(ec) - m_e);
-                hit = hit && !(cp.g_a * dl * dl + cp.g_b * de * de >= cp.g_max);
             }
-            // points that some line may see behind the origin wait for the end
-            const bool behind = at_origin || !(rc > m_r);
-            far_side = far_side || __any(in && (behind && (hit || at_origin)));
-            unsigned long long mask = __ballot(in && hit && !behind);
+            far_side = far_side || __any(in && seen.hit && seen.behind);  // for the end
+            unsigned long long mask = __ballot(in && seen.hit && !seen.behind);
             // (B) one line per lane: the points one by one
             while (mask) {
                 const int k = __builtin_ctzll(mask);
@@ -364,33 +376,39 @@ __global__ __launch_bounds__(1024, 8) void project_range_kernel(ProjCommon c, Cu
             // The points set aside, by the tile kernel's rule: the side of the origin that a line
             // sees a point on decides its distance and bin.  Their bins are this wave's, or bin 0
             // from bin 1 (both in the line's first run), and stored by now.
-            for (int i = R.start[b0 + w0]; i < i1; i++) {
+            for (i0 = R.start[b0 + w0]; i0 < i1; i0 += 64) {
+                const int i = min(i0 + lane, i1 - 1);
                 const float4 p = recs[2 * (size_t)i], q = recs[2 * (size_t)i + 1];
-                const bool at_origin = __float_as_int(q.y) <= 1;
-                const float rc = dot_fused(p.x, p.y, p.z, patch.rx, patch.ry, patch.rz);
-                if (!at_origin && !(rc > -m_r && rc <= m_r)) continue;
-                if (!dst) continue;
-                const LineGeom& L = c.lines[line];
-                const Local o{p.x * L.rx + p.y * L.ry + p.z * L.rz, p.x * lx + p.y * ly + p.z * lz,
-                              p.x * ex + p.y * ey + p.z * ez};
-                const float r = copysignf(q.x, o.r);
-                int bn = __float_as_int(q.y);
-                float si = q.w;
-                if (r < 0.0f || (r == 0.0f && signbit(r))) {
-                    // the far side: bin 0, or none.  Its sub-sample delay is that of the near side
-                    // negated, or the same half sample where the near side rounds up to bin 1.
-                    if (bn == 0) si = -si;
-                    double ti;
-                    bn = at_origin ? radial_bin(c, r, ti) : -1;
+                const Seen seen = test(p, q);
+                unsigned long long mask = __ballot(i0 + lane < i1 && seen.hit && seen.behind);
+                while (mask) {
+                    const int k = __builtin_ctzll(mask);
+                    mask &= mask - 1;
+                    if (COUNT) n_pairs++;
+                    const float dx = read_lane(p.x, k), dy = read_lane(p.y, k), dz = read_lane(p.z, k);
+                    const LineGeom& L = c.lines[line];
+                    const Local o{dx * L.rx + dy * L.ry + dz * L.rz, dx * lx + dy * ly + dz * lz,
+                                  dx * ex + dy * ey + dz * ez};
+                    const float r = copysignf(read_lane(q.x, k), o.r);
+                    int bn = __builtin_amdgcn_readlane(__float_as_int(q.y), k);
+                    float si = read_lane(q.w, k);
+                    if (signbit(r)) {
+                        // the far side: bin 0, or none.  Its sub-sample delay is that of the near side
+                        // negated, or the same half sample where the near side rounds up to bin 1.
+                        if (bn == 0) si = -si;
+                        double ti;
+                        bn = bn <= 1 ? radial_bin(c, r, ti) : -1;
+                    }
+                    if (bn < 0 || !dst) continue;
+                    Tally t;
+                    const float w =
+                        (LUT ? lut_weight(P, r, o.l, o.e, t) : gauss_weight(P, o.l, o.e, t)) * read_lane(p.w, k);
+                    if (COUNT) n_evals += t.evals, n_adds += w != 0.0f ? (unsigned)E : 0u;
+                    if (w == 0.0f) continue;
+                    float* d = dst + (bn - b0 - w0) * E;
+                    d[0] += PHASE ? w * read_lane(q.z, k) : w;
+                    if (PHASE) d[1] += w * si;
                 }
-                if (bn < 0) continue;
-                Tally t;
-                const float w = (LUT ? lut_weight(P, r, o.l, o.e, t) : gauss_weight(P, o.l, o.e, t)) * p.w;
-                if (COUNT) n_pairs++, n_evals += t.evals, n_adds += w != 0.0f ? (unsigned)E : 0u;
-                if (w == 0.0f) continue;
-                float* d = dst + (bn - b0 - w0) * E;
-                d[0] += PHASE ? w * q.z : w;
-                if (PHASE) d[1] += w * si;
             }
         }
         if (COUNT) {

@@ -228,7 +228,7 @@ struct RangeLaunch {
     const float* table;       // the lookup table as [r][e][l], or null
     int max_slices;           // radial slices of it that a window can need
     int cell_floats;          // LDS floats of one staged radial cell
-    int run_bins;             // bins of a wave's run (a multiple of 4)
+    int run_bins;             // bins of a wave's run (even)
     int window_bins;          // bins of a workgroup's window (a multiple of run_bins)
     int group;                // patches of a workgroup
     int block;                // threads per workgroup

@@ -512,6 +512,7 @@ struct bcsim_sim {
     DevBuf d_lines, d_H, d_demod, d_tw, d_bins, d_iq;
     DevBuf d_patches;  // RangePatch[n_patches] of the lines' directions
     int n_patches = 0;
+    float patch_dl = 0.0f, patch_de = 0.0f;  // means of their dl and de
     bool dirty_patches = true;
     DevBuf d_stats;  // with store_kernel_details: per projection launch, weight evaluations and LDS additions
 
@@ -1864,6 +1865,8 @@ struct bcsim_sim {
         hip_check(hipMemcpy(d_patches.p, patches.data(), patches.size() * sizeof(RangePatch), hipMemcpyHostToDevice),
                   "hipMemcpy");
         n_patches = (int)patches.size();
+        patch_dl = patch_de = 0.0f;
+        for (const RangePatch& q : patches) patch_dl += q.dl / n_patches, patch_de += q.de / n_patches;
         dirty_patches = false;
     }
 
@@ -1891,25 +1894,47 @@ struct bcsim_sim {
             build_patches();
         }
         R.n_patches = n_patches;
-        R.run_bins = 4;  // one store of four bins; longer runs leave too few waves at the sizes of a 2D sector
+        // A patch's waves visit every point that reaches any of its lines.  Where few of its 64
+        // lanes have a line in reach of a point and each bin has many points, the tile kernel's
+        // visits (a line, 64 points of a chunk) are fewer: 38 lines over 70 degrees against 405k
+        // points 20.5 us a frame there, 26 here (lanes in use about 0.14); 128 lines against
+        // 100k 23 there, 15 here (0.30).  A table costs the tile kernel more than it does here.
+        const double per_bin = (double)t.n / num_rf;
+        const double mid = 0.5 * (double)line_length;
+        const auto share = [&](double beam, float turn) { return (beam + 1.5e-3) / (beam + mid * turn); };
+        const double beam_l = lut_profile ? 0.5 * std::fabs((double)lut_l1 - lut_l0) : std::sqrt(cp.g_max / cp.g_a);
+        const double beam_e = lut_profile ? 0.5 * std::fabs((double)lut_e1 - lut_e0) : std::sqrt(cp.g_max / cp.g_b);
+        const double lanes = (double)lines.size() / (kRangePatch * (double)n_patches) * share(beam_l, patch_dl) *
+                             share(beam_e, patch_de);
+        if (per_bin >= 16.0 && lanes < (lut_profile ? 0.1 : 0.2)) return R;
+        // A wave's run of bins: four, one store; two where that leaves fewer than 4096 waves and
+        // each has many points (225 lines x 218k points with a table 57 -> 54 us a frame, 163 x
+        // 437k 57 -> 53; 128 x 100k 15.1 -> 16.4, which keeps four).
+        const double runs4 = (double)n_patches * num_rf / 4.0;
+        R.run_bins = runs4 < 4096.0 && per_bin >= 16.0 ? 2 : 4;
         if (lut_profile) {
-            // A window spans less than two radial cells, so that the staged cells leave room
-            // for two workgroups of 16 waves on a CU; 16 patches share them.  (1M points, 4096
-            // lines, frames one after another: windows of 24 / 32 / 36 bins 0.852 / 0.874 /
-            // 0.876 ms, 8 or 32 patches 0.955 / 1.007.)
-            R.block = 1024;
-            R.group = 16;
-            for (R.window_bins = 24;; R.window_bins -= R.run_bins) {
+            // Sixteen patches or fewer share the staged cells.  Small cells: windows of 12 bins and
+            // 8 waves, several workgroups on a CU (1378 lines x 662k points, 32 x 32 samples a
+            // slice: 345 -> 313 us a frame against 24 bins and 16 waves).  Cells that leave room for
+            // two workgroups only: 24 and 16, as long as they span less than two radial cells and
+            // the two fit (1M-point volume, 64 x 64 samples: 834 us against 929).
+            const int groups = (n_patches + 15) / 16;
+            R.group = (n_patches + groups - 1) / groups;
+            const bool wide = 2 * R.cell_floats * sizeof(float) > (size_t)kLdsBytes / 4;
+            R.block = wide ? 1024 : 512;
+            for (R.window_bins = wide && R.run_bins == 4 ? 24 : 12;; R.window_bins -= R.run_bins) {
                 const double radial = (double)R.window_bins * (double)cp.r_per_bin * (double)t.c.prof.inv_dr;
                 R.max_slices = (int)std::min<double>(lut_nr, std::floor(radial + 2.0 * (1e-3 + 2e-6 * lut_nr)) + 3.0);
                 if (R.window_bins == R.run_bins || range_lds_bytes(R) <= (size_t)kLdsBytes / 2 - 512) break;
             }
             if (range_lds_bytes(R) > (size_t)kLdsBytes - 512) return R;
         } else {
-            // nothing to share: small workgroups of four waves, a patch and a run each
-            R.block = 256;
-            R.group = std::min(R.n_patches, 4);
-            R.window_bins = R.run_bins * (4 / R.group);
+            // nothing to share: a workgroup is one wave (409 lines x 247k points: 52 -> 42 us a
+            // frame against four), four where that makes few workgroups
+            const int waves = runs4 < 2048.0 ? 4 : 1;
+            R.block = 64 * waves;
+            R.group = std::min(n_patches, waves);
+            R.window_bins = R.run_bins * ((waves + R.group - 1) / R.group);
         }
         const RangeOrders::Key key{lines[0].ox, lines[0].oy, lines[0].oz, t.c.phase_per_sample, t.c.bin_scale, t.c.bin_denom};
         const auto sort = [&](RangeRec* recs, int* start, int* rank) {
