@@ -158,6 +158,12 @@ BCSIM_API bcsim_status bcsim_get_output_shape(bcsim_sim* sim, int* num_lines, in
 BCSIM_API bcsim_status bcsim_simulate_lines(bcsim_sim* sim, float* out, size_t capacity,
                                             int* num_lines, int* num_samples);
 
+/* bcsim_simulate_lines with the output as [sample][line]: the (num_samples,
+ * num_lines) array that pyrfsim's simulate_lines returns
+ * (src/python/PythonInterface.cpp:58-323). */
+BCSIM_API bcsim_status bcsim_simulate_lines_by_sample(bcsim_sim* sim, float* out, size_t capacity,
+                                                      int* num_lines, int* num_samples);
+
 /* Device-resident variant of simulate_lines: enqueues the frame on the
  * handle's stream with the IQ written to device memory d_out (complex64,
  * [line][sample]) and returns without waiting.  bcsim_synchronize waits. */

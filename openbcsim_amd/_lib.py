@@ -37,6 +37,7 @@ SIGNATURES = {
     "bcsim_set_lut_profile": [_h] + [C.c_float] * 6 + [_fp, C.c_int, C.c_int, C.c_int],
     "bcsim_get_output_shape": [_h, _ip, _ip],
     "bcsim_simulate_lines": [_h, _fp, C.c_size_t, _ip, _ip],
+    "bcsim_simulate_lines_by_sample": [_h, _fp, C.c_size_t, _ip, _ip],
     "bcsim_simulate_lines_device": [_h, C.c_void_p, C.c_size_t, _ip, _ip],
     "bcsim_simulate_lines_device_noalloc": [_h, C.c_void_p, C.c_size_t, _ip, _ip],
     "bcsim_synchronize": [_h],
@@ -88,6 +89,9 @@ def load(path: str = LIB_PATH):
         fn.argtypes = args
     _lib = lib
     return lib
+
+
+OUT_OF_MEMORY = 4  # BCSIM_ERR_OUT_OF_MEMORY
 
 
 class BcsimError(RuntimeError):

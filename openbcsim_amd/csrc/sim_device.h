@@ -142,6 +142,7 @@ struct ConvParams {
     int fold_log2;
     int out_stride;
     float2* iq;             // [L][n_out]
+    float2* turned;         // or null: the IQ as [n_out][L] too, once iq is written
     // additive noise on the bins before convolution (CpuAlgorithm.cpp:340-347)
     float noise_amplitude;
     uint32_t noise_seed;

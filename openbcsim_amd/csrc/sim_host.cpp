@@ -173,6 +173,15 @@ BCSIM_API bcsim_status bcsim_simulate_lines(bcsim_sim* sim, float* out, size_t c
     });
 }
 
+BCSIM_API bcsim_status bcsim_simulate_lines_by_sample(bcsim_sim* sim, float* out, size_t capacity, int* num_lines,
+                                                      int* num_samples) {
+    return guarded([&] {
+        need(sim);
+        if (!out) fail(BCSIM_ERR_INVALID_ARGUMENT, "null output buffer");
+        sim->simulate_host(out, capacity, num_lines, num_samples, true);
+    });
+}
+
 BCSIM_API bcsim_status bcsim_simulate_lines_device(bcsim_sim* sim, void* d_out, size_t capacity, int* num_lines,
                                                    int* num_samples) {
     return guarded([&] {

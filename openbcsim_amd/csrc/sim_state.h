@@ -509,7 +509,7 @@ struct bcsim_sim {
     bool dirty_scan = true, dirty_conv = true, dirty_basis = true;
     int num_rf = 0, fft_len = 0, log2_len = 0, n_out = 0;
     int tables_fft = 0, tables_out = 0;  // frame shape the convolution tables were built for
-    DevBuf d_lines, d_H, d_demod, d_tw, d_bins, d_iq;
+    DevBuf d_lines, d_H, d_demod, d_tw, d_bins, d_iq, d_iq_turned;
     DevBuf d_patches;  // RangePatch[n_patches] of the lines' directions
     int n_patches = 0;
     float patch_dl = 0.0f, patch_de = 0.0f;  // means of their dl and de
@@ -523,10 +523,10 @@ struct bcsim_sim {
             (void)hipStreamSynchronize(stream);
             (void)hipStreamDestroy(stream);
         }
-        for (int i = 0; i < 2; i++) {
-            if (stage[i]) (void)hipHostFree(stage[i]);
-            if (stage_ev[i]) (void)hipEventDestroy(stage_ev[i]);
-        }
+        for (void* p : stage)
+            if (p) (void)hipHostFree(p);
+        for (hipEvent_t e : stage_ev)
+            if (e) (void)hipEventDestroy(e);
     }
 
     void log(int level, const std::string& msg) {
@@ -799,7 +799,7 @@ struct bcsim_sim {
 
     // Device bytes this simulator holds for its frames (not the shared datasets).
     size_t frame_bytes() const {
-        size_t b = d_lines.bytes + d_H.bytes + d_demod.bytes + d_tw.bytes + d_bins.bytes + d_iq.bytes;
+        size_t b = d_lines.bytes + d_H.bytes + d_demod.bytes + d_tw.bytes + d_bins.bytes + d_iq.bytes + d_iq_turned.bytes;
         for (auto& sc : spline_scan) b += sc->basis.bytes + sc->rendered.bytes;
         return b;
     }
@@ -1969,8 +1969,9 @@ struct bcsim_sim {
 
     // Enqueue one frame.  fm: an allocation-free frame (its bins and rendered points
     // in the fixed scratch array; heuristic or user-set launch shapes, no tuning
-    // trials, no block-order buffers, no timing events).
-    void enqueue_frame(float2* d_out, FrameMem* fm = nullptr) {
+    // trials, no block-order buffers, no timing events).  turned: device memory for the
+    // IQ as [sample][line] as well, or null.
+    void enqueue_frame(float2* d_out, FrameMem* fm = nullptr, float2* turned = nullptr) {
         if (!fm) prepare();
         if (store_details || count_pairs) debug.clear();
         if (store_details) record_fused_keys();
@@ -2059,6 +2060,7 @@ struct bcsim_sim {
         ConvParams p = conv_params(d_out);
         p.bins = bins;
         p.radix = frame_radix;
+        p.turned = turned;
         {
             Timed t(this, "kernel_convolve_demodulate_ms", "kernel_forward_fft_ms");
             hip_check(launch_convolve_demod(p, stream), "convolve/demodulate kernel");
@@ -2171,20 +2173,24 @@ struct bcsim_sim {
         if (ns) *ns = n_out;
     }
 
-    void simulate_host(float* out, size_t capacity, int* nl, int* ns) {
+    // One frame into host memory, [line][sample] or, with by_sample, [sample][line].
+    void simulate_host(float* out, size_t capacity, int* nl, int* ns, bool by_sample = false) {
         prepare();
         last_frame_noalloc = false;
         const size_t need = lines.size() * (size_t)n_out;
         if (capacity < need) fail(BCSIM_ERR_CAPACITY, "output capacity too small");
-        d_iq.ensure(need * sizeof(float2));
-        enqueue_frame(d_iq.as<float2>());
         const size_t bytes = need * sizeof(float2);
+        d_iq.ensure(bytes);
+        if (by_sample) d_iq_turned.ensure(bytes);
+        float2* turned = by_sample ? d_iq_turned.as<float2>() : nullptr;
+        enqueue_frame(d_iq.as<float2>(), nullptr, turned);
+        const void* src = by_sample ? d_iq_turned.p : d_iq.p;
         if (bytes >= kStagedCopyMin && host_pageable(out)) {
-            copy_staged(out, d_iq.p, bytes);
+            copy_staged(out, src, bytes);
         } else {
             {
                 Timed t(this, "kernel_memcpy_ms");
-                hip_check(hipMemcpyAsync(out, d_iq.p, bytes, hipMemcpyDeviceToHost, stream), "hipMemcpyAsync");
+                hip_check(hipMemcpyAsync(out, src, bytes, hipMemcpyDeviceToHost, stream), "hipMemcpyAsync");
                 t.stop();
             }
             hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
@@ -2194,35 +2200,53 @@ struct bcsim_sim {
         if (ns) *ns = n_out;
     }
 
-    // Frames copied into pageable host memory pass through two pinned pieces of
-    // kStagePiece bytes: the DMA of piece c + 1 runs while host threads move piece
-    // c into the caller's buffer (the runtime's own path to pageable memory is
-    // about a third of the DMA rate).
-    static constexpr size_t kStagedCopyMin = (size_t)8 << 20;
+    // Frames copied into pageable host memory pass through pinned pieces: the DMA of the
+    // next pieces runs while the host moves one into the caller's buffer (the runtime's own
+    // path to pageable memory takes 0.33 ms for 1 MB and 0.18 for 3, this 0.06 and 0.13).
+    // Up to kStagePiece bytes are one pinned buffer in up to four pieces; more, two buffers
+    // of kStagePiece by turns, whose pieces several host threads move.
+    static constexpr size_t kStagedCopyMin = (size_t)128 << 10;
     static constexpr size_t kStagePiece = (size_t)32 << 20;
+    static constexpr int kStagePieces = 4;
     void* stage[2] = {nullptr, nullptr};
-    hipEvent_t stage_ev[2] = {nullptr, nullptr};
+    size_t stage_bytes[2] = {0, 0};
+    hipEvent_t stage_ev[kStagePieces] = {};
+
+    void ensure_stage(int i, size_t bytes) {
+        if (bytes <= stage_bytes[i]) return;
+        if (stage[i]) (void)hipHostFree(stage[i]);
+        stage[i] = nullptr;
+        stage_bytes[i] = 0;
+        hip_check(hipHostMalloc(&stage[i], bytes, 0), "hipHostMalloc");
+        stage_bytes[i] = bytes;
+    }
 
     void copy_staged(void* dst, const void* src, size_t bytes) {
-        for (int i = 0; i < 2; i++) {
-            if (!stage[i]) hip_check(hipHostMalloc(&stage[i], kStagePiece, 0), "hipHostMalloc");
-            if (!stage_ev[i]) hip_check(hipEventCreateWithFlags(&stage_ev[i], hipEventDisableTiming), "hipEventCreate");
-        }
-        const size_t pieces = (bytes + kStagePiece - 1) / kStagePiece;
-        auto piece_len = [&](size_t c) { return std::min(kStagePiece, bytes - c * kStagePiece); };
+        for (auto& e : stage_ev)
+            if (!e) hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
+        const bool small = bytes <= kStagePiece;
+        ensure_stage(0, small ? bytes : kStagePiece);
+        if (!small) ensure_stage(1, kStagePiece);
+        // pieces of about 768 KiB in one buffer, or whole buffers by turns
+        const size_t count = std::min<size_t>(kStagePieces, std::max<size_t>(1, bytes / ((size_t)768 << 10)));
+        const size_t piece = small ? ((bytes + count - 1) / count + 255) & ~(size_t)255 : kStagePiece;
+        const size_t pieces = (bytes + piece - 1) / piece;
+        const int ahead = small ? (int)pieces : 2;  // pieces that may be under way
+        auto piece_len = [&](size_t c) { return std::min(piece, bytes - c * piece); };
+        auto staged = [&](size_t c) { return small ? (char*)stage[0] + c * piece : (char*)stage[c % 2]; };
         auto issue = [&](size_t c) {
-            hip_check(hipMemcpyAsync(stage[c % 2], (const char*)src + c * kStagePiece, piece_len(c),
-                                     hipMemcpyDeviceToHost, stream),
+            hip_check(hipMemcpyAsync(staged(c), (const char*)src + c * piece, piece_len(c), hipMemcpyDeviceToHost, stream),
                       "hipMemcpyAsync");
-            hip_check(hipEventRecord(stage_ev[c % 2], stream), "hipEventRecord");
+            hip_check(hipEventRecord(stage_ev[c % ahead], stream), "hipEventRecord");
         };
         Timed t(this, "kernel_memcpy_ms");
-        issue(0);
+        size_t issued = 0;
         for (size_t c = 0; c < pieces; c++) {
-            if (c + 1 < pieces) issue(c + 1);  // its pinned piece was emptied in the previous round
-            if (c + 1 == pieces) t.stop();
-            hip_check(hipEventSynchronize(stage_ev[c % 2]), "hipEventSynchronize");
-            parallel_copy((char*)dst + c * kStagePiece, stage[c % 2], piece_len(c));
+            // a buffer's earlier piece was moved out in an earlier turn
+            for (; issued < pieces && issued < c + ahead; issued++) issue(issued);
+            if (issued == pieces) t.stop();
+            hip_check(hipEventSynchronize(stage_ev[c % ahead]), "hipEventSynchronize");
+            parallel_copy((char*)dst + c * piece, staged(c), piece_len(c));
         }
         hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
     }

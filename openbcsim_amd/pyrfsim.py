@@ -18,7 +18,7 @@ import ctypes as C
 import numpy as np
 
 from . import _lib
-from ._lib import BcsimError, check
+from ._lib import OUT_OF_MEMORY, BcsimError, check
 
 __all__ = ["RfSimulator", "BcsimError"]
 
@@ -159,7 +159,17 @@ class RfSimulator:
 
     def simulate_lines(self) -> np.ndarray:
         """IQ frame as complex64 (num_samples, num_lines), like the reference binding."""
-        return np.ascontiguousarray(self.simulate_frame().T)
+        L, S = self.output_shape()
+        out = np.empty((S, L), np.complex64)
+        nl, ns = C.c_int(), C.c_int()
+        try:
+            check(self._lib.bcsim_simulate_lines_by_sample(self._h, out.ctypes.data_as(C.POINTER(C.c_float)), out.size,
+                                                           C.byref(nl), C.byref(ns)))
+        except BcsimError as e:
+            if e.status != OUT_OF_MEMORY:
+                raise
+            out[:] = self.simulate_frame().T  # no room on the device for the IQ in both orders
+        return out
 
     def simulate_lines_device(self, device_ptr: int, capacity: int):
         """Enqueue a frame whose IQ goes to device memory at device_ptr; returns (L, S)."""

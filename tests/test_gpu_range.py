@@ -126,6 +126,20 @@ def test_several_datasets_accumulate(lut):
     check(wl)
 
 
+@pytest.mark.parametrize("lines,decimation", [(1, 1), (33, 3), (96, 1), (700, 2)])
+def test_frame_by_sample_is_the_frame_turned(lines, decimation):
+    """simulate_lines' (samples, lines) array is simulate_frame's transposed, for host copies
+    below, at and above the sizes where they pass through pinned pieces."""
+    from openbcsim_amd.pyrfsim import RfSimulator
+    g = RfSimulator("gpu")
+    W.fixed_sector_2d(3000, lines, seed=13, decimation=decimation).apply(g)
+    a = g.simulate_frame()
+    b = g.simulate_lines()
+    assert b.shape == a.T.shape and b.flags.c_contiguous and b.dtype == np.complex64
+    assert np.abs(a).max() > 0 and rel_l2(b, a.T) < 1e-6
+    g.close()
+
+
 def test_changes_between_frames():
     """New directions, time, length, origin and demodulation between frames of one simulator:
     each frame equals a new simulator's."""
