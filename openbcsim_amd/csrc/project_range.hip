@@ -47,10 +47,6 @@ namespace bcsim_hip {
 
 // ---- sort ----------------------------------------------------------------------
 
-__global__ __launch_bounds__(256) void range_clear_kernel(int* __restrict__ start) {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i <= kRangeBins; i += gridDim.x * blockDim.x) start[i] = 0;
-}
-
 // Bin of point i among its distance's points, or -1 (outside every line).
 __device__ __forceinline__ int range_bin(const ProjCommon& c, const float4& p, float ox, float oy, float oz, float3& d,
                                          float& absd, double& ti) {
@@ -59,8 +55,8 @@ __device__ __forceinline__ int range_bin(const ProjCommon& c, const float4& p, f
     return radial_bin(c, absd, ti);
 }
 
-// start[b + 1] counts the points of bin b; rank[i]: point i's place among them.
-__global__ __launch_bounds__(256) void range_count_kernel(ProjCommon c, FixedSet s, int* __restrict__ start,
+// Adds the points of each bin to count; rank[i]: point i's place among its bin's.
+__global__ __launch_bounds__(256) void range_count_kernel(ProjCommon c, FixedSet s, int* __restrict__ count,
                                                           int* __restrict__ rank) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= s.n) return;
@@ -69,17 +65,23 @@ __global__ __launch_bounds__(256) void range_count_kernel(ProjCommon c, FixedSet
     float absd;
     double ti;
     const int bin = range_bin(c, s.pts[i], L.ox, L.oy, L.oz, d, absd, ti);
-    rank[i] = bin >= 0 ? atomicAdd(&start[bin + 1], 1) : -1;
+    rank[i] = bin >= 0 ? atomicAdd(&count[bin], 1) : -1;
 }
 
-// Counts to first positions, in place: start[b] = points of the bins before b.
-__global__ __launch_bounds__(1024) void range_scan_kernel(int* __restrict__ start) {
+// start[b] = points of the bins before b; the counts go back to zero for the next sort.
+__global__ __launch_bounds__(1024) void range_scan_kernel(int* __restrict__ count, int* __restrict__ start) {
     constexpr int Q = kRangeBins / 1024;
     __shared__ int wsum[16];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int4* mine = reinterpret_cast<int4*>(count + threadIdx.x * Q);
     int v[Q], sum = 0;
 #pragma unroll
-    for (int q = 0; q < Q; q++) sum += (v[q] = start[1 + threadIdx.x * Q + q]);
+    for (int q = 0; q < Q / 4; q++) {
+        const int4 c = mine[q];
+        v[4 * q] = c.x, v[4 * q + 1] = c.y, v[4 * q + 2] = c.z, v[4 * q + 3] = c.w;
+        sum += c.x + c.y + c.z + c.w;
+        mine[q] = make_int4(0, 0, 0, 0);
+    }
     int incl = sum;
     for (int d = 1; d < 64; d <<= 1) {
         const int t = __shfl_up(incl, d);
@@ -89,6 +91,7 @@ __global__ __launch_bounds__(1024) void range_scan_kernel(int* __restrict__ star
     __syncthreads();
     int run = incl - sum;
     for (int w = 0; w < wave; w++) run += wsum[w];
+    if (threadIdx.x == 0) start[0] = 0;
 #pragma unroll
     for (int q = 0; q < Q; q++) start[1 + threadIdx.x * Q + q] = (run += v[q]);
 }
@@ -439,9 +442,8 @@ hipError_t launch_range_sort(const ProjCommon& c_in, const FixedSet& s, const Ra
     ProjCommon c = c_in;
     c.num_rf = kRangeBins;  // every bin a line of any length can have
     const dim3 grid((s.n + 255) / 256), block(256);
-    hipLaunchKernelGGL(range_clear_kernel, dim3(32), block, 0, stream, R.start);
-    hipLaunchKernelGGL(range_count_kernel, grid, block, 0, stream, c, s, R.start, R.rank);
-    hipLaunchKernelGGL(range_scan_kernel, dim3(1), dim3(1024), 0, stream, R.start);
+    hipLaunchKernelGGL(range_count_kernel, grid, block, 0, stream, c, s, R.count, R.rank);
+    hipLaunchKernelGGL(range_scan_kernel, dim3(1), dim3(1024), 0, stream, R.count, R.start);
     hipLaunchKernelGGL(range_scatter_kernel, grid, block, 0, stream, c, s, R.start, R.rank, R.recs);
     return hipGetLastError();
 }

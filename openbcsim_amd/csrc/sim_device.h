@@ -224,6 +224,7 @@ struct RangeLaunch {
     RangeRec* recs;           // points sorted by bin, or null: the tile kernel runs
     int* start;               // [kRangeBins + 1]: first record of each bin
     int* rank;                // [n] scratch of the sort
+    int* count;               // [kRangeBins] points per bin: zeros before and after a sort
     const RangePatch* patches;
     int n_patches;
     const float* table;       // the lookup table as [r][e][l], or null

@@ -184,11 +184,11 @@ struct RangeOrders {
         auto o = std::make_unique<Order>();
         o->key = key;
         try {
-            DevBuf rank;
+            DevBuf scratch;
             o->recs.ensure(n * sizeof(RangeRec));
             o->start.ensure((kRangeBins + 1) * sizeof(int));
-            rank.ensure(n * sizeof(int));
-            (*sort)(o->recs.as<RangeRec>(), o->start.as<int>(), rank.as<int>());
+            scratch.ensure((kRangeBins + n) * sizeof(int));
+            (*sort)(o->recs.as<RangeRec>(), o->start.as<int>(), scratch.as<int>());
         } catch (const BcsimError& e) {
             if (e.code != BCSIM_ERR_OUT_OF_MEMORY) throw;
             (void)hipGetLastError();
@@ -235,6 +235,7 @@ struct SplineScan {
     DevBuf basis;     // SplineLineBasis[num_lines]
     DevBuf rendered;  // float4[n], all-timestamps-equal path (culled with the dataset's boxes,
                       // since a rendered point lies in the box of its control points)
+    DevBuf recs, sort;  // the rendered points in range order, and their sort's counts and ranks
 };
 
 // Largest |a[i * stride]| over n values (infinite if one of them is not
@@ -800,7 +801,7 @@ struct bcsim_sim {
     // Device bytes this simulator holds for its frames (not the shared datasets).
     size_t frame_bytes() const {
         size_t b = d_lines.bytes + d_H.bytes + d_demod.bytes + d_tw.bytes + d_bins.bytes + d_iq.bytes + d_iq_turned.bytes;
-        for (auto& sc : spline_scan) b += sc->basis.bytes + sc->rendered.bytes;
+        for (auto& sc : spline_scan) b += sc->basis.bytes + sc->rendered.bytes + sc->recs.bytes + sc->sort.bytes;
         return b;
     }
 
@@ -1871,18 +1872,27 @@ struct bcsim_sim {
     }
 
     // Projection of target t in range order (project_range.hip), or a launch without
-    // records: the tile kernel runs.  It takes arc projection of fixed points onto
-    // lines of one origin, when nothing in the tile kernel's shape was set by hand,
-    // the amplitudes and the table are finite (its skipped pairs then add exactly 0)
-    // and the slices of a window fit LDS.
-    RangeLaunch range_launch(const ProjTarget& t, const FixedDataset* ds, const TileLaunch& shape, float* bins,
-                             bool create) {
+    // records: the tile kernel runs.  It takes arc projection of points (fixed ones, or
+    // splines rendered for the frame) onto lines of one origin, when nothing in the tile
+    // kernel's shape was set by hand, the amplitudes and the table are finite (its
+    // skipped pairs then add exactly 0) and the slices of a window fit LDS.
+    RangeLaunch range_launch(const ProjTarget& t, const TileLaunch& shape, float* bins, bool create) {
         RangeLaunch R{};
         const bool lut_profile = profile == kProfileLut;
         const bool by_hand = tune.windows || tune.lines || tune.block || tune.slices || bin_mode;
-        if (!ds || direct_mode || !arc || by_hand || (int)lines.size() < kRangeMinLines || !std::isfinite(t.c.prof.w_cut) ||
-            !std::isfinite(ds->peak_amp) || !shared_origin())
+        const bool rendered = std::strcmp(t.kind, "rendered") == 0;
+        if (std::strcmp(t.kind, "spline") == 0 || direct_mode || !arc || by_hand || (int)lines.size() < kRangeMinLines ||
+            !std::isfinite(t.c.prof.w_cut) || !std::isfinite(rendered ? t.sp->peak_amp : t.fixed->peak_amp) ||
+            !shared_origin())
             return R;
+        if (rendered) {
+            // Their sort costs about 20 us a frame, which many (point, line) pairs earn: frames of
+            // 512 lines x 200k splines 111 -> 54 us (with a table 221 -> 74), 512 x 10k 30 -> 30
+            // (38 -> 30), 128 x 200k 33 -> 35 (60 -> 42), 128 x 40k 17 -> 19 (23 -> 21), 32 x 200k
+            // 17 -> 17 (26 -> 33).
+            const double pairs = (double)t.n * (double)lines.size();
+            if (!create || lines.size() < (lut_profile ? 96 : 160) || pairs < (lut_profile ? 5e6 : 1e7)) return R;
+        }
         const CullParams cp = cull_params(t.c);
         if (lut_profile) {
             if (!lut_rel || !(cp.lut_dl > 0.0f)) return R;
@@ -1936,18 +1946,42 @@ struct bcsim_sim {
             R.group = std::min(n_patches, waves);
             R.window_bins = R.run_bins * ((waves + R.group - 1) / R.group);
         }
+        if (rendered) {  // other points every frame: sorted by each, into this simulator's buffers
+            try {
+                t.scan->recs.ensure(t.n * sizeof(RangeRec));
+                DevBuf& w = t.scan->sort;
+                const size_t ints = 2 * kRangeBins + 4 + t.n;  // count, start, rank
+                if (w.bytes < ints * sizeof(int)) {
+                    w.ensure(ints * sizeof(int));
+                    hip_check(launch_fill_zero(w.as<float>(), kRangeBins, stream), "fill kernel");
+                }
+                R.count = w.as<int>();
+                R.start = R.count + kRangeBins;
+                R.rank = R.start + kRangeBins + 4;
+            } catch (const BcsimError& e) {
+                if (e.code != BCSIM_ERR_OUT_OF_MEMORY) throw;
+                (void)hipGetLastError();
+                return RangeLaunch{};
+            }
+            R.sort = 1;
+            R.patches = d_patches.as<RangePatch>();
+            R.recs = t.scan->recs.as<RangeRec>();
+            return R;
+        }
         const RangeOrders::Key key{lines[0].ox, lines[0].oy, lines[0].oz, t.c.phase_per_sample, t.c.bin_scale, t.c.bin_denom};
-        const auto sort = [&](RangeRec* recs, int* start, int* rank) {
+        const auto sort = [&](RangeRec* recs, int* start, int* scratch) {
             TileLaunch g = shape;
             g.range = R;
             g.range.recs = recs;
             g.range.start = start;
-            g.range.rank = rank;
+            g.range.count = scratch;
+            g.range.rank = scratch + kRangeBins;
             g.range.sort = 2;
+            hip_check(launch_fill_zero(reinterpret_cast<float*>(scratch), kRangeBins, stream), "fill kernel");
             launch_target(t, g, bins);
             hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
         };
-        const RangeOrders::Order* o = ds->by_range.get(key, ds->n, create ? &sort : nullptr);
+        const RangeOrders::Order* o = t.fixed->by_range.get(key, t.n, create ? &sort : nullptr);
         if (!o) return R;
         R.patches = d_patches.as<RangePatch>();
         R.start = o->start.as<int>();
@@ -1993,7 +2027,7 @@ struct bcsim_sim {
             } else {
                 plans.push_back(plan_tile(t, autotune && !fm));
                 TileLaunch& g = plans.back();
-                g.range = range_launch(t, t.fixed, g, bins, fm == nullptr);
+                g.range = range_launch(t, g, bins, fm == nullptr);
                 last_plan += std::string(t.kind) + (t.ss.iboxes ? " (interval boxes)" : "") +
                              ": lines=" + std::to_string(g.tile_lines) +
                              " block=" + std::to_string(g.block) + " slices=" + std::to_string(g.slices) +

@@ -126,6 +126,31 @@ def test_several_datasets_accumulate(lut):
     check(wl)
 
 
+@pytest.mark.parametrize("splines,lines,lut", [(70001, 200, False), (60000, 128, True)])
+def test_rendered_splines(splines, lines, lut):
+    """Splines at one time are sorted for every frame: frames at several times, and a frame
+    after another simulator's, equal the tile kernel's."""
+    from openbcsim_amd.pyrfsim import RfSimulator
+    wl = W.spline_mmode(splines, lines, seed=12, all_timestamps_equal=True, line_length=0.05, phase_delay=True)
+    for s in wl.splines:
+        s.control_points *= np.float32(0.45)
+    if lut:
+        wl.profile = table(40, 24, 0.05)
+    g = RfSimulator("gpu")
+    wl.apply(g)
+    o, d, l, _, length = wl.scan
+    for t in (0.1, 0.83, 0.1):
+        ts = np.full(lines, t, np.float32)
+        wl.scan = (o, d, l, ts, length)
+        g.set_scan_sequence(o, d, length, l, ts, True)
+        a = g.simulate_frame()
+        assert "range order" in g.get_parameter("launch_plan")
+        b, plan = frame(wl, tile_lines="1")
+        assert "range order" not in plan and rel_l2(a, b) < 1e-6
+        assert np.array_equal(g.simulate_lines(), g.simulate_frame().T) or rel_l2(g.simulate_lines(), a.T) < 1e-6
+    g.close()
+
+
 @pytest.mark.parametrize("lines,decimation", [(1, 1), (33, 3), (96, 1), (700, 2)])
 def test_frame_by_sample_is_the_frame_turned(lines, decimation):
     """simulate_lines' (samples, lines) array is simulate_frame's transposed, for host copies
