@@ -151,7 +151,57 @@ struct ConvParams {
     // frames: launch_fill_segments advances it at the start of every frame)
     const uint32_t* noise_counter_ptr;
     int radix;              // largest FFT pass radix: 4 or 8
+    // twiddles of the transforms of constant length (conv_roots_size), or null
+    const float2* roots;
 };
+
+// The complex transform of all N points: complex bins (phase delay) or noise.  Other
+// frames have real bins, transformed as N/2 complex points.
+__host__ __device__ inline bool conv_full(const ConvParams& p) { return p.complex_bins || p.noise_amplitude > 0.0f; }
+
+// ---- transforms of constant length (convolve_fixed.hip) ----
+
+constexpr int kConvFixedMin = 11, kConvFixedMax = 14;  // log2 of the lengths
+constexpr int kConvFixedFolds = 3;                     // fold_log2 0 .. 2
+
+// The passes of a forward transform of 2^log2n points, and log2 of the radix of pass i: 16s, then
+// 8s, as few as there can be.  Packed real transforms end with an 8: a thread holds two of the
+// last butterflies.
+__host__ __device__ constexpr int conv_passes(int log2n) { return log2n == 12 ? 4 : (log2n + 3) / 4; }
+__host__ __device__ constexpr int conv_radix_log2(int log2n, int i) {
+    const int passes = conv_passes(log2n);
+    return i < log2n - 3 * passes ? 4 : 3;
+}
+
+// Sixteen points a thread of the longer transform: frames of many lines keep four waves a
+// SIMD in registers and LDS.
+__host__ __device__ constexpr int conv_fixed_threads(int log2n, bool full, int fold) {
+    return 1 << (full || fold == 0 ? log2n - 4 : log2n - 5);
+}
+
+// The twiddles of a frame: for each pass of the forward transform but the last, over blocks of B
+// points with radix R, exp(-2 pi i s j / B) as [R - 1][B / R]; the same for the passes of the
+// inverse transform (its radices are the forward ones, the last one scaled to its length;
+// from the longest block on; the kernel conjugates them); exp(-2 pi i k / N) for the
+// butterflies k of the forward transform's last pass.
+struct ConvRoots {
+    int forward, last, inverse, inverse_first;  // points and last (first) radices, log2
+};
+__host__ __device__ constexpr ConvRoots conv_roots_shape(int log2n, bool full, int fold) {
+    const int f = full ? log2n : log2n - 1, r = conv_radix_log2(f, conv_passes(f) - 1);
+    return ConvRoots{f, r, log2n - fold, log2n - fold - (f - r)};
+}
+__host__ __device__ constexpr int conv_roots_size(int log2n, bool full, int fold) {
+    const ConvRoots s = conv_roots_shape(log2n, full, fold);
+    return (1 << s.forward) - (1 << s.last) + (1 << s.inverse) - (1 << s.inverse_first) + (1 << (s.forward - s.last));
+}
+
+// The constant lengths are the faster from 2^12 points on (figures in convolve_fixed.hip) and
+// within 1 us of conv_line at 2^11; noise, radix 4, other lengths and deeper folds take conv_line.
+__host__ __device__ inline bool conv_fixed(const ConvParams& p) {
+    return p.roots && p.radix == 8 && p.log2_len >= kConvFixedMin && p.log2_len <= kConvFixedMax &&
+           p.fold_log2 < kConvFixedFolds && p.num_rf >= 2 && !(p.noise_amplitude > 0.0f);
+}
 
 // LDS points (float2) of one line's convolution buffer; its twiddle table follows
 // it.  Real bins without noise, folded (fold_log2 >= 1): the N/2-point transform
@@ -164,8 +214,7 @@ __host__ __device__ inline int conv_slot(int i) { return i + (i >> kConvPadShift
 
 // LDS float2 slots of the convolution's transform buffer (padded).
 __host__ __device__ inline int conv_buffer_len(const ConvParams& p) {
-    const bool real_in = !p.complex_bins && !(p.noise_amplitude > 0.0f);
-    return conv_slot((real_in && p.fold_log2 > 0) ? p.fft_len / 2 : p.fft_len);
+    return conv_slot((!conv_full(p) && p.fold_log2 > 0) ? p.fft_len / 2 : p.fft_len);
 }
 
 // ---- culled tile projection (project_tile.hip) ----
@@ -331,6 +380,10 @@ hipError_t launch_render_spline(const SplineSet& s, const SplineLineBasis& basis
                                 hipStream_t stream);
 hipError_t launch_convolve_demod(const ConvParams& p, hipStream_t stream);
 int conv_block_threads(int fft_len);
+// Frames of constant-length transforms (conv_fixed), convolve_fixed.hip.
+hipError_t launch_convolve_fixed(const ConvParams& p, hipStream_t stream);
+hipError_t launch_convolve_fixed_batch(int variant, const ConvParams* jobs, const int2* items, int n_items, size_t lds,
+                                       hipStream_t stream);
 
 // project_tile.hip: fixed (spline == nullptr) or spline dataset, chunked and
 // boxed by the host; `shared_origin` when every line starts at lines[0]'s origin.
@@ -361,16 +414,22 @@ inline int batch_variant(int flags) {
 }
 
 // LDS bytes of one line's convolution: the padded transform buffer and the
-// two-level twiddle table.
+// two-level twiddle table (constant lengths: only the buffer).
 __host__ __device__ inline size_t conv_lds_bytes(const ConvParams& p) {
+    if (conv_fixed(p)) return (size_t)(!conv_full(p) && p.fold_log2 > 0 ? p.fft_len / 2 : p.fft_len) * sizeof(float2);
     return ((size_t)conv_buffer_len(p) + (size_t)(p.fft_len >> p.twiddle_bits) + ((size_t)1 << p.twiddle_bits)) *
            sizeof(float2);
 }
 
 // Kernel variant of a batched convolution job: workgroup size class (1024 threads
-// for FFTs of 4096 points and more, else 256), radix and bin kind.
-enum ConvVariant { kConvComplex = 1, kConvRadix8 = 2, kConvWide = 4 };
+// for FFTs of 4096 points and more, else 256), radix and bin kind; or the constant
+// length, fold and kind of transform.
+enum ConvVariant { kConvComplex = 1, kConvRadix8 = 2, kConvWide = 4, kConvFixed = 8, kConvFull = 16 };
+inline int conv_variant_log2(int variant) { return kConvFixedMin + ((variant >> 5) & 3); }
+inline int conv_variant_fold(int variant) { return variant >> 7; }
 inline int conv_variant(const ConvParams& p, int block_threads) {
+    if (conv_fixed(p))
+        return kConvFixed | (conv_full(p) ? kConvFull : 0) | (p.log2_len - kConvFixedMin) << 5 | p.fold_log2 << 7;
     return (block_threads == 1024 ? kConvWide : 0) | (p.radix == 8 ? kConvRadix8 : 0) |
            (p.complex_bins ? kConvComplex : 0);
 }

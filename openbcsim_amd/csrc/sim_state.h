@@ -67,6 +67,42 @@ struct DevBuf {
     T* as() const { return static_cast<T*>(p); }
 };
 
+// The twiddles of constant-length transforms (sim_device.h, conv_roots_size) on a device, shared by
+// the simulators whose frames have that shape: immutable, freed with the last of them.
+struct ConvShape {
+    int log2n;
+    bool full;
+    int fold;
+    bool operator==(const ConvShape& o) const { return log2n == o.log2n && full == o.full && fold == o.fold; }
+};
+inline std::shared_ptr<DevBuf> conv_roots(int device, const ConvShape& c) {
+    static std::mutex mu;
+    static std::map<std::array<int, 4>, std::weak_ptr<DevBuf>> tables;
+    std::lock_guard<std::mutex> g(mu);
+    auto& slot = tables[{device, c.log2n, c.full ? 1 : 0, c.fold}];
+    if (auto t = slot.lock()) return t;
+    const int n = 1 << c.log2n;
+    std::vector<float2> unit(n), all;
+    for (int i = 0; i < n; i++) {
+        const double a = -2.0 * M_PI * (double)i / (double)n;
+        unit[i] = make_float2((float)std::cos(a), (float)std::sin(a));
+    }
+    const ConvRoots shape = conv_roots_shape(c.log2n, c.full, c.fold);
+    for (int block : {shape.forward, shape.inverse})
+        for (int i = 0; i + 1 < conv_passes(shape.forward); i++) {
+            const int r = conv_radix_log2(shape.forward, i);
+            for (int s = 1; s < (1 << r); s++)
+                for (int j = 0; j < (1 << (block - r)); j++) all.push_back(unit[(s * j) << (c.log2n - block)]);
+            block -= r;
+        }
+    all.insert(all.end(), unit.begin(), unit.begin() + (1 << (shape.forward - shape.last)));
+    auto t = std::make_shared<DevBuf>();
+    t->ensure(all.size() * sizeof(float2));
+    hip_check(hipMemcpy(t->p, all.data(), all.size() * sizeof(float2), hipMemcpyHostToDevice), "hipMemcpy");
+    slot = t;
+    return t;
+}
+
 // Datasets are stored in Morton (z-curve) order of position, in chunks of
 // kChunk scatterers with one bounding box each, so the tile kernel can skip
 // whole chunks that lie outside a beam.  The order of the scatterers does not
@@ -511,6 +547,8 @@ struct bcsim_sim {
     int num_rf = 0, fft_len = 0, log2_len = 0, n_out = 0;
     int tables_fft = 0, tables_out = 0;  // frame shape the convolution tables were built for
     DevBuf d_lines, d_H, d_demod, d_tw, d_bins, d_iq, d_iq_turned;
+    std::shared_ptr<DevBuf> roots;  // conv_roots of roots_shape, or null
+    ConvShape roots_shape{0, false, 0};
     DevBuf d_patches;  // RangePatch[n_patches] of the lines' directions
     int n_patches = 0;
     float patch_dl = 0.0f, patch_de = 0.0f;  // means of their dl and de
@@ -1177,6 +1215,14 @@ struct bcsim_sim {
             hip_check(hipMemcpy(d_lines.p, lines.data(), sizeof(LineGeom) * lines.size(), hipMemcpyHostToDevice),
                       "hipMemcpy");
             dirty_scan = dirty_conv = false;
+        }
+        const ConvShape shape = conv_shape();
+        if (!(roots_shape == shape)) {
+            quiesce();  // frames in flight may read the old table
+            roots.reset();
+            if (log2_len >= kConvFixedMin && log2_len <= kConvFixedMax && shape.fold < kConvFixedFolds)
+                roots = conv_roots(device, shape);
+            roots_shape = shape;
         }
         if (dirty_basis) {
             upload_spline_basis();
@@ -2102,6 +2148,14 @@ struct bcsim_sim {
         }
     }
 
+    // The inverse transform is folded by the largest power of two dividing the
+    // decimation, keeping at least 16 points.
+    ConvShape conv_shape() const {
+        int f = 0;
+        while (((decimation >> f) & 1) == 0 && log2_len - (f + 1) >= 4) f++;
+        return ConvShape{log2_len, phase_delay, f};
+    }
+
     // Arguments of the convolution of this frame (prepare() done); advances the
     // noise stream's frame counter.
     ConvParams conv_params(float2* d_out) {
@@ -2114,17 +2168,14 @@ struct bcsim_sim {
         p.log2_len = log2_len;
         p.twiddle_bits = log2_len / 2;
         p.twiddles = d_tw.as<float2>();
+        p.roots = roots && roots_shape == conv_shape() ? roots->as<float2>() : nullptr;
         p.H = d_H.as<float2>();
         p.demod = d_demod.as<float2>();
         p.center = center;
         p.decimation = decimation;
         p.n_out = n_out;
-        // fold the inverse transform by the largest power of two dividing the
-        // decimation, keeping at least 16 points
-        int f = 0;
-        while (((decimation >> f) & 1) == 0 && log2_len - (f + 1) >= 4) f++;
-        p.fold_log2 = f;
-        p.out_stride = decimation >> f;
+        p.fold_log2 = conv_shape().fold;
+        p.out_stride = decimation >> p.fold_log2;
         p.iq = d_out;
         p.noise_amplitude = noise_amplitude > 0.0f ? noise_amplitude : 0.0f;
         p.noise_seed = noise_seed;
