@@ -183,6 +183,11 @@ struct bcsim_batch {
         const double per_item = total / ((double)workgroups * items_per_workgroup);
         for (size_t k = 0; k < pjobs.size(); k++) {
             ProjJob& J = pjobs[k];
+            if (J.g.range.recs) {  // its items share the runs
+                J.g.slices = 1;
+                J.g.chunks_per_slice = J.nchunks;
+                continue;
+            }
             const double want_items = std::max(1.0, cost[k] / std::max(per_item, 1.0));
             int slices = (int)std::ceil(want_items / J.blocks_per_slice);
             slices = std::max(1, std::min(slices, std::max(1, J.nchunks / 16)));
@@ -235,7 +240,10 @@ struct bcsim_batch {
                 J.ss = t.ss;
                 J.boxes = t.boxes;
                 J.bins = s->d_bins.as<float>();
-                J.g = s->plan_tile(t, tune_now);
+                // one accumulation mode for jobs of a kind, whose launch they share (trials of like
+                // shapes differ by less than they scatter: 24 spline jobs in two launches 122 us,
+                // in one 106)
+                J.g = s->plan_tile(t, tune_now, false);
                 if (tile_lines > 0) {
                     TileTune tt = s->tune;
                     tt.lines = tile_lines;
@@ -245,14 +253,19 @@ struct bcsim_batch {
                 J.g.chunks = t.chunk_order;
                 J.g.chunk_dist = t.chunk_dist;
                 J.nchunks = t.nchunks;
+                // One dataset, a Gaussian beam: in range order where a frame of its own would be
+                // (48 jobs, half of them of about 25k points on 48 lines: these 85 -> 46 us).
+                // A table's staged cells would tie an item's waves to one window of one job.
+                if (targets.size() == 1 && !lut && tile_lines <= 0 && std::strcmp(t.kind, "fixed") == 0)
+                    J.g.range = s->range_launch(t, J.g, J.bins, true);
                 J.flags = (s->arc ? kJobArc : 0) | (cplx ? kJobPhase : 0) | (lut ? kJobLut : 0) |
                           (is_spline ? kJobSpline : 0) | (shared && !is_spline ? kJobShared : 0) |
-                          (J.g.fixed ? kJobFixed : 0);
+                          (J.g.fixed ? kJobFixed : 0) | (J.g.range.recs ? kJobRange : 0);
                 const int tiles = (t.c.num_lines + J.g.tile_lines - 1) / J.g.tile_lines;
                 J.blocks_per_slice = tiles * J.g.windows;
                 J.g.work = nullptr;
                 J.g.order = nullptr;
-                if (s->tile_order && J.blocks_per_slice >= kMinOrderedJobBlocks &&
+                if (s->tile_order && !J.g.range.recs && J.blocks_per_slice >= kMinOrderedJobBlocks &&
                     J.blocks_per_slice <= kMaxOrderedTiles) {
                     // the job's blocks in the order of the work they listed in the previous
                     // frame, heaviest first (counts in the simulator's own buffer: zeroed on
@@ -261,7 +274,7 @@ struct bcsim_batch {
                     ordered.push_back({(int)pjobs.size(), J.g.work});
                 }
                 pjobs.push_back(J);
-                pcost.push_back((double)t.nchunks * t.c.num_lines * (is_spline ? 3.0 : 1.0));
+                pcost.push_back((double)t.nchunks * t.c.num_lines * (is_spline ? 3.0 : J.g.range.recs ? 0.25 : 1.0));
                 if (std::strcmp(t.kind, "rendered") == 0) {
                     Render r{t.ss, {}, t.scan->rendered.as<float4>()};
                     s->host_basis_line0(*t.sp, r.basis);

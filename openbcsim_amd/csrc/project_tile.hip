@@ -890,6 +890,7 @@ static hipError_t launch_batch_kind(int kind, bool fixed, const ProjJob* jobs, c
 hipError_t launch_project_batch(int variant, const ProjJob* jobs, const int2* items, int n_items, int* counter,
                                 size_t lds, int workgroups, hipStream_t stream) {
     if (n_items == 0) return hipSuccess;
+    if (variant & kJobRange) return launch_range_batch(variant & kJobPhase, jobs, items, n_items, stream);
     const bool arc = variant & kJobArc, phase = variant & kJobPhase, lut = variant & kJobLut;
     const int kind = (variant & kJobSpline) ? 2 : (arc && (variant & kJobShared)) ? 1 : 0;
     const bool fixed = variant & kJobFixed;

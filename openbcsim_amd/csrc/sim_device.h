@@ -323,7 +323,8 @@ constexpr int kMaxOrderedTiles = 65536;
 
 // One projection job of a batch: a (simulator, dataset) pair with everything its
 // tile kernel would receive as arguments.
-enum JobFlags { kJobArc = 1, kJobPhase = 2, kJobLut = 4, kJobSpline = 8, kJobShared = 16, kJobFixed = 32 };
+enum JobFlags { kJobArc = 1, kJobPhase = 2, kJobLut = 4, kJobSpline = 8, kJobShared = 16, kJobFixed = 32,
+                kJobRange = 64 };  // projected in range order (J.g.range; a Gaussian beam, bins stored)
 
 struct ProjJob {
     ProjCommon c;
@@ -393,6 +394,8 @@ hipError_t launch_project_tile(const ProjCommon& c, const CullParams& cp, const 
                                hipStream_t stream);
 // project_range.hip: sorts the points s (lines[0]'s origin) into R's buffers; projects
 // them, storing every bin of every line or, with `accumulate`, adding to it.
+// The items of the range-order jobs of a batch (launch_project_batch).
+hipError_t launch_range_batch(bool phase, const ProjJob* jobs, const int2* items, int n_items, hipStream_t stream);
 hipError_t launch_range_sort(const ProjCommon& c, const FixedSet& s, const RangeLaunch& R, hipStream_t stream);
 hipError_t launch_project_range(const ProjCommon& c, const CullParams& cp, const RangeLaunch& R, float* out,
                                 bool phase, bool lut, int accumulate, unsigned long long* stats, hipStream_t stream);
@@ -408,6 +411,7 @@ hipError_t launch_order_segments(const OrderSeg* segs, int n_segs, hipStream_t s
 // The JobFlags that select projection code: arc, phase, LUT, spline, and a
 // shared origin (which only matters for fixed points with arc projection).
 inline int batch_variant(int flags) {
+    if (flags & kJobRange) return flags & (kJobRange | kJobArc | kJobPhase);
     int f = flags & (kJobArc | kJobPhase | kJobLut | kJobSpline | kJobShared | kJobFixed);
     if (!(f & kJobArc) || (f & kJobSpline)) f &= ~kJobShared;
     return f;

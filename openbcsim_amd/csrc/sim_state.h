@@ -1803,7 +1803,8 @@ struct bcsim_sim {
 
     // Launch shape for a target: shape fields set by the user win, then the
     // tuned shape (when tuning is on), then the heuristic.
-    TileLaunch plan_tile(const ProjTarget& t, bool tune_now) {
+    // tuned_bins: a trial's accumulation mode too (else target_fixed's rule).
+    TileLaunch plan_tile(const ProjTarget& t, bool tune_now, bool tuned_bins = true) {
         TileTune eff = tune;
         if (tune_now) {
             const TileTune tt = tuned_tile(t);
@@ -1811,7 +1812,7 @@ struct bcsim_sim {
             if (!eff.lines) eff.lines = tt.lines;
             if (!eff.block) eff.block = tt.block;
             if (!eff.slices) eff.slices = tt.slices;
-            eff.bins = tt.bins;
+            if (tuned_bins) eff.bins = tt.bins;
         }
         return tile_launch(t.nchunks, eff, std::strcmp(t.kind, "spline") == 0, target_fixed(t, eff.bins));
     }
@@ -1833,7 +1834,12 @@ struct bcsim_sim {
         noise_counter = counter;
         std::string trials;
         double best_ms = 0.0;
-        for (int cand : {4, 8}) {
+        p.radix = 8;
+        // Alone a small frame's time is latency, where radix 4 can come out ahead; the constant
+        // lengths issue about half the instructions (48 lines of 2^12 samples alone 8.9 us
+        // against 8.3, 24 such frames in one batch 15 against 40).
+        const int first = conv_fixed(p) ? 8 : 4;
+        for (int cand = first; cand <= 8; cand += 4) {
             p.radix = cand;
             const double ms =
                 time_launches(stream, [&] { hip_check(launch_convolve_demod(p, stream), "convolve"); }, 3, 2);

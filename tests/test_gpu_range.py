@@ -204,3 +204,30 @@ def test_counters_match_the_tile_kernel():
     assert abs(got[0][0] - got[1][0]) <= 1e-5 * got[1][0] + 2
     assert abs(got[0][1] - got[1][1]) <= 1e-5 * got[1][1] + 2
     assert 64 * got[0][2] >= got[0][0]
+
+
+def test_batch_jobs():
+    """Fixed points of a Gaussian beam in a batch: patches of one and several, runs of two and
+    four bins, phase delay, an odd last run, beside jobs of the tile kernels; equal to the tile
+    kernels' bins, and the same on a second frame and after the batch's jobs change."""
+    from openbcsim_amd.batch import Batch
+    from openbcsim_amd.pyrfsim import RfSimulator
+    sims = []
+    for n, lines, length, phase in ((5000, 16, 0.03, False), (25001, 48, 0.0601, True), (90000, 65, 0.02, False),
+                                    (8000, 200, 0.05, True), (3000, 9, 0.04, False)):
+        g = RfSimulator("gpu")
+        W.fixed_sector_2d(n, lines, seed=lines, line_length=length, phase_delay=phase).apply(g)
+        sims.append(g)
+    batch, tiles = Batch(sims), Batch(sims)
+    tiles.set_parameter("tile_lines", "1")
+    for g in sims:
+        assert ("range order" in (g.simulate_frame() is not None and g.get_parameter("launch_plan"))) == (g.output_shape()[0] >= 16)
+    want = tiles.simulate()
+    for _ in range(2):
+        for a, b in zip(batch.simulate(), want):
+            assert np.abs(b).max() > 0 and rel_l2(a, b) < 1e-6
+    sims[0].set_parameter("sound_speed", "1500")
+    for a, b in zip(batch.simulate(), tiles.simulate()):
+        assert rel_l2(a, b) < 1e-6
+    for x in (batch, tiles, *sims):
+        x.close()
