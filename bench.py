@@ -17,12 +17,14 @@ on the simulator's stream (store_kernel_details) over K frames.  `traffic` is it
 HBM bytes per launch from two rocprofv3 --pmc runs of this script in a child
 process (FETCH_SIZE, then WRITE_SIZE), each scaled by what the same counter reads
 for a plain copy kernel of known size; achieved = traffic / duration against the
-8 TB/s HBM peak.  Beside it, the units that bind the kernel: its own counts of
-profile-weight evaluations (LUT record gathers) and LDS float additions per
-launch, as rates against ceilings measured on the device by kernels of the same
-access shape (openbcsim_amd/ceilings.py), the busy fraction of the texture
-addresser and data units (a third counter run), and the per-line streaming model
-of the reference's kernel (16 B per scatterer evaluation) as a ratio to the peak.
+8 TB/s HBM peak.  Beside it, the units that bind the kernel (project_range_kernel
+where the launch plan says range order, else the line or tile kernel): VALU issue
+and HBM, and for the line and tile kernels their counts of profile-weight
+evaluations (LUT record gathers) and LDS additions per launch, as rates against
+ceilings measured on the device by kernels of the same access shape
+(openbcsim_amd/ceilings.py), the busy fraction of the texture addresser and data
+units (a third counter run), and the per-line streaming model of the reference's
+kernel (16 B per scatterer evaluation) as a ratio to the peak.
 
 cpu_baseline: the reference's own CPU algorithm (CpuAlgorithm, compiled from the
 reference sources into oracle/_ref) on a bounded sample of the same workload --
@@ -120,7 +122,10 @@ def run_gpu(wl, steps: int, warmup: int, tile=None, bins=None):
     for key in ("projection_weight_evals", "projection_lds_adds", "projection_chunk_line_pairs"):
         counts[key] = float(sum(sim.get_debug_data(key)))
     sim.set_parameter("projection_counters", "off")
-    counts["bins"] = "fixed" if "bins=fixed" in sim.get_parameter("launch_plan") else "float"
+    plan = sim.get_parameter("launch_plan")
+    ranged = "range order" in plan
+    counts["bins"] = "registers" if ranged else "fixed" if "bins=fixed" in plan else "float"
+    counts["kernel"] = PROJECTION_KERNELS[0 if ranged else 1 if ": lines=1 " in plan else 2]
     # PCIe-inclusive rate (host output), reported beside the device-resident value
     sim.simulate_frame()
     t2 = time.perf_counter()
@@ -642,6 +647,7 @@ def _pmc_values(out_dir: str):
 # they run apart; the SQ instruction counts ride along with the first
 PMC_PASSES = (("FETCH_SIZE", "SQ_INSTS_VALU", "SQ_INSTS_LDS", "SQ_INSTS_VMEM_RD"), ("WRITE_SIZE",),
               ("TD_TD_BUSY_sum", "TA_TA_BUSY_sum", "GRBM_GUI_ACTIVE"))
+PROJECTION_KERNELS = ("project_range_kernel", "project_line_kernel", "project_tile_kernel")
 # MI355X: GRBM_GUI_ACTIVE adds up the active cycles of its 8 accelerator complex dies
 XCDS = 8
 
@@ -700,11 +706,13 @@ def measure_traffic(workload: str, keep_dir=None):
         if not cal:
             return None, f"no copy_kernel dispatch in the {counter} run"
         scale[counter] = COPY_CALIBRATION_BYTES / (cal * 1024.0)  # bytes per KiB the counter reports
-    for name, substr in (("projection", "project_tile_kernel"), ("convolution", "convolve_demod_kernel")):
+    for name, substrs in (("projection", PROJECTION_KERNELS), ("convolution", ("conv_fixed_kernel", "convolve_demod_kernel"))):
+        # one of them ran every frame (a counter run has a few frames of one workload)
+        substr = max(substrs, key=lambda k: sum(len(v) for n, v in readings.get("FETCH_SIZE", {}).items() if k in n))
         f, w = pick("FETCH_SIZE", substr), pick("WRITE_SIZE", substr)
         if f is None or w is None:
             continue
-        res[name] = {"fetch_kib": f, "write_kib": w,
+        res[name] = {"kernel": substr, "fetch_kib": f, "write_kib": w,
                      "bytes": f * 1024.0 * scale["FETCH_SIZE"] + w * 1024.0 * scale["WRITE_SIZE"]}
         for c in PMC_PASSES[0][1:] + PMC_PASSES[2]:
             v = pick(c, substr)
@@ -718,15 +726,17 @@ def measure_traffic(workload: str, keep_dir=None):
     return res, None
 
 
-def roofline_object(wl, kind, L, proj_ms, counts, traffic, traffic_err, ceilings, fixed_bins=False):
+def roofline_object(wl, kind, L, proj_ms, counts, traffic, traffic_err, ceilings, fixed_bins=False,
+                    kernel="project_tile_kernel"):
     """The dominant kernel against HBM (measured bytes) and against the measured
     ceilings of the units its counters show busy: LDS atomics, LUT record
-    gathers and spline control-point loads (the launch's own counts), VALU issue (SQ_INSTS_VALU), and the texture
+    gathers and spline control-point loads (the launch's own counts; range order has
+    no atomics and looks its table up in LDS), VALU issue (SQ_INSTS_VALU), and the texture
     addresser and data units (their busy cycles per CU over the kernel's active
     cycles, from the counter run)."""
     N = wl.num_scatterers
     t = proj_ms * 1e-3
-    rl = {"bound": "hbm", "peak": HBM_PEAK_GBS, "unit": "GB/s", "kernel": "project_tile_kernel",
+    rl = {"bound": "hbm", "peak": HBM_PEAK_GBS, "unit": "GB/s", "kernel": kernel,
           "kernel_ms": round(proj_ms, 4)}
     proj = (traffic or {}).get("projection")
     if proj:
@@ -744,6 +754,8 @@ def roofline_object(wl, kind, L, proj_ms, counts, traffic, traffic_err, ceilings
     units = {}
     if ceilings:
         adds, evals = (counts or {}).get("projection_lds_adds"), (counts or {}).get("projection_weight_evals")
+        if kernel == "project_range_kernel":
+            adds = evals = None
         if adds:
             # the launch's bins: float (ds_add_f32) or 64-bit fixed point (ds_add_u64)
             name, key = (("lds_int64_atomics", "lds_int64_atomics_per_s") if fixed_bins else
@@ -835,9 +847,9 @@ def main():
     ceil = CE.measure()
     ceil["compute_units"] = CE.cu_count()
     log(f"ceilings: {ceil}")
-    lds_bins = counts.pop("bins", None)
+    lds_bins, kernel = counts.pop("bins", None), counts.pop("kernel")
     roofline = (roofline_object(wl, kind, L, proj_ms, counts, traffic, traffic_err, ceil,
-                                fixed_bins=lds_bins == "fixed") if proj_ms else None)
+                                fixed_bins=lds_bins == "fixed", kernel=kernel) if proj_ms else None)
     line = {
         "metric": "IQ lines/s & scatterer-evals/s at 1M scatterers; serving p50/p99 frame latency",
         "value": round(L / (ms * 1e-3), 1),

@@ -65,7 +65,8 @@ BCSIM_API bcsim_status bcsim_destroy(bcsim_sim* sim);
  * ("tiled", the culled tile kernel, default; "direct", every line-scatterer
  * pair, for checking); autotune (on/off, default off: time candidate launch
  * shapes once per shape class, process-wide, and use the fastest); fft_radix
- * (4 or 8; 0 = tuned or default); tile_lines, tile_block, tile_slices,
+ * (4 or 8; 0 = tuned or default; 8 includes the passes of 16 points that frames
+ * of 2^11 to 2^14 points use); tile_lines, tile_block, tile_slices,
  * tile_windows (tile-kernel launch shape; 0 = tuned or heuristic); tile_order
  * (on/off, default on: large projection launches run their blocks heaviest
  * first, by the previous frame's counts); chunk_order (on/off, default on: the

@@ -2276,7 +2276,7 @@ struct bcsim_sim {
         float2* turned = by_sample ? d_iq_turned.as<float2>() : nullptr;
         enqueue_frame(d_iq.as<float2>(), nullptr, turned);
         const void* src = by_sample ? d_iq_turned.p : d_iq.p;
-        if (bytes >= kStagedCopyMin && host_pageable(out)) {
+        if (bytes >= kStagedCopyMin && host_pageable(out) && stage_ready(bytes)) {
             copy_staged(out, src, bytes);
         } else {
             {
@@ -2303,21 +2303,29 @@ struct bcsim_sim {
     size_t stage_bytes[2] = {0, 0};
     hipEvent_t stage_ev[kStagePieces] = {};
 
-    void ensure_stage(int i, size_t bytes) {
-        if (bytes <= stage_bytes[i]) return;
-        if (stage[i]) (void)hipHostFree(stage[i]);
-        stage[i] = nullptr;
-        stage_bytes[i] = 0;
-        hip_check(hipHostMalloc(&stage[i], bytes, 0), "hipHostMalloc");
-        stage_bytes[i] = bytes;
+    // Pinned pieces for a copy of `bytes`; false without memory for them (the runtime copies).
+    bool stage_ready(size_t bytes) {
+        const bool small = bytes <= kStagePiece;
+        const auto ensure = [&](int i, size_t n) {
+            if (n <= stage_bytes[i]) return true;
+            if (stage[i]) (void)hipHostFree(stage[i]);
+            stage[i] = nullptr;
+            stage_bytes[i] = 0;
+            if (hipHostMalloc(&stage[i], n, 0) != hipSuccess) {
+                (void)hipGetLastError();
+                stage[i] = nullptr;
+                return false;
+            }
+            stage_bytes[i] = n;
+            return true;
+        };
+        return ensure(0, small ? bytes : kStagePiece) && (small || ensure(1, kStagePiece));
     }
 
     void copy_staged(void* dst, const void* src, size_t bytes) {
         for (auto& e : stage_ev)
             if (!e) hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
         const bool small = bytes <= kStagePiece;
-        ensure_stage(0, small ? bytes : kStagePiece);
-        if (!small) ensure_stage(1, kStagePiece);
         // pieces of about 768 KiB in one buffer, or whole buffers by turns
         const size_t count = std::min<size_t>(kStagePieces, std::max<size_t>(1, bytes / ((size_t)768 << 10)));
         const size_t piece = small ? ((bytes + count - 1) / count + 255) & ~(size_t)255 : kStagePiece;
