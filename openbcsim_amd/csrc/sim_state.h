@@ -82,10 +82,14 @@ inline std::shared_ptr<DevBuf> conv_roots(int device, const ConvShape& c) {
     auto& slot = tables[{device, c.log2n, c.full ? 1 : 0, c.fold}];
     if (auto t = slot.lock()) return t;
     const int n = 1 << c.log2n;
-    std::vector<float2> unit(n), all;
-    for (int i = 0; i < n; i++) {
-        const double a = -2.0 * M_PI * (double)i / (double)n;
-        unit[i] = make_float2((float)std::cos(a), (float)std::sin(a));
+    std::vector<float2> unit(n), all;  // exp(-2 pi i k / n), from its first octant
+    for (int i = 0; i <= n / 8; i++) {
+        const double a = 2.0 * M_PI * (double)i / (double)n;
+        const float c = (float)std::cos(a), s = (float)std::sin(a);
+        const int h = n / 2, q = n / 4;
+        unit[i] = make_float2(c, -s), unit[q - i] = make_float2(s, -c), unit[q + i] = make_float2(-s, -c);
+        unit[h - i] = make_float2(-c, -s), unit[h + i] = make_float2(-c, s), unit[h + q - i] = make_float2(-s, c);
+        unit[h + q + i] = make_float2(s, c), unit[(n - i) & (n - 1)] = make_float2(c, s);
     }
     const ConvRoots shape = conv_roots_shape(c.log2n, c.full, c.fold);
     for (int block : {shape.forward, shape.inverse})
@@ -190,7 +194,7 @@ struct ChunkOrders {
 };
 
 // A dataset's points sorted by radial bin from a scan origin (project_range.hip), one
-// copy (32 bytes a point) per origin, bin rule and demodulation phase.  Like the chunk
+// copy (36 bytes a point) per origin, bin rule and demodulation phase.  Like the chunk
 // orders they live as long as the dataset; further origins run the tile kernel.
 struct RangeOrders {
     struct Key {
@@ -202,7 +206,9 @@ struct RangeOrders {
     };
     struct Order {
         Key key;
-        DevBuf recs, start;
+        DevBuf mem;  // the records, the first record of each bin, and the sort's counts and ranks
+        RangeRec* recs;
+        int* start;
     };
     static constexpr size_t kMaxOrders = 4;
     std::mutex mu;
@@ -220,11 +226,11 @@ struct RangeOrders {
         auto o = std::make_unique<Order>();
         o->key = key;
         try {
-            DevBuf scratch;
-            o->recs.ensure(n * sizeof(RangeRec));
-            o->start.ensure((kRangeBins + 1) * sizeof(int));
-            scratch.ensure((kRangeBins + n) * sizeof(int));
-            (*sort)(o->recs.as<RangeRec>(), o->start.as<int>(), scratch.as<int>());
+            // one allocation (a new dataset's first frame waits for each)
+            o->mem.ensure(n * sizeof(RangeRec) + (2 * kRangeBins + 4 + n) * sizeof(int));
+            o->recs = o->mem.as<RangeRec>();
+            o->start = reinterpret_cast<int*>(o->recs + n);
+            (*sort)(o->recs, o->start, o->start + kRangeBins + 4);
         } catch (const BcsimError& e) {
             if (e.code != BCSIM_ERR_OUT_OF_MEMORY) throw;
             (void)hipGetLastError();
@@ -2036,8 +2042,8 @@ struct bcsim_sim {
         const RangeOrders::Order* o = t.fixed->by_range.get(key, t.n, create ? &sort : nullptr);
         if (!o) return R;
         R.patches = d_patches.as<RangePatch>();
-        R.start = o->start.as<int>();
-        R.recs = o->recs.as<RangeRec>();
+        R.start = o->start;
+        R.recs = o->recs;
         return R;
     }
 
