@@ -540,7 +540,7 @@ struct bcsim_sim {
     int profile = -1;
     float sigma_l = 0.f, sigma_e = 0.f;
     std::shared_ptr<DevBuf> lut;  // float4 quad pairs [n_rad][n_ele][n_lat][2]; replaced, never rewritten
-    std::shared_ptr<DevBuf> lut_rel;  // the samples as [n_rad][n_ele][n_lat] (project_range.hip); null if one is not finite
+    std::shared_ptr<DevBuf> lut_rel;  // the samples as [n_rad][n_ele][n_lat] (project_range.hip); null if one is not finite or they do not fit
     std::shared_ptr<const std::vector<float>> lut_samples;  // the table as given, for the cutoff's boxes
     float lut_peak = 0.0f;                                   // largest |sample|
     std::shared_ptr<DevBuf> lut_boxes;                       // ProfileParams::slice_box for lut_boxes_cut
@@ -1050,14 +1050,24 @@ struct bcsim_sim {
                     finite = finite && std::isfinite(v);
                     rel[((size_t)r * ne + e) * nl + l] = v;
                 }
-        lut_rel.reset();
+        std::shared_ptr<DevBuf> samples_only;
         if (finite) {
-            lut_rel = std::make_shared<DevBuf>();
-            lut_rel->ensure(cells * sizeof(float));
-            hip_check(hipMemcpy(lut_rel->p, rel.data(), cells * sizeof(float), hipMemcpyHostToDevice), "hipMemcpy");
+            samples_only = std::make_shared<DevBuf>();
+            try {
+                samples_only->ensure(cells * sizeof(float));
+            } catch (const BcsimError& e) {
+                if (e.code != BCSIM_ERR_OUT_OF_MEMORY) throw;
+                (void)hipGetLastError();
+                samples_only.reset();  // the tile kernel, which reads the quads, projects every frame
+            }
+            if (samples_only)
+                hip_check(hipMemcpy(samples_only->p, rel.data(), cells * sizeof(float), hipMemcpyHostToDevice), "hipMemcpy");
         }
+        auto given = std::make_shared<const std::vector<float>>(samples, samples + cells);
+        // nothing below fails: until here the profile is the one there was
         lut = std::move(table);
-        lut_samples = std::make_shared<const std::vector<float>>(samples, samples + cells);
+        lut_rel = std::move(samples_only);
+        lut_samples = std::move(given);
         lut_peak = 0.0f;
         for (size_t i = 0; i < cells; i++) lut_peak = std::max(lut_peak, std::fabs(samples[i]));
         lut_boxes.reset();

@@ -1,0 +1,192 @@
+// Test infrastructure (CPU only): the host code around the projection in range order
+// under the mock runtime of mock_hip.cpp, with device allocations and copies that fail
+// on request.  The mock is compiled with its hipMalloc, hipMemcpy and
+// launch_project_tile renamed (mock_*); the ones here inject the failures and check
+// what a range-order launch reads before they pass the call on.
+//   usage: memory_driver <scenario>
+#include <hip/hip_runtime.h>
+
+#include <cmath>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <functional>
+#include <random>
+#include <string>
+#include <vector>
+#include <unistd.h>
+
+#include "../../include/bcsim_c.h"
+#include "../../openbcsim_amd/csrc/sim_device.h"
+
+using namespace bcsim_hip;
+
+extern "C" hipError_t mock_hipMalloc(void** ptr, size_t size);
+extern "C" hipError_t mock_hipMemcpy(void* dst, const void* src, size_t n, hipMemcpyKind kind);
+namespace bcsim_hip {
+hipError_t mock_launch_project_tile(const ProjCommon& c, const CullParams& cp, const FixedSet* fixed,
+                                    const SplineSet* spline, const ChunkBox* boxes, int nchunks, void* bins, bool arc,
+                                    bool phase, bool lut, bool shared_origin, const TileLaunch& cfg, hipStream_t s);
+}
+
+#define REQUIRE(x)                                                                                 \
+    do {                                                                                           \
+        if (!(x)) {                                                                                \
+            fprintf(stderr, "FAIL %s:%d %s (%s)\n", __FILE__, __LINE__, #x, bcsim_last_error());    \
+            _exit(1);                                                                              \
+        }                                                                                          \
+    } while (0)
+#define CHK(x) REQUIRE((x) == BCSIM_OK)
+
+// ---- failures: the allocation or copy for which the predicate holds fails
+static std::function<bool(size_t)> fail_malloc, fail_copy;
+static int mallocs = 0;  // allocations since the last reset
+
+extern "C" hipError_t hipMalloc(void** ptr, size_t size) {
+    mallocs++;
+    if (fail_malloc && fail_malloc(size)) {
+        *ptr = nullptr;
+        return hipErrorOutOfMemory;
+    }
+    return mock_hipMalloc(ptr, size);
+}
+extern "C" hipError_t hipMemcpy(void* dst, const void* src, size_t n, hipMemcpyKind kind) {
+    if (fail_copy && fail_copy(n)) return hipErrorUnknown;
+    return mock_hipMemcpy(dst, src, n, kind);
+}
+
+static bool live(const void* p) {
+    hipPointerAttribute_t a;
+    return p && hipPointerGetAttributes(&a, p) == hipSuccess;
+}
+
+static int range_launches = 0;  // projections in range order
+static float table_value = 0.0f;  // what every sample of the profile's table is
+
+namespace bcsim_hip {
+hipError_t launch_project_tile(const ProjCommon& c, const CullParams& cp, const FixedSet* fixed, const SplineSet* spline,
+                               const ChunkBox* boxes, int nchunks, void* bins, bool arc, bool phase, bool lut,
+                               bool shared_origin, const TileLaunch& cfg, hipStream_t s) {
+    const RangeLaunch& R = cfg.range;
+    if (R.recs) {
+        REQUIRE(live(R.recs) && live(R.start) && !spline);
+        REQUIRE(live(fixed->pts));
+        if (R.sort) REQUIRE(live(R.count) && live(R.rank));
+        if (R.sort != 2) {
+            range_launches++;
+            REQUIRE(live(R.patches) && R.n_patches > 0);
+            if (lut) {
+                REQUIRE(live(R.table));
+                const int n = c.prof.nr * c.prof.nl * c.prof.ne;
+                REQUIRE(R.table[0] == table_value && R.table[n - 1] == table_value);
+            }
+        }
+    }
+    return mock_launch_project_tile(c, cp, fixed, spline, boxes, nchunks, bins, arc, phase, lut, shared_origin, cfg, s);
+}
+}  // namespace bcsim_hip
+
+// ---- simulators
+struct Scan {
+    std::vector<float> o, d, l, t;
+    float len = 0.05f;
+};
+static Scan sector(int n, float x0 = 0.0f) {
+    Scan s;
+    for (int k = 0; k < n; k++) {
+        const double a = -0.6 + 1.2 * k / (n - 1);
+        s.o.insert(s.o.end(), {x0, 0, 0});
+        s.d.insert(s.d.end(), {(float)sin(a), 0, (float)cos(a)});
+        s.l.insert(s.l.end(), {(float)cos(a), 0, (float)-sin(a)});
+        s.t.push_back(0);
+    }
+    return s;
+}
+static void set_scan(bcsim_sim* s, const Scan& q, bool at_once = false) {
+    CHK(bcsim_set_scan_sequence(s, (int)q.t.size(), q.o.data(), q.d.data(), q.l.data(), q.t.data(), q.len, at_once));
+}
+static std::vector<float> box_points(size_t n) {
+    std::mt19937 rng(3);
+    std::uniform_real_distribution<float> u(0, 1);
+    std::vector<float> p;
+    for (size_t i = 0; i < n; i++)
+        p.insert(p.end(), {0.05f * u(rng) - 0.025f, 0.004f * u(rng) - 0.002f, 0.005f + 0.04f * u(rng), u(rng) - 0.5f});
+    return p;
+}
+static bcsim_sim* simulator(int lines, size_t points) {
+    bcsim_sim* s;
+    CHK(bcsim_create("gpu", &s));
+    std::vector<float> pulse(55, 0.5f);
+    CHK(bcsim_set_excitation(s, pulse.data(), 55, 27, 50e6f, 2.5e6f));
+    set_scan(s, sector(lines));
+    if (points) {
+        const std::vector<float> p = box_points(points);
+        CHK(bcsim_add_fixed_scatterers(s, p.data(), points));
+    }
+    CHK(bcsim_set_analytical_profile(s, 1e-3f, 1e-3f));
+    return s;
+}
+static bcsim_status set_table(bcsim_sim* s, int nr) {
+    std::vector<float> t((size_t)nr * 24 * 24, 1.0f / nr);
+    const bcsim_status st =
+        bcsim_set_lut_profile(s, 0, 0.05f, -0.01f, 0.01f, -0.01f, 0.01f, t.data(), nr, 24, 24);
+    if (st == BCSIM_OK) table_value = 1.0f / nr;
+    return st;
+}
+static std::string plan(bcsim_sim* s) {
+    char b[2048];
+    CHK(bcsim_get_parameter(s, "launch_plan", b, sizeof b));
+    return b;
+}
+// One frame; whether it ran in range order.
+static bool ranged(bcsim_sim* s) {
+    int L, S;
+    CHK(bcsim_get_output_shape(s, &L, &S));
+    std::vector<float> out((size_t)L * S * 2);
+    const int before = range_launches;
+    CHK(bcsim_simulate_lines(s, out.data(), (size_t)L * S, &L, &S));
+    REQUIRE((plan(s).find("range order") != std::string::npos) == (range_launches > before));
+    return range_launches > before;
+}
+
+// A table whose samples or quads do not fit, or whose copies fail, leaves the profile
+// that was there; without room for the samples alone the frames run the tile kernel.
+static void table_failures() {
+    bcsim_sim* s = simulator(128, 20000);
+    CHK(set_table(s, 16));
+    REQUIRE(ranged(s));
+    int k = 0;
+    fail_malloc = [&](size_t) { return ++k == 1; };  // the quads
+    REQUIRE(set_table(s, 20) == BCSIM_ERR_OUT_OF_MEMORY);
+    fail_malloc = nullptr;
+    REQUIRE(ranged(s));  // with the old table
+    for (int copy : {1, 2}) {
+        k = 0;
+        fail_copy = [&](size_t) { return ++k == copy; };
+        REQUIRE(set_table(s, 20) == BCSIM_ERR_DEVICE);
+        fail_copy = nullptr;
+        REQUIRE(ranged(s));
+    }
+    k = 0;
+    fail_malloc = [&](size_t) { return ++k == 2; };  // the samples
+    CHK(set_table(s, 20));
+    fail_malloc = nullptr;
+    REQUIRE(!ranged(s));
+    CHK(set_table(s, 20));
+    REQUIRE(ranged(s));
+    CHK(bcsim_destroy(s));
+}
+
+int main(int argc, char** argv) {
+    const std::string what = argc > 1 ? argv[1] : "";
+    const std::vector<std::pair<std::string, void (*)()>> all = {{"table_failures", table_failures}};
+    for (auto& e : all)
+        if (e.first == what) {
+            e.second();
+            fprintf(stderr, "DONE %s\n", what.c_str());
+            fflush(stderr);
+            _exit(0);
+        }
+    fprintf(stderr, "unknown scenario\n");
+    return 2;
+}
