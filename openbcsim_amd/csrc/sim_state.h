@@ -43,6 +43,19 @@ inline void hip_check(hipError_t e, const char* what) {
     }
 }
 
+// Runs f, which allocates what a frame can do without; false without memory for it.
+template <typename F>
+bool where_it_fits(F&& f) {
+    try {
+        f();
+        return true;
+    } catch (const BcsimError& e) {
+        if (e.code != BCSIM_ERR_OUT_OF_MEMORY) throw;
+        (void)hipGetLastError();
+        return false;
+    }
+}
+
 // Device buffer owned by a simulator.
 struct DevBuf {
     void* p = nullptr;
@@ -225,17 +238,14 @@ struct RangeOrders {
         if (!sort || orders.size() >= kMaxOrders) return nullptr;
         auto o = std::make_unique<Order>();
         o->key = key;
-        try {
+        const bool fits = where_it_fits([&] {
             // one allocation (a new dataset's first frame waits for each)
             o->mem.ensure(n * sizeof(RangeRec) + (2 * kRangeBins + 4 + n) * sizeof(int));
             o->recs = o->mem.as<RangeRec>();
             o->start = reinterpret_cast<int*>(o->recs + n);
             (*sort)(o->recs, o->start, o->start + kRangeBins + 4);
-        } catch (const BcsimError& e) {
-            if (e.code != BCSIM_ERR_OUT_OF_MEMORY) throw;
-            (void)hipGetLastError();
-            return nullptr;
-        }
+        });
+        if (!fits) return nullptr;
         orders.push_back(std::move(o));
         return orders.back().get();
     }
@@ -1053,13 +1063,8 @@ struct bcsim_sim {
         std::shared_ptr<DevBuf> samples_only;
         if (finite) {
             samples_only = std::make_shared<DevBuf>();
-            try {
-                samples_only->ensure(cells * sizeof(float));
-            } catch (const BcsimError& e) {
-                if (e.code != BCSIM_ERR_OUT_OF_MEMORY) throw;
-                (void)hipGetLastError();
-                samples_only.reset();  // the tile kernel, which reads the quads, projects every frame
-            }
+            // else the tile kernel, which reads the quads, projects every frame
+            if (!where_it_fits([&] { samples_only->ensure(cells * sizeof(float)); })) samples_only.reset();
             if (samples_only)
                 hip_check(hipMemcpy(samples_only->p, rel.data(), cells * sizeof(float), hipMemcpyHostToDevice), "hipMemcpy");
         }
@@ -1237,7 +1242,7 @@ struct bcsim_sim {
             quiesce();  // frames in flight may read the old table
             roots.reset();
             if (log2_len >= kConvFixedMin && log2_len <= kConvFixedMax && shape.fold < kConvFixedFolds)
-                roots = conv_roots(device, shape);
+                where_it_fits([&] { roots = conv_roots(device, shape); });
             roots_shape = shape;
         }
         if (dirty_basis) {
@@ -1968,8 +1973,7 @@ struct bcsim_sim {
             R.cell_floats = 2 * (lut_nl | 1) * lut_ne;
         }
         if (dirty_patches) {
-            if (!create) return R;
-            build_patches();
+            if (!create || !where_it_fits([&] { build_patches(); })) return R;
         }
         R.n_patches = n_patches;
         // A patch's waves visit every point that reaches any of its lines.  Where few of its 64
@@ -2015,7 +2019,7 @@ struct bcsim_sim {
             R.window_bins = R.run_bins * ((waves + R.group - 1) / R.group);
         }
         if (rendered) {  // other points every frame: sorted by each, into this simulator's buffers
-            try {
+            const bool fits = where_it_fits([&] {
                 t.scan->recs.ensure(t.n * sizeof(RangeRec));
                 DevBuf& w = t.scan->sort;
                 const size_t ints = 2 * kRangeBins + 4 + t.n;  // count, start, rank
@@ -2026,11 +2030,8 @@ struct bcsim_sim {
                 R.count = w.as<int>();
                 R.start = R.count + kRangeBins;
                 R.rank = R.start + kRangeBins + 4;
-            } catch (const BcsimError& e) {
-                if (e.code != BCSIM_ERR_OUT_OF_MEMORY) throw;
-                (void)hipGetLastError();
-                return RangeLaunch{};
-            }
+            });
+            if (!fits) return RangeLaunch{};
             R.sort = 1;
             R.patches = d_patches.as<RangePatch>();
             R.recs = t.scan->recs.as<RangeRec>();

@@ -177,9 +177,31 @@ static void table_failures() {
     CHK(bcsim_destroy(s));
 }
 
+// Without room for the constant-length transforms' twiddles, the patches, or a range order
+// the frames run the kernels that do without them.
+static void optional_buffers() {
+    for (size_t bytes : {conv_roots_size(12, false, 0) * sizeof(float2), 2 * sizeof(RangePatch)}) {
+        bcsim_sim* s = simulator(128, 20000);
+        int failed = 0;
+        fail_malloc = [&](size_t n) { return n == bytes && ++failed; };
+        const bool in_order = ranged(s);
+        fail_malloc = nullptr;
+        REQUIRE(failed > 0 && in_order == (bytes != 2 * sizeof(RangePatch)));
+        REQUIRE(ranged(s));  // there is room again
+        CHK(bcsim_destroy(s));
+    }
+    bcsim_sim* s = simulator(128, 20000);
+    fail_malloc = [&](size_t n) { return n > 20000 * sizeof(RangeRec) && n < 21000 * sizeof(RangeRec) + 200000; };
+    REQUIRE(!ranged(s));
+    fail_malloc = nullptr;
+    REQUIRE(ranged(s));
+    CHK(bcsim_destroy(s));
+}
+
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
-    const std::vector<std::pair<std::string, void (*)()>> all = {{"table_failures", table_failures}};
+    const std::vector<std::pair<std::string, void (*)()>> all = {
+        {"table_failures", table_failures}, {"optional_buffers", optional_buffers}};
     for (auto& e : all)
         if (e.first == what) {
             e.second();
