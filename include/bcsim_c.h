@@ -85,7 +85,9 @@ BCSIM_API bcsim_status bcsim_destroy(bcsim_sim* sim);
  * (integer LDS atomics; each contribution rounded to a power-of-two grid chosen
  * per launch from the dataset's amplitudes, about 1e-12 of a typical one, then
  * summed exactly) or float; auto tunes the choice where tuning is on and is
- * otherwise fixed for the Gaussian profile and float for a LUT.  With auto and no
+ * otherwise fixed for the Gaussian profile and, for a LUT, float, or double where a
+ * workgroup keeps one line's bins (straight scans, splines with a time per line, of
+ * fewer than about 2048 lines).  With auto and no
  * tile_* shape set, arc projection of points onto lines of one origin runs in range
  * order instead of the tile kernel (points sorted by bin; register sums, double for
  * the Gaussian and float for a LUT), which launch_plan reports.  Datasets whose

@@ -18,13 +18,19 @@ namespace bcsim_hip {
 // Tile-kernel launch shape; 0 in a field means "the heuristic's choice".
 struct TileTune {
     int windows = 0, lines = 0, block = 0, slices = 0;
-    int bins = 0;  // LDS bin accumulation: 1 fixed point, 2 float, 0 automatic
+    int bins = 0;  // LDS bin accumulation (BinMode)
 };
+
+// kBinsWide: double, where a tile is one line of a lookup table's frame (else as float).
+enum BinMode { kBinsAuto = 0, kBinsFixed = 1, kBinsFloat = 2, kBinsWide = 3 };
+inline const char* bin_name(int m) {
+    return m == kBinsFixed ? "fixed" : m == kBinsFloat ? "float" : m == kBinsWide ? "double" : "auto";
+}
 
 inline std::string describe(const TileTune& t) {
     char buf[112];
     std::snprintf(buf, sizeof buf, "lines=%d block=%d slices=%d windows=%d bins=%s", t.lines, t.block, t.slices,
-                  t.windows, t.bins == 1 ? "fixed" : t.bins == 2 ? "float" : "auto");
+                  t.windows, bin_name(t.bins));
     return buf;
 }
 

@@ -247,7 +247,7 @@ struct bcsim_batch {
                 if (tile_lines > 0) {
                     TileTune tt = s->tune;
                     tt.lines = tile_lines;
-                    J.g = s->tile_launch(t.nchunks, tt, is_spline, s->target_fixed(t));
+                    J.g = s->tile_launch(t.nchunks, tt, is_spline, s->target_bins(t, tt));
                 }
                 J.g.block = 1024;
                 J.g.chunks = t.chunk_order;
@@ -260,7 +260,8 @@ struct bcsim_batch {
                     J.g.range = s->range_launch(t, J.g, J.bins, true);
                 J.flags = (s->arc ? kJobArc : 0) | (cplx ? kJobPhase : 0) | (lut ? kJobLut : 0) |
                           (is_spline ? kJobSpline : 0) | (shared && !is_spline ? kJobShared : 0) |
-                          (J.g.fixed ? kJobFixed : 0) | (J.g.range.recs ? kJobRange : 0);
+                          (J.g.fixed ? kJobFixed : 0) | (J.g.wide ? kJobWide : 0) |
+                          (J.g.range.recs ? kJobRange : 0);
                 const int tiles = (t.c.num_lines + J.g.tile_lines - 1) / J.g.tile_lines;
                 J.blocks_per_slice = tiles * J.g.windows;
                 J.g.work = nullptr;
@@ -328,7 +329,7 @@ struct bcsim_batch {
                 groups.push_back(ProjGroup{vkey[j], (int)pitems.size(), 0, 0});
             ProjGroup& G = groups.back();
             const ProjJob& J = pjobs[j];
-            G.lds = std::max(G.lds, tile_lds_bytes(J.g.window_bins, tile_bin_bytes((J.flags & kJobPhase) != 0, J.g.fixed),
+            G.lds = std::max(G.lds, tile_lds_bytes(J.g.window_bins, tile_bin_bytes((J.flags & kJobPhase) != 0, J.g.fixed || J.g.wide),
                                                    J.g.tile_lines, J.g.list_cap, J.g.list_packed));
             first_item[j] = pitems.size();
             const int n = J.blocks_per_slice * J.g.slices;

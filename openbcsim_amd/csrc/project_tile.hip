@@ -25,7 +25,8 @@
 // The block leaves LDS once: plain stores when the workgroup saw every chunk,
 // otherwise atomic adds of the non-zero bins.
 //
-// LDS bins are float (ds_add_f32) or 64-bit fixed point (ds_add_u64, FIXED).
+// LDS bins are float (ds_add_f32), 64-bit fixed point (ds_add_u64, FIXED) or, for one-line
+// tiles of a lookup table, double (ds_add_f64).
 // On gfx950 an LDS float atomic add retires about one lane per three cycles
 // while an integer one retires a wave's 64 lanes about ten times faster
 // (measured: ~2e11 against ~2e12 lane additions per second on the chip), so the
@@ -122,11 +123,16 @@ __device__ __forceinline__ void lds_add(long long* b, float v) {
     atomicAdd(reinterpret_cast<unsigned long long*>(b), (unsigned long long)q);
 }
 
+// Double bins: as fast as the integers and without a grid, so that the tails of a table's beam
+// keep float's relative precision and a sample that is not finite reaches the bin.
+__device__ __forceinline__ void lds_add(double* b, float v) { unsafeAtomicAdd(b, (double)v); }
+
 // A bin sum as float.
 __device__ __forceinline__ float bin_value(float v, const ProjCommon&) { return v; }
 __device__ __forceinline__ float bin_value(long long v, const ProjCommon& c) {
     return (float)((double)v * (double)c.inv_amp_scale);
 }
+__device__ __forceinline__ float bin_value(double v, const ProjCommon&) { return (float)v; }
 
 // Weight times amplitude added at window-relative bin lb (CpuAlgorithm.cpp:77-95).
 // With fixed-point bins the amplitude was scaled by amp_scale, a power of two, so
@@ -637,13 +643,13 @@ __device__ __forceinline__ void project_list(const ProjCommon& c, const FixedSet
 // tile_block for a tile of one line (any origin; splines at the line's time): the
 // line's geometry and spline basis stay in registers, the list needs no masks, and a
 // chunk's scatterers are loaded while the previous chunk's are projected.
-template <bool ARC, bool PHASE, bool LUT, bool SPLINE, bool FIXED>
+// Acc: the type of its bins (long long: fixed point).
+template <bool ARC, bool PHASE, bool LUT, bool SPLINE, class Acc>
 __device__ __forceinline__ void line_block(const ProjCommon& c, const CullParams& cp, const FixedSet& fs,
                                            const SplineSet& ss, const ChunkBox* __restrict__ boxes, int nchunks,
                                            float* __restrict__ out, const TileLaunch& g, int wg, int slice,
                                            float* lds, int& list_n) {
     constexpr int E = PHASE ? 2 : 1;
-    using Acc = typename std::conditional<FIXED, long long, float>::type;
     const int window = wg % g.windows;
     const int line = wg / g.windows;
     const int b0 = window * g.window_bins;
@@ -700,7 +706,7 @@ __device__ __forceinline__ void line_block(const ProjCommon& c, const CullParams
         const int n = __builtin_amdgcn_readfirstlane(list_n);
         __syncthreads();
         if (next < cend && n <= g.list_cap - step) continue;
-        const float scale = FIXED ? c.amp_scale : 1.0f;
+        const float scale = std::is_same<Acc, long long>::value ? c.amp_scale : 1.0f;
         if (!SPLINE)
             project_list<ARC, PHASE, LUT, false, 1>(c, fs, ss, L, 0, basis, list, n, bins, b0, nb, scale, tally);
         else if (count == 4)
@@ -741,14 +747,14 @@ __global__ __launch_bounds__(1024) void project_tile_kernel(ProjCommon c, CullPa
                                                        list_n);
 }
 
-template <bool ARC, bool PHASE, bool LUT, bool SPLINE, bool FIXED>
+template <bool ARC, bool PHASE, bool LUT, bool SPLINE, class Acc>
 __global__ __launch_bounds__(1024, 8) void project_line_kernel(ProjCommon c, CullParams cp, FixedSet fs, SplineSet ss,
                                                             const ChunkBox* __restrict__ boxes, int nchunks,
                                                             float* __restrict__ out, TileLaunch g) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     __shared__ int list_n;
     const int wg = __builtin_amdgcn_readfirstlane(g.order ? g.order[blockIdx.x] : (int)blockIdx.x);
-    line_block<ARC, PHASE, LUT, SPLINE, FIXED>(c, cp, fs, ss, boxes, nchunks, out, g, wg, blockIdx.y, lds, list_n);
+    line_block<ARC, PHASE, LUT, SPLINE, Acc>(c, cp, fs, ss, boxes, nchunks, out, g, wg, blockIdx.y, lds, list_n);
 }
 
 // Order of the next tile launch's blocks: by the (chunk, line) pairs each listed
@@ -836,8 +842,9 @@ hipError_t launch_order_segments(const OrderSeg* segs, int n_segs, hipStream_t s
 // Persistent projection over many jobs (simulators x datasets) of one kernel
 // variant: every workgroup takes (job, block) items from a global counter until
 // the list is exhausted, and runs the block.  KIND: 0 fixed points, 1 fixed
-// points with a shared origin (arc projection), 2 splines; FIXED: fixed-point bins.
-template <bool ARC, bool PHASE, bool LUT, int KIND, bool FIXED>
+// points with a shared origin (arc projection), 2 splines; Acc: the type of the bins
+// (long long: fixed point; double: one-line tiles only).
+template <bool ARC, bool PHASE, bool LUT, int KIND, class Acc>
 __global__ __launch_bounds__(1024) void project_batch_kernel(const ProjJob* __restrict__ jobs,
                                                              const int2* __restrict__ items, int n_items,
                                                              int* __restrict__ counter) {
@@ -855,20 +862,21 @@ __global__ __launch_bounds__(1024) void project_batch_kernel(const ProjJob* __re
         const int blk = __builtin_amdgcn_readfirstlane(w.y);
         const int per_slice = J.blocks_per_slice;
         const int wg = blk % per_slice, slice = blk / per_slice;
-        if (KIND != 1 && J.g.tile_lines == 1)
-            line_block<ARC, PHASE, LUT, KIND == 2, FIXED>(J.c, J.cp, J.fs, J.ss, J.boxes, J.nchunks, J.bins, J.g, wg,
-                                                          slice, lds, list_n);
-        else
+        constexpr bool FIXED = std::is_same<Acc, long long>::value, LINE = std::is_same<Acc, double>::value;
+        if (LINE || (KIND != 1 && J.g.tile_lines == 1))
+            line_block<ARC, PHASE, LUT, KIND == 2, Acc>(J.c, J.cp, J.fs, J.ss, J.boxes, J.nchunks, J.bins, J.g, wg,
+                                                        slice, lds, list_n);
+        else if constexpr (!LINE)
             tile_block<ARC, PHASE, LUT, KIND == 2, KIND == 1, FIXED>(J.c, J.cp, J.fs, J.ss, J.boxes, J.nchunks, J.bins,
                                                                      J.g, wg, slice, lds, list_n);
         __syncthreads();  // the next item reuses the LDS
     }
 }
 
-template <bool ARC, bool PHASE, bool LUT, int KIND, bool FIXED>
+template <bool ARC, bool PHASE, bool LUT, int KIND, class Acc>
 static hipError_t launch_batch_t(const ProjJob* jobs, const int2* items, int n_items, int* counter, size_t lds,
                                  int workgroups, hipStream_t stream) {
-    auto k = project_batch_kernel<ARC, PHASE, LUT, KIND, FIXED>;
+    auto k = project_batch_kernel<ARC, PHASE, LUT, KIND, Acc>;
     hipError_t e = allow_lds((const void*)k, lds);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k, dim3(workgroups), dim3(1024), lds, stream, jobs, items, n_items, counter);
@@ -876,15 +884,22 @@ static hipError_t launch_batch_t(const ProjJob* jobs, const int2* items, int n_i
 }
 
 template <bool ARC, bool PHASE, bool LUT>
-static hipError_t launch_batch_kind(int kind, bool fixed, const ProjJob* jobs, const int2* items, int n_items,
+static hipError_t launch_batch_kind(int kind, bool fixed, bool wide, const ProjJob* jobs, const int2* items, int n_items,
                                     int* counter, size_t lds, int workgroups, hipStream_t stream) {
-#define BCSIM_BATCH_K(K)                                                                                          \
-    return fixed ? launch_batch_t<ARC, PHASE, LUT, K, true>(jobs, items, n_items, counter, lds, workgroups, stream) \
-                 : launch_batch_t<ARC, PHASE, LUT, K, false>(jobs, items, n_items, counter, lds, workgroups, stream)
-    if (kind == 2) BCSIM_BATCH_K(2);
-    if (kind == 1) BCSIM_BATCH_K(1);
+#define BCSIM_BATCH_T(K, T) launch_batch_t<ARC, PHASE, LUT, K, T>(jobs, items, n_items, counter, lds, workgroups, stream)
+#define BCSIM_BATCH_K(K)                                           \
+    if constexpr (LUT && K != 1)                                   \
+        if (wide) return BCSIM_BATCH_T(K, double);                 \
+    return fixed ? BCSIM_BATCH_T(K, long long) : BCSIM_BATCH_T(K, float)
+    if (kind == 2) {
+        BCSIM_BATCH_K(2);
+    }
+    if (kind == 1) {
+        BCSIM_BATCH_K(1);
+    }
     BCSIM_BATCH_K(0);
 #undef BCSIM_BATCH_K
+#undef BCSIM_BATCH_T
 }
 
 hipError_t launch_project_batch(int variant, const ProjJob* jobs, const int2* items, int n_items, int* counter,
@@ -893,9 +908,10 @@ hipError_t launch_project_batch(int variant, const ProjJob* jobs, const int2* it
     if (variant & kJobRange) return launch_range_batch(variant & kJobPhase, jobs, items, n_items, stream);
     const bool arc = variant & kJobArc, phase = variant & kJobPhase, lut = variant & kJobLut;
     const int kind = (variant & kJobSpline) ? 2 : (arc && (variant & kJobShared)) ? 1 : 0;
-    const bool fixed = variant & kJobFixed;
+    const bool fixed = variant & kJobFixed, wide = variant & kJobWide;
+    if (wide && (!lut || kind == 1)) return hipErrorInvalidValue;
 #define BCSIM_BATCH(A, P, U) \
-    return launch_batch_kind<A, P, U>(kind, fixed, jobs, items, n_items, counter, lds, workgroups, stream)
+    return launch_batch_kind<A, P, U>(kind, fixed, wide, jobs, items, n_items, counter, lds, workgroups, stream)
     if (arc) {
         if (phase) {
             if (lut) BCSIM_BATCH(true, true, true);
@@ -927,7 +943,10 @@ static hipError_t launch_tile_f(const ProjCommon& c, const CullParams& cp, const
         tile_lds_bytes(cfg.window_bins, tile_bin_bytes(PHASE, FIXED), cfg.tile_lines, cfg.list_cap, cfg.list_packed);
     auto k = project_tile_kernel<ARC, PHASE, LUT, SPLINE, SHARED, FIXED>;
     if constexpr (!SHARED)
-        if (cfg.tile_lines == 1) k = project_line_kernel<ARC, PHASE, LUT, SPLINE, FIXED>;
+        if (cfg.tile_lines == 1)
+            k = project_line_kernel<ARC, PHASE, LUT, SPLINE, typename std::conditional<FIXED, long long, float>::type>;
+    if constexpr (LUT && !SHARED && FIXED)
+        if (cfg.wide) k = project_line_kernel<ARC, PHASE, LUT, SPLINE, double>;
     hipError_t e = allow_lds((const void*)k, lds);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k, dim3(tiles * cfg.windows, cfg.slices), dim3(cfg.block), lds, stream, c, cp, fs, ss, boxes,
@@ -939,7 +958,8 @@ template <bool ARC, bool PHASE, bool LUT, bool SPLINE, bool SHARED>
 static hipError_t launch_tile_t(const ProjCommon& c, const CullParams& cp, const FixedSet& fs, const SplineSet& ss,
                                 const ChunkBox* boxes, int nchunks, float* bins, const TileLaunch& cfg,
                                 hipStream_t stream) {
-    if (cfg.fixed)
+    if (cfg.wide && (!LUT || SHARED || cfg.tile_lines != 1)) return hipErrorInvalidValue;
+    if (cfg.fixed || cfg.wide)  // bins of eight bytes
         return launch_tile_f<ARC, PHASE, LUT, SPLINE, SHARED, true>(c, cp, fs, ss, boxes, nchunks, bins, cfg, stream);
     return launch_tile_f<ARC, PHASE, LUT, SPLINE, SHARED, false>(c, cp, fs, ss, boxes, nchunks, bins, cfg, stream);
 }

@@ -298,6 +298,7 @@ struct TileLaunch {
     int block;                // threads per workgroup (multiple of 64)
     int atomic;               // flush with global atomics
     int fixed;                // LDS bins as 64-bit fixed point (ProjCommon::amp_scale), else float
+    int wide;                 // LDS bins as double: one-line tiles of a lookup table (fixed is 0)
     int list_cap;             // chunk list entries in LDS (multiple of 64)
     int list_packed;          // 1: an entry is one 32-bit word, chunk << 4 | line mask (tiles of at most
                               // 4 lines, fewer than 2^28 chunks); 0: two words, chunk and mask
@@ -324,7 +325,7 @@ constexpr int kMaxOrderedTiles = 65536;
 // One projection job of a batch: a (simulator, dataset) pair with everything its
 // tile kernel would receive as arguments.
 enum JobFlags { kJobArc = 1, kJobPhase = 2, kJobLut = 4, kJobSpline = 8, kJobShared = 16, kJobFixed = 32,
-                kJobRange = 64 };  // projected in range order (J.g.range; a Gaussian beam, bins stored)
+                kJobRange = 64, kJobWide = 128 };  // projected in range order (J.g.range; a Gaussian beam, bins stored)
 
 struct ProjJob {
     ProjCommon c;
@@ -399,8 +400,8 @@ hipError_t launch_range_batch(bool phase, const ProjJob* jobs, const int2* items
 hipError_t launch_range_sort(const ProjCommon& c, const FixedSet& s, const RangeLaunch& R, hipStream_t stream);
 hipError_t launch_project_range(const ProjCommon& c, const CullParams& cp, const RangeLaunch& R, float* out,
                                 bool phase, bool lut, int accumulate, unsigned long long* stats, hipStream_t stream);
-// Bytes of one LDS bin of the tile kernel: float or 64-bit fixed point, real or complex.
-inline size_t tile_bin_bytes(bool complex_bins, bool fixed) { return (fixed ? 8 : 4) * (complex_bins ? 2 : 1); }
+// Bytes of one LDS bin of the tile kernel: float, or wide (64-bit fixed point, double), real or complex.
+inline size_t tile_bin_bytes(bool complex_bins, bool wide) { return (wide ? 8 : 4) * (complex_bins ? 2 : 1); }
 size_t tile_lds_bytes(int window_bins, size_t bin_bytes, int tile_lines, int list_cap, int list_packed);
 // Orders blocks 0..n-1 (n <= kMaxOrderedTiles) by work[], heaviest first, into
 // order[] and clears work[] for the next tile launch to fill.
@@ -412,7 +413,7 @@ hipError_t launch_order_segments(const OrderSeg* segs, int n_segs, hipStream_t s
 // shared origin (which only matters for fixed points with arc projection).
 inline int batch_variant(int flags) {
     if (flags & kJobRange) return flags & (kJobRange | kJobArc | kJobPhase);
-    int f = flags & (kJobArc | kJobPhase | kJobLut | kJobSpline | kJobShared | kJobFixed);
+    int f = flags & (kJobArc | kJobPhase | kJobLut | kJobSpline | kJobShared | kJobFixed | kJobWide);
     if (!(f & kJobArc) || (f & kJobSpline)) f &= ~kJobShared;
     return f;
 }

@@ -516,10 +516,10 @@ struct bcsim_sim {
     // integer LDS atomics; exact sums of contributions rounded to a grid of about
     // 2^-61 of the launch's largest possible bin), float ("float", ds_add_f32), or
     // "auto" (0): tuned where tuning is on, else fixed for the Gaussian profile and
-    // float for a LUT (target_fixed).  Datasets whose amplitudes the grid does not
+    // float or double for a LUT (target_bins).  Datasets whose amplitudes the grid does not
     // resolve (a non-finite amplitude, or a peak beyond ~2^39/n times the median;
     // set_fixed_scale) use float bins.
-    int bin_mode = 0;  // 0 auto, 1 fixed, 2 float (TileTune::bins)
+    int bin_mode = kBinsAuto;  // or kBinsFixed, kBinsFloat
     std::vector<std::unique_ptr<DevBuf>> tile_order_bufs;  // per projection target: [work | order]
     int radix = 0;          // FFT pass radix set by the user (4 or 8); 0 = tuned or default
     std::string last_plan;  // launch shapes of the last frame, for get_parameter("launch_plan")
@@ -723,7 +723,7 @@ struct bcsim_sim {
         if (key == "autotune") return autotune ? "on" : "off";
         if (key == "tile_order") return tile_order ? "on" : "off";
         if (key == "chunk_order") return chunk_order ? "on" : "off";
-        if (key == "bin_accumulation") return bin_mode == 1 ? "fixed" : bin_mode == 2 ? "float" : "auto";
+        if (key == "bin_accumulation") return bin_name(bin_mode);
         if (key == "fft_radix") return std::to_string(radix);
         if (key == "launch_plan") return last_plan;
         if (key == "autotune_report") return TuneCache::get().report();
@@ -1477,14 +1477,15 @@ struct bcsim_sim {
         return true;
     }
 
-    // Launch shape of the tile kernel for `tune` (0 fields: heuristic): one
+    // Launch shape of the tile kernel for `tune` (0 fields: heuristic) and `bins`
+    // (target_bins): one
     // radial window unless a line's bins overflow LDS, up to 16 lines per
     // workgroup (while at least ~1024 workgroups remain), and enough chunk
     // slices to fill the chip.
-    TileLaunch tile_launch(int nchunks, const TileTune& tune, bool per_line_splines, bool fixed_bins) const {
+    TileLaunch tile_launch(int nchunks, const TileTune& tune, bool per_line_splines, int bins) const {
         TileLaunch cfg{};
         const int L = (int)lines.size();
-        const size_t bin_bytes = tile_bin_bytes(phase_delay, fixed_bins);
+        const size_t bin_bytes = tile_bin_bytes(phase_delay, bins != kBinsFloat);
         const size_t avail = (size_t)kLdsBytes - 64 * 8 - 256;  // keep room for a 64-entry list
         // radial windows: one by default (measured fastest on the workloads of the tests
         // and bench); more if one line's bins (and its geometry, kTileLineLds) do not fit
@@ -1525,7 +1526,8 @@ struct bcsim_sim {
         cfg.slices = std::max(1, (nchunks + cfg.chunks_per_slice - 1) / cfg.chunks_per_slice);
         cfg.block = tune.block > 0 ? tune.block : 1024;
         cfg.atomic = cfg.slices > 1 ? 1 : 0;
-        cfg.fixed = fixed_bins ? 1 : 0;
+        cfg.fixed = bins == kBinsFixed ? 1 : 0;
+        cfg.wide = bins == kBinsWide ? 1 : 0;
         // the rest of the LDS holds the chunk list.  When the LDS would hold it below
         // its cap and a tile has at most 4 lines, an entry is one word (chunk << 4 |
         // line mask) instead of two: twice the entries, so the list drains half as
@@ -1558,24 +1560,25 @@ struct bcsim_sim {
     // Largest |weight| of the beam profile: 1 for the Gaussian, the largest |sample| of a LUT.
     double profile_peak() const { return profile == kProfileLut ? (double)lut_peak : 1.0; }
 
-    // Does this target's launch use fixed-point bins?  Not where its amplitudes do
-    // not allow it (amp_scale 0); else the parameter if set, then `tuned` (a
+    // The LDS bins of a target's launch of shape `tt`.  Fixed point only where its
+    // amplitudes allow it (amp_scale); else the parameter if set, then `tuned` (a
     // TileTune::bins), then the default: fixed for the Gaussian profile, whose LDS
     // additions weigh on the kernel (fixed-point ones are ~10x cheaper).  For a LUT
-    // float on tiles of several lines, which the wider bins would halve (1M-point
-    // volume: 1.91 against 1.65 ms of projection) and for points of one origin; fixed
-    // where a tile is one line anyway (project_line_kernel: 191 lines against 150k
-    // points in a straight scan 79 -> 66 us a frame, 131 spline lines with phase delay
-    // 80 -> 69).
-    bool target_fixed(const ProjTarget& t, int tuned = 0) const {
-        if (!(t.c.amp_scale > 0.0f)) return false;
+    // float on tiles of several lines, which wider bins would halve (1M-point
+    // volume: 1.91 against 1.65 ms of projection) and for points of one origin; double
+    // where a tile is one line anyway (project_line_kernel, frames among others by float /
+    // fixed / double: 191 lines against 150k points in a straight scan 55.0 / 46.6 / 45.5 us,
+    // with phase delay 96 / 55 / 53, 50 lines x 300k 31.2 / 26.5 / 26.0).
+    int target_bins(const ProjTarget& t, const TileTune& tt, int tuned = kBinsAuto) const {
         const int m = bin_mode ? bin_mode : tuned;
-        if (m) return m == 1;
-        if (profile != kProfileLut) return true;
+        if (m == kBinsFixed || (!m && profile != kProfileLut))
+            return t.c.amp_scale > 0.0f ? kBinsFixed : kBinsFloat;
         const bool spline = std::strcmp(t.kind, "spline") == 0;
-        if (!spline && arc && shared_origin()) return false;
-        return tile_launch(t.nchunks, tune, spline, true).tile_lines == 1 &&
-               tile_launch(t.nchunks, tune, spline, false).tile_lines == 1;
+        if (m == kBinsFloat || profile != kProfileLut || (!spline && arc && shared_origin())) return kBinsFloat;
+        return tile_launch(t.nchunks, tt, spline, kBinsWide).tile_lines == 1 &&
+                       tile_launch(t.nchunks, tt, spline, kBinsFloat).tile_lines == 1
+                   ? kBinsWide
+                   : kBinsFloat;
     }
 
     // Key of this scan's chunk visiting order (see ChunkOrders).
@@ -1681,6 +1684,10 @@ struct bcsim_sim {
         hip_check(launch_render_spline(t.ss, B0, const_cast<float4*>(t.fs.pts), stream), "render kernel");
     }
 
+    static const char* bins_name(const TileLaunch& g) {
+        return bin_name(g.fixed ? kBinsFixed : g.wide ? kBinsWide : kBinsFloat);
+    }
+
     // Blocks (tile, window) of one slice of a tile launch.
     int tile_blocks(const TileLaunch& cfg) const {
         return (((int)lines.size() + cfg.tile_lines - 1) / cfg.tile_lines) * cfg.windows;
@@ -1745,7 +1752,7 @@ struct bcsim_sim {
         // blocks heaviest first by the counts of its own previous launch, so two warm
         // launches settle the order before three are timed
         auto cost = [&](const TileTune& tt) {
-            TileLaunch cfg = tile_launch(t.nchunks, tt, spl, target_fixed(t, tt.bins));
+            TileLaunch cfg = tile_launch(t.nchunks, tt, spl, target_bins(t, tt, tt.bins));
             const int blocks = tile_blocks(cfg);
             const bool ordered = tile_order && blocks >= kMinOrderedBlocks && blocks <= kMaxOrderedTiles;
             DevBuf order;
@@ -1766,7 +1773,7 @@ struct bcsim_sim {
                 3, 2);
             char b[64];
             std::snprintf(b, sizeof b, " [%d,%d,%d,%d,%s]=%.3f", cfg.tile_lines, cfg.block, cfg.slices, cfg.windows,
-                          cfg.fixed ? "fixed" : "float", ms);
+                          bins_name(cfg), ms);
             trials += b;
             return ms;
         };
@@ -1775,10 +1782,12 @@ struct bcsim_sim {
         // the LDS, and windows give back lines per tile (measured on the 1M-point volume
         // with phase delay: fixed bins in 4 windows of 4 lines, 2.50 ms of projection
         // against 2.67 for float bins in whole lines of 2)
-        best.bins = target_fixed(t) ? 1 : 2;
+        best.bins = target_bins(t, best);
         double best_ms = cost(best);
         std::vector<int> modes{best.bins};
-        if (fixed_ok && !bin_mode) modes.push_back(best.bins == 1 ? 2 : 1);
+        if (!bin_mode)
+            for (int b : {kBinsFixed, kBinsFloat})
+                if (b != best.bins && (b != kBinsFixed || (fixed_ok && best.bins != kBinsWide))) modes.push_back(b);
         for (int b : modes) {
             for (int K : {1, 2, 4}) {
                 if (b == best.bins && K == 1 && best.windows == 0) continue;  // the heuristic shape, timed above
@@ -1789,17 +1798,16 @@ struct bcsim_sim {
                 if (ms < best_ms) best = c, best_ms = ms;
             }
         }
-        const bool fx = target_fixed(t, best.bins);
         TileTune wide = best;  // the most lines a tile of the chosen bins and windows holds
         wide.lines = 32;
-        const int tmax = tile_launch(t.nchunks, wide, spl, fx).tile_lines;
+        const int tmax = tile_launch(t.nchunks, wide, spl, target_bins(t, wide, best.bins)).tile_lines;
         for (int T = 1; T <= tmax; T *= 2) {
             TileTune c = best;
             c.lines = T;
             const double ms = cost(c);
             if (ms < best_ms) best = c, best_ms = ms;
         }
-        const TileLaunch cur = tile_launch(t.nchunks, best, spl, fx);  // (best.bins stays as chosen)
+        const TileLaunch cur = tile_launch(t.nchunks, best, spl, target_bins(t, best, best.bins));  // (best.bins stays as chosen)
         const int blocks = (((int)lines.size() + cur.tile_lines - 1) / cur.tile_lines) * cur.windows;
         for (int wgs : {256, 512, 1024, 2048, 4096}) {
             TileTune c = best;
@@ -1824,7 +1832,7 @@ struct bcsim_sim {
 
     // Launch shape for a target: shape fields set by the user win, then the
     // tuned shape (when tuning is on), then the heuristic.
-    // tuned_bins: a trial's accumulation mode too (else target_fixed's rule).
+    // tuned_bins: a trial's accumulation mode too (else target_bins' rule).
     TileLaunch plan_tile(const ProjTarget& t, bool tune_now, bool tuned_bins = true) {
         TileTune eff = tune;
         if (tune_now) {
@@ -1835,7 +1843,7 @@ struct bcsim_sim {
             if (!eff.slices) eff.slices = tt.slices;
             if (tuned_bins) eff.bins = tt.bins;
         }
-        return tile_launch(t.nchunks, eff, std::strcmp(t.kind, "spline") == 0, target_fixed(t, eff.bins));
+        return tile_launch(t.nchunks, eff, std::strcmp(t.kind, "spline") == 0, target_bins(t, eff, eff.bins));
     }
 
     // FFT pass radix of this frame's convolution: set by the user, tuned per
@@ -2100,7 +2108,7 @@ struct bcsim_sim {
                 last_plan += std::string(t.kind) + (t.ss.iboxes ? " (interval boxes)" : "") +
                              ": lines=" + std::to_string(g.tile_lines) +
                              " block=" + std::to_string(g.block) + " slices=" + std::to_string(g.slices) +
-                             " windows=" + std::to_string(g.windows) + " bins=" + (g.fixed ? "fixed" : "float") +
+                             " windows=" + std::to_string(g.windows) + " bins=" + bins_name(g) +
                              " list=" + std::to_string(g.list_cap) + (g.list_packed ? " packed" : "") +
                              (g.range.recs ? " (replaced by range order: patches of " + std::to_string(kRangePatch) +
                                                  " lines, windows of " + std::to_string(g.range.window_bins) + " bins)"
