@@ -258,6 +258,7 @@ struct bcsim_batch {
                 // A table's staged cells would tie an item's waves to one window of one job.
                 if (targets.size() == 1 && !lut && tile_lines <= 0 && std::strcmp(t.kind, "fixed") == 0)
                     J.g.range = s->range_launch(t, J.g, J.bins, true);
+                if (J.g.range.split) J.g.range = RangeLaunch{};  // crowded points: no parts in a batch
                 J.flags = (s->arc ? kJobArc : 0) | (cplx ? kJobPhase : 0) | (lut ? kJobLut : 0) |
                           (is_spline ? kJobSpline : 0) | (shared && !is_spline ? kJobShared : 0) |
                           (J.g.fixed ? kJobFixed : 0) | (J.g.wide ? kJobWide : 0) |

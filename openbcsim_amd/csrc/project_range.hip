@@ -198,7 +198,9 @@ __global__ __launch_bounds__(1024, 8) void project_range_kernel(ProjCommon c, Cu
     const int patch0 = (turn % groups) * R.group;
     const int b0 = window * R.window_bins;
     const int nb = min(R.window_bins, c.num_rf - b0);
-    constexpr bool SINGLE = false;
+    constexpr bool SINGLE = false, PARTS = false;
+    constexpr int part_lo = 0, part_hi = 0, subs = 1;
+    constexpr double* sums = nullptr;
 #include "range_window.inc"
 }
 
@@ -215,6 +217,92 @@ static hipError_t launch_range_t(const ProjCommon& c, const CullParams& cp, cons
     return hipGetLastError();
 }
 
+// The crowded blocks of bins (more than R.split points), which project_range_kernel left at zero:
+// a block's points in up to kRangeParts parts, a workgroup takes one part and a few patches, each
+// patch by several waves where there are fewer patches than waves.  The waves' sums meet in LDS
+// as doubles; a bin then takes one float atomic a part.
+// What it is for: a wave of project_range_kernel walks all points of a run, one after another
+// (0.17 us a point with a Gaussian, 0.2 with a table).  Points crowded at some distances leave
+// the chip to a few such waves.  Frames by the runs alone, with the parts, and by the tile kernel
+// (which takes over where that is much the faster): 128 lines x 100k points within 1 mm of depth
+// 641 / 48 / 34 us, 512 x 200k 604 / 101 / 101, with a table 3495 / 142 / 205, 64 x 20k points at
+// one depth 3344 / 39 / 27.
+template <bool PHASE, bool LUT, bool COUNT>
+__global__ __launch_bounds__(512, 4) void project_range_parts_kernel(ProjCommon c, CullParams cp, RangeLaunch R,
+                                                                     float* __restrict__ out,
+                                                                     unsigned long long* __restrict__ stats) {
+    constexpr int E = PHASE ? 2 : 1, SUMS = kRangePartPatches * kRangePatch * kRangeBlock * E;
+    constexpr bool SINGLE = false, PARTS = true, ADD = true;
+    extern __shared__ __attribute__((aligned(16))) float2 cells[];  // the staged cells, then the sums
+    double* sums = reinterpret_cast<double*>(reinterpret_cast<char*>(cells) + (LUT ? range_lds_bytes(R) : 0));
+    __shared__ unsigned wave_items[8];
+    __shared__ unsigned item_of[2];
+    const int groups = (R.n_patches + kRangePartPatches - 1) / kRangePartPatches;
+    const int blocks = (c.num_rf + kRangeBlock - 1) / kRangeBlock;
+    unsigned base = 0, next = blockIdx.x;  // items of the blocks before; this workgroup's next item
+    for (int q0 = 0; q0 < blocks; q0 += 512) {
+        // items of each thread's block, and of those before it
+        const int q = q0 + (int)threadIdx.x;
+        unsigned n = 0;
+        if (q < blocks) {
+            const int len = R.start[kRangeBlock * q + kRangeBlock] - R.start[kRangeBlock * q];
+            if (len > R.split) n = (unsigned)range_parts(len) * (unsigned)groups;
+        }
+        unsigned incl = n;
+        for (int d = 1; d < 64; d <<= 1) {
+            const unsigned t = __shfl_up(incl, d);
+            if ((int)(threadIdx.x & 63) >= d) incl += t;
+        }
+        if ((threadIdx.x & 63) == 63) wave_items[threadIdx.x >> 6] = incl;
+        __syncthreads();
+        unsigned total = 0, before = base + incl - n;
+        for (int w = 0; w < 8; w++) {
+            total += wave_items[w];
+            if (w < (int)(threadIdx.x >> 6)) before += wave_items[w];
+        }
+        __syncthreads();
+        for (; next < base + total; next += gridDim.x) {
+            if (next >= before && next < before + n) item_of[0] = (unsigned)q, item_of[1] = next - before;
+            for (int i = threadIdx.x; i < SUMS; i += 512) sums[i] = 0.0;
+            __syncthreads();
+            const int b0 = kRangeBlock * (int)__builtin_amdgcn_readfirstlane(item_of[0]);
+            const int item = (int)__builtin_amdgcn_readfirstlane(item_of[1]);
+            const int nb = min(kRangeBlock, c.num_rf - b0), patch0 = item % groups * kRangePartPatches;
+            const int begin = R.start[b0], end = R.start[b0 + nb];
+            // parts of the whole block, whose last bins may lie beyond the line
+            const int len = R.start[b0 + kRangeBlock] - begin;
+            const int each = (len - 1) / range_parts(len) + 1;
+            const int part_lo = min(begin + item / groups * each, end), part_hi = min(part_lo + each, end);
+            const int patches = min(kRangePartPatches, R.n_patches - patch0);
+            const int subs = max(1, 8 / patches);
+            {
+#include "range_window.inc"
+            }
+            __syncthreads();
+            for (int i = threadIdx.x; i < patches * kRangePatch * kRangeBlock * E; i += 512) {
+                const int bin = i / E % kRangeBlock, line = i / E / kRangeBlock;
+                const RangePatch& p = R.patches[patch0 + line / kRangePatch];
+                const float v = (float)sums[i];
+                if (line % kRangePatch < p.n && bin < nb && v != 0.0f)
+                    unsafeAtomicAdd(out + ((size_t)p.line[line % kRangePatch] * c.num_rf + b0 + bin) * E + i % E, v);
+            }
+            __syncthreads();  // the next item reuses the LDS
+        }
+        base += total;
+    }
+}
+
+template <bool PHASE, bool LUT, bool COUNT>
+static hipError_t launch_parts_t(const ProjCommon& c, const CullParams& cp, const RangeLaunch& R, float* out,
+                                 unsigned long long* stats, hipStream_t stream) {
+    auto k = project_range_parts_kernel<PHASE, LUT, COUNT>;
+    const size_t lds = (LUT ? range_lds_bytes(R) : 0) + range_part_lds_bytes(PHASE);
+    const hipError_t e = allow_lds((const void*)k, lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k, dim3(kRangePartGrid), dim3(512), lds, stream, c, cp, R, out, stats);
+    return hipGetLastError();
+}
+
 // The runs of many jobs' patches, for Gaussian beams.  A job's items share its runs, far ones
 // first: 16 waves an item, in workgroups of four (nothing in LDS ties them together).
 template <bool PHASE>
@@ -226,7 +314,9 @@ __global__ __launch_bounds__(256, 8) void project_range_batch_kernel(const ProjJ
     const CullParams& cp = J.cp;
     const RangeLaunch& R = J.g.range;
     float* __restrict__ out = J.bins;
-    constexpr bool LUT = false, ADD = false, COUNT = false, SINGLE = true;
+    constexpr bool LUT = false, ADD = false, COUNT = false, SINGLE = true, PARTS = false;
+    constexpr int part_lo = 0, part_hi = 0, subs = 1;
+    constexpr double* sums = nullptr;
     constexpr unsigned long long* stats = nullptr;
     const int turn = __builtin_amdgcn_readfirstlane((blockIdx.x & 3) * 4 + (threadIdx.x >> 6));
     const int all_runs = (c.num_rf + R.run_bins - 1) / R.run_bins;
@@ -253,8 +343,8 @@ hipError_t launch_range_sort(const ProjCommon& c_in, const FixedSet& s, const Ra
     return hipGetLastError();
 }
 
-hipError_t launch_project_range(const ProjCommon& c, const CullParams& cp, const RangeLaunch& R, float* out,
-                                bool phase, bool lut, int accumulate, unsigned long long* stats, hipStream_t stream) {
+static hipError_t launch_runs(const ProjCommon& c, const CullParams& cp, const RangeLaunch& R, float* out, bool phase,
+                              bool lut, int accumulate, unsigned long long* stats, hipStream_t stream) {
 #define BCSIM_RANGE(P, U)                                                                  \
     return stats ? (accumulate ? launch_range_t<P, U, true, true>(c, cp, R, out, stats, stream)   \
                                : launch_range_t<P, U, false, true>(c, cp, R, out, stats, stream)) \
@@ -267,6 +357,22 @@ hipError_t launch_project_range(const ProjCommon& c, const CullParams& cp, const
     if (lut) BCSIM_RANGE(false, true);
     BCSIM_RANGE(false, false);
 #undef BCSIM_RANGE
+}
+
+hipError_t launch_project_range(const ProjCommon& c, const CullParams& cp, const RangeLaunch& R, float* out,
+                                bool phase, bool lut, int accumulate, unsigned long long* stats, hipStream_t stream) {
+    const hipError_t e = launch_runs(c, cp, R, out, phase, lut, accumulate, stats, stream);
+    if (e != hipSuccess || !R.split) return e;
+#define BCSIM_PARTS(P, U)                                                     \
+    return stats ? launch_parts_t<P, U, true>(c, cp, R, out, stats, stream)   \
+                 : launch_parts_t<P, U, false>(c, cp, R, out, stats, stream)
+    if (phase) {
+        if (lut) BCSIM_PARTS(true, true);
+        BCSIM_PARTS(true, false);
+    }
+    if (lut) BCSIM_PARTS(false, true);
+    BCSIM_PARTS(false, false);
+#undef BCSIM_PARTS
 }
 
 }  // namespace bcsim_hip

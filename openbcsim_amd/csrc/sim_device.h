@@ -284,10 +284,24 @@ struct RangeLaunch {
     int group;                // patches of a workgroup
     int block;                // threads per workgroup
     int sort;                 // 1: sort the points into recs, start first; 2: sort only
+    // or 0: blocks of kRangeBlock bins with more points than this are projected in parts, by
+    // another kernel (window_bins >= kRangeBlock; its LDS beside the staged cells)
+    int split;
 };
 
+// The parts kernel: a crowded block's bins, the patches of a workgroup, the most parts of a block
+// (a bin takes a float atomic from each) and the workgroups of a launch.
+constexpr int kRangeBlock = 4, kRangePartPatches = 8, kRangeParts = 64, kRangePartGrid = 1024;
+__host__ __device__ inline int range_parts(int points) {
+    const int parts = (points - 1) / 512 + 1;
+    return parts < kRangeParts ? parts : kRangeParts;
+}
+inline size_t range_part_lds_bytes(bool phase) {
+    return (size_t)kRangePartPatches * kRangePatch * kRangeBlock * (phase ? 2 : 1) * sizeof(double);
+}
+
 // LDS of a projection workgroup with a lookup table: the staged radial cells.
-inline size_t range_lds_bytes(const RangeLaunch& R) { return (size_t)(R.max_slices - 1) * R.cell_floats * 4; }
+__host__ __device__ inline size_t range_lds_bytes(const RangeLaunch& R) { return (size_t)(R.max_slices - 1) * R.cell_floats * 4; }
 
 struct TileLaunch {
     int tile_lines;           // lines whose bins one workgroup keeps in LDS (<= 32)

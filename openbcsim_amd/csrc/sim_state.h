@@ -20,6 +20,7 @@
 #include "../../include/bcsim_c.h"
 #include "autotune.h"
 #include "host_copy.h"
+#include "range_rule.h"
 #include "sim_device.h"
 
 
@@ -258,6 +259,7 @@ struct FixedDataset {
     int nchunks = 0;
     double peak_amp = 0.0;  // largest |amplitude| (infinite if any is not finite)
     double typ_amp = 0.0;   // median |amplitude| of the non-zero amplitudes
+    PointSample sample;
     mutable ChunkOrders visit;
     mutable RangeOrders by_range;
 };
@@ -279,6 +281,7 @@ struct SplineDataset {
     // (measured on the 200k-spline M-mode phantom with 0.5 mm of jitter: 0.1265 ->
     // 0.1287 ms with them, against 0.1393 -> 0.1361 ms on a phantom contracting by 8 mm)
     bool use_iboxes = false;
+    PointSample sample;
     mutable ChunkOrders visit;
 };
 
@@ -568,6 +571,14 @@ struct bcsim_sim {
     DevBuf d_patches;  // RangePatch[n_patches] of the lines' directions
     int n_patches = 0;
     float patch_dl = 0.0f, patch_de = 0.0f;  // means of their dl and de
+    ScanCone cone{};                         // of all lines (its beam is set per frame)
+    // where the points of this configuration's datasets crowd
+    struct Crowd {
+        const void* set;
+        uint64_t version;
+        RangeCrowd at;
+    };
+    std::vector<Crowd> crowds;
     bool dirty_patches = true;
     DevBuf d_stats;  // with store_kernel_details: per projection launch, weight evaluations and LDS additions
 
@@ -903,6 +914,12 @@ struct bcsim_sim {
             boxes[c] = acc.box();
         }
         ds->visit.set_boxes(boxes);
+        ds->sample.resize(n, PointSample::kPoints, 1);
+        const std::vector<size_t> at = PointSample::choose(n, PointSample::kPoints);
+        for (size_t i = 0; i < at.size(); i++) {
+            const float* p = &sorted[4 * at[i]];
+            ds->sample.x[i] = p[0], ds->sample.y[i] = p[1], ds->sample.z[i] = p[2];
+        }
         ds->pts.ensure(n * sizeof(float4));
         ds->boxes.ensure(boxes.size() * sizeof(ChunkBox));
         if (n) {
@@ -987,6 +1004,13 @@ struct bcsim_sim {
             }
             ds->use_iboxes = part < 0.95 * whole;
         }
+        ds->sample.resize(n, PointSample::kSplines, num_cp);
+        const std::vector<size_t> at = PointSample::choose(n, PointSample::kSplines);
+        for (int k = 0; k < num_cp; k++)
+            for (size_t i = 0; i < at.size(); i++) {
+                const size_t from = (size_t)k * n + at[i], to = (size_t)k * at.size() + i;
+                ds->sample.x[to] = px[from], ds->sample.y[to] = py[from], ds->sample.z[to] = pz[from];
+            }
         const size_t b = px.size() * sizeof(float);
         ds->cx.ensure(b);
         ds->cy.ensure(b);
@@ -1947,9 +1971,29 @@ struct bcsim_sim {
         hip_check(hipMemcpy(d_patches.p, patches.data(), patches.size() * sizeof(RangePatch), hipMemcpyHostToDevice),
                   "hipMemcpy");
         n_patches = (int)patches.size();
+        bound(order.data(), order.data() + order.size(), &LineGeom::rx, cone.r);
+        bound(order.data(), order.data() + order.size(), &LineGeom::lx, cone.l);
+        bound(order.data(), order.data() + order.size(), &LineGeom::ex, cone.e);
         patch_dl = patch_de = 0.0f;
         for (const RangePatch& q : patches) patch_dl += q.dl / n_patches, patch_de += q.de / n_patches;
         dirty_patches = false;
+    }
+
+    // Where target t's points crowd, by distance from lines[0]'s origin: worked out once per
+    // configuration.
+    const RangeCrowd& crowd(const ProjTarget& t, float beam_l, float beam_e) {
+        const void* set = t.fixed ? (const void*)t.fixed : t.sp;
+        for (const Crowd& q : crowds)
+            if (q.set == set && q.version == version) return q.at;
+        if (!crowds.empty() && crowds[0].version != version) crowds.clear();
+        SplineLineBasis B{0, 1, {1.0f}};
+        if (t.sp) host_basis_line0(*t.sp, B);
+        cone.beam_l = beam_l, cone.beam_e = beam_e;
+        const LineGeom& L = lines[0];
+        crowds.push_back({set, version,
+                          range_crowd(t.sp ? t.sp->sample : t.fixed->sample, B.lo, B.count, B.b, L.ox, L.oy, L.oz, cone,
+                                      (float)t.c.bins_per_metre, num_rf, kRangeBlock)});
+        return crowds.back().at;
     }
 
     // Projection of target t in range order (project_range.hip), or a launch without
@@ -2026,6 +2070,55 @@ struct bcsim_sim {
             R.group = std::min(n_patches, waves);
             R.window_bins = R.run_bins * ((waves + R.group - 1) / R.group);
         }
+        // What points that crowd at some distances cost (they leave the chip to a few waves that walk
+        // them one by one).  Estimates in us, fitted to the kernel times of 3000 frames of uniform
+        // points, shells and mixtures of both, 16 to 4096 lines, 1k to 1M points; half lie within
+        // 15 %, nearly all within 50 %: this kernel apart from its longest run, that run by its wave
+        // (or its window by a workgroup), the crowded blocks in parts, and the tile kernel.
+        const RangeCrowd& at = crowd(t, (float)std::min(beam_l, 1e3), (float)std::min(beam_e, 1e3));
+        double reach = 1.0, frac = 1.0;  // shares of the points in reach of a line, of a patch
+        const auto axis = [&](double beam, float whole, float part) {
+            const double w = mid * (double)whole + 1e-9;
+            reach *= std::min(1.0, beam / w);
+            frac *= std::min(1.0, (beam + mid * (double)part) / w);
+        };
+        axis(beam_l, cone.l[3], patch_dl);
+        axis(beam_e, cone.e[3], patch_de);
+        const double mega_bins = 1e-6 * (double)lines.size() * num_rf * (phase_delay ? 2 : 1);
+        const double visits = 1e-6 * at.seen * n_patches, pairs = 1e-6 * at.seen * (double)lines.size();
+        const double few = std::log10(std::max(1.0, at.seen / 1000.0));
+        const double run = at.heaviest(R.run_bins, kRangeBlock), block = at.heaviest(kRangeBlock, kRangeBlock);
+        double base, longest, tile;
+        if (lut_profile) {
+            const double windows = std::ceil((double)num_rf / R.window_bins) * ((n_patches + R.group - 1) / R.group);
+            const double cells = 1e-6 * windows * (R.max_slices - 1) * lut_nl * lut_ne;
+            base = 8.0 + 1.25 * mega_bins + 1.5 * cells + 10.7 * visits;
+            longest = frac * std::max(0.2 * run, (0.045 + 12.8 * R.group / R.block) * at.heaviest(R.window_bins, kRangeBlock));
+            tile = 8.5 + 7.0 * few + 2.7 * mega_bins + (phase_delay ? 8.1 : 4.6) * pairs * reach + 0.14 * pairs;
+        } else {
+            base = 5.5 + 2.3 * mega_bins + 6.7 * visits;
+            longest = frac * 0.15 * run;
+            tile = 8.4 + 4.7 * few + 2.6 * mega_bins + (phase_delay ? 3.8 : 2.4) * pairs * reach + 0.15 * pairs;
+        }
+        const double limit = 0.5 * base + 8.0;  // a walk this long hides behind the rest
+        double parts = INFINITY;
+        if (longest > limit && !(lut_profile && R.window_bins < kRangeBlock) &&
+            range_part_lds_bytes(phase_delay) + (lut_profile ? range_lds_bytes(R) : 0) <= (size_t)kLdsBytes - 512) {
+            const int waves = std::max(1, 8 / std::min(n_patches, kRangePartPatches));  // of a patch
+            const double walk = frac * std::max(std::min(512.0, block), block / kRangeParts) / waves;
+            const double items = std::ceil((double)n_patches / kRangePartPatches) * (at.seen / 512.0 + 2.0 * at.seen / block);
+            parts = limit + 6.0 + std::ceil(items / 512.0) * (lut_profile ? 20.0 + 0.2 * walk : 6.0 + 0.15 * walk);
+            if (parts < longest) R.split = (int)std::min(1e9, std::max(64.0, block * limit / longest));
+        }
+        // The tile kernel where it clearly saves time: alone, walks are the frame's latency, but among
+        // other frames the chip works on those meanwhile.  700 frames as above: uniform points
+        // 0.65 of the tile kernel's time (median) to 1.26 (95th percentile), crowded ones 1.0 to
+        // 2.9, which took 4.3 and 134 times as long before this rule and the parts.
+        if (base + std::min(parts, longest) > 1.1 * tile + 60.0) return RangeLaunch{};
+        // Few points do not earn the staging of a large table (1000 points, 48 lines, 256 x 64 x 64
+        // samples 21 us a frame, by the tile kernel 17; 10k points 22.9 and 24.6).
+        if (lut_profile && at.seen < 4000.0 && base > tile) return RangeLaunch{};
+        if (rendered && R.split) return RangeLaunch{};  // their sort, too, counts a bin's points one by one
         if (rendered) {  // other points every frame: sorted by each, into this simulator's buffers
             const bool fits = where_it_fits([&] {
                 t.scan->recs.ensure(t.n * sizeof(RangeRec));
@@ -2111,7 +2204,10 @@ struct bcsim_sim {
                              " windows=" + std::to_string(g.windows) + " bins=" + bins_name(g) +
                              " list=" + std::to_string(g.list_cap) + (g.list_packed ? " packed" : "") +
                              (g.range.recs ? " (replaced by range order: patches of " + std::to_string(kRangePatch) +
-                                                 " lines, windows of " + std::to_string(g.range.window_bins) + " bins)"
+                                                 " lines, windows of " + std::to_string(g.range.window_bins) + " bins" +
+                                                 (g.range.split ? ", blocks of more than " +
+                                                                      std::to_string(g.range.split) + " points in parts)"
+                                                                : std::string(")"))
                                            : "") +
                              "\n";
             }

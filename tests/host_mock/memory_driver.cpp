@@ -198,10 +198,60 @@ static void optional_buffers() {
     CHK(bcsim_destroy(s));
 }
 
+// Points that crowd: few lines and points are projected in parts, many by the tile kernel;
+// uniform points, and points beyond the lines, in range order as they are.
+static std::vector<float> shell_points(size_t n, float radius, float share) {
+    std::vector<float> p = box_points(n);
+    std::mt19937 rng(4);
+    std::uniform_real_distribution<float> u(-0.6f, 0.6f);
+    for (size_t i = 0; i < (size_t)(share * n); i++) {
+        const float a = u(rng);
+        p[4 * i] = radius * sinf(a), p[4 * i + 1] = 0, p[4 * i + 2] = radius * cosf(a);
+    }
+    return p;
+}
+static void crowds() {
+    struct Case {
+        int lines;
+        size_t n;
+        float radius, share;
+        bool table, in_order, parts;
+    };
+    for (const Case& q : {Case{128, 100000, 0.03f, 0.0f, false, true, false}, Case{128, 100000, 0.03f, 0.0f, true, true, false},
+                          Case{40, 8000, 0.03f, 1.0f, false, true, true}, Case{40, 8000, 0.03f, 1.0f, true, true, true},
+                          Case{128, 400000, 0.03f, 1.0f, false, false, false}, Case{64, 100000, 0.03f, 0.3f, true, true, true},
+                          Case{128, 100000, 0.2f, 0.5f, false, true, false}}) {
+        bcsim_sim* s = simulator(q.lines, 0);
+        const std::vector<float> p = shell_points(q.n, q.radius, q.share);
+        CHK(bcsim_add_fixed_scatterers(s, p.data(), q.n));
+        if (q.table) CHK(set_table(s, 16));
+        const bool in_order = ranged(s);
+        const bool parts = plan(s).find("in parts") != std::string::npos;
+        if (in_order != q.in_order || parts != q.parts) fprintf(stderr, "%d lines %zu points: %s", q.lines, q.n, plan(s).c_str());
+        REQUIRE(in_order == q.in_order && parts == q.parts);
+        // the same points as splines at one time: sorted every frame, which crowds slow down too
+        if (q.lines == 128 && !q.table) {
+            std::vector<float> cp, amp;
+            for (size_t i = 0; i < q.n; i++) {
+                for (int k = 0; k < 4; k++) cp.insert(cp.end(), {p[4 * i], p[4 * i + 1], p[4 * i + 2]});
+                amp.push_back(p[4 * i + 3]);
+            }
+            const float knots[] = {0, 0, 0, 0, 1, 1, 1, 1};
+            CHK(bcsim_clear_fixed_scatterers(s));
+            CHK(bcsim_add_spline_scatterers(s, 3, knots, 8, cp.data(), amp.data(), q.n, 4));
+            Scan wide = sector(256);
+            for (auto& t : wide.t) t = 0.4f;
+            set_scan(s, wide, true);
+            REQUIRE(ranged(s) == (q.share == 0.0f || q.radius > 0.05f));
+        }
+        CHK(bcsim_destroy(s));
+    }
+}
+
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     const std::vector<std::pair<std::string, void (*)()>> all = {
-        {"table_failures", table_failures}, {"optional_buffers", optional_buffers}};
+        {"table_failures", table_failures}, {"optional_buffers", optional_buffers}, {"crowds", crowds}};
     for (auto& e : all)
         if (e.first == what) {
             e.second();
