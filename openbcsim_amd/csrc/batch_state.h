@@ -74,6 +74,7 @@ struct bcsim_batch {
         float4* out;
     };
     std::vector<Render> renders;
+    std::vector<RangeOrders::Ref> orders;  // what the job table names
     int workgroups = 256;
     bool have_cu_count = false;
     bool autotune = true;          // tune each job's shape class before its first batched frame
@@ -212,6 +213,7 @@ struct bcsim_batch {
         }
         plan.clear();
         renders.clear();
+        orders.clear();
         std::vector<ProjJob> pjobs;
         std::vector<double> pcost;  // per-item cost estimate of each projection job
         std::vector<ConvParams> cjobs;
@@ -259,6 +261,8 @@ struct bcsim_batch {
                 if (targets.size() == 1 && !lut && tile_lines <= 0 && std::strcmp(t.kind, "fixed") == 0)
                     J.g.range = s->range_launch(t, J.g, J.bins, true);
                 if (J.g.range.split) J.g.range = RangeLaunch{};  // crowded points: no parts in a batch
+                if (J.g.range.recs) orders.insert(orders.end(), s->order_refs.begin(), s->order_refs.end());
+                s->order_refs.clear();
                 J.flags = (s->arc ? kJobArc : 0) | (cplx ? kJobPhase : 0) | (lut ? kJobLut : 0) |
                           (is_spline ? kJobSpline : 0) | (shared && !is_spline ? kJobShared : 0) |
                           (J.g.fixed ? kJobFixed : 0) | (J.g.wide ? kJobWide : 0) |

@@ -6,6 +6,7 @@
 
 #include <algorithm>
 #include <array>
+#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -208,14 +209,19 @@ struct ChunkOrders {
 };
 
 // A dataset's points sorted by radial bin from a scan origin (project_range.hip), one
-// copy (36 bytes a point) per origin, bin rule and demodulation phase.  Like the chunk
-// orders they live as long as the dataset; further origins run the tile kernel.
+// copy (36 bytes a point) per origin, bin rule and, for frames with phase delay,
+// demodulation phase.  At most kMaxOrders; a further origin runs the tile kernel, and takes
+// the place of the order longest unused once it comes again and that one has not been used
+// in between: a scan that stays where it went gets its order, one that wanders, or more
+// scans by turns than there are orders, does not sort for every frame.
 struct RangeOrders {
     struct Key {
         float ox, oy, oz, phase;
         double scale, denom;
-        bool operator==(const Key& k) const {
-            return ox == k.ox && oy == k.oy && oz == k.oz && phase == k.phase && scale == k.scale && denom == k.denom;
+        // any_phase: for frames without phase delay, which do not read the rotations
+        bool serves(const Key& k, bool any_phase) const {
+            return ox == k.ox && oy == k.oy && oz == k.oz && (any_phase || phase == k.phase) && scale == k.scale &&
+                   denom == k.denom;
         }
     };
     struct Order {
@@ -223,22 +229,37 @@ struct RangeOrders {
         DevBuf mem;  // the records, the first record of each bin, and the sort's counts and ranks
         RangeRec* recs;
         int* start;
+        uint64_t used;  // get()'s count when it was last asked for
     };
+    // Held while a frame is enqueued or a batch's tables name it; frames in flight are waited
+    // for when it is freed.
+    using Ref = std::shared_ptr<const Order>;
     static constexpr size_t kMaxOrders = 4;
     std::mutex mu;
-    std::vector<std::unique_ptr<Order>> orders;
+    std::vector<std::shared_ptr<Order>> orders;
+    struct Refusal {
+        Key key;
+        uint64_t at;
+    };
+    std::vector<Refusal> refusals;  // the last kMaxOrders keys without an order
+    uint64_t asked = 0;
 
     // The order of `key`, or null.  `sort` fills a new order's buffers and waits for
     // them (other simulators may read them next, on streams of their own); null: only
     // an order built earlier.  Without memory for another copy there is no order.
     template <class Sort>
-    const Order* get(const Key& key, size_t n, const Sort* sort) {
+    Ref get(const Key& key, bool any_phase, size_t n, const Sort* sort) {
         std::lock_guard<std::mutex> g(mu);
+        asked++;
         for (auto& o : orders)
-            if (o->key == key) return o.get();
-        if (!sort || orders.size() >= kMaxOrders) return nullptr;
-        auto o = std::make_unique<Order>();
+            if (o->key.serves(key, any_phase)) {
+                o->used = asked;
+                return o;
+            }
+        if (!sort || (orders.size() >= kMaxOrders && !replace(key, any_phase))) return nullptr;
+        auto o = std::make_shared<Order>();
         o->key = key;
+        o->used = asked;
         const bool fits = where_it_fits([&] {
             // one allocation (a new dataset's first frame waits for each)
             o->mem.ensure(n * sizeof(RangeRec) + (2 * kRangeBins + 4 + n) * sizeof(int));
@@ -247,8 +268,30 @@ struct RangeOrders {
             (*sort)(o->recs, o->start, o->start + kRangeBins + 4);
         });
         if (!fits) return nullptr;
-        orders.push_back(std::move(o));
-        return orders.back().get();
+        orders.push_back(o);
+        return o;
+    }
+
+  private:
+    // Gives back the order that `key` may take the place of, if there is one (mu held).
+    bool replace(const Key& key, bool any_phase) {
+        const auto known = std::find_if(refusals.begin(), refusals.end(),
+                                        [&](const Refusal& r) { return r.key.serves(key, any_phase); });
+        if (known == refusals.end()) {
+            if (refusals.size() >= kMaxOrders) refusals.erase(refusals.begin());
+            refusals.push_back({key, asked});
+            return false;
+        }
+        auto oldest = orders.end();
+        for (auto o = orders.begin(); o != orders.end(); ++o)
+            if (o->use_count() == 1 && (*o)->used < known->at && (oldest == orders.end() || (*o)->used < (*oldest)->used))
+                oldest = o;
+        if (oldest == orders.end()) return false;
+        refusals.erase(known);
+        std::atomic_thread_fence(std::memory_order_acquire);  // its last holder let go of it
+        hip_check(hipDeviceSynchronize(), "hipDeviceSynchronize");  // frames in flight may read it
+        orders.erase(oldest);
+        return true;
     }
 };
 
@@ -579,6 +622,7 @@ struct bcsim_sim {
         RangeCrowd at;
     };
     std::vector<Crowd> crowds;
+    std::vector<RangeOrders::Ref> order_refs;  // what range_launch() handed out, for its caller to keep or drop
     bool dirty_patches = true;
     DevBuf d_stats;  // with store_kernel_details: per projection launch, weight evaluations and LDS additions
 
@@ -2151,8 +2195,9 @@ struct bcsim_sim {
             launch_target(t, g, bins);
             hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
         };
-        const RangeOrders::Order* o = t.fixed->by_range.get(key, t.n, create ? &sort : nullptr);
+        const RangeOrders::Ref o = t.fixed->by_range.get(key, !phase_delay, t.n, create ? &sort : nullptr);
         if (!o) return R;
+        order_refs.push_back(o);
         R.patches = d_patches.as<RangePatch>();
         R.start = o->start;
         R.recs = o->recs;
@@ -2187,6 +2232,7 @@ struct bcsim_sim {
 
         const std::vector<ProjTarget> targets = proj_targets(fm);
         enqueue_renders(targets);
+        order_refs.clear();
         // plan every launch first: tuning trials write the bins
         std::vector<TileLaunch> plans;
         std::vector<ProjLaunch> direct_plans;
@@ -2273,6 +2319,7 @@ struct bcsim_sim {
             hip_check(launch_convolve_demod(p, stream), "convolve/demodulate kernel");
             t.stop();
         }
+        order_refs.clear();
     }
 
     // The inverse transform is folded by the largest power of two dividing the

@@ -40,10 +40,11 @@ hipError_t mock_launch_project_tile(const ProjCommon& c, const CullParams& cp, c
 
 // ---- failures: the allocation or copy for which the predicate holds fails
 static std::function<bool(size_t)> fail_malloc, fail_copy;
-static int mallocs = 0;  // allocations since the last reset
+static int mallocs = 0;  // allocations of count_bytes
+static size_t count_bytes = 0;
 
 extern "C" hipError_t hipMalloc(void** ptr, size_t size) {
-    mallocs++;
+    mallocs += size == count_bytes;
     if (fail_malloc && fail_malloc(size)) {
         *ptr = nullptr;
         return hipErrorOutOfMemory;
@@ -248,10 +249,70 @@ static void crowds() {
     }
 }
 
+// Orders of a dataset: four, the one longest unused giving way to an origin that stays.
+static void origins() {
+    const size_t n = 20000;
+    bcsim_sim* s = simulator(64, n);
+    count_bytes = n * sizeof(RangeRec) + (2 * kRangeBins + 4 + n) * sizeof(int);
+    const auto at = [&](float x) {
+        set_scan(s, sector(64, x));
+        return ranged(s);
+    };
+    const auto allocated = [&] {
+        const int k = mallocs;
+        mallocs = 0;
+        return k;
+    };
+    (void)allocated();
+    // demodulation frequencies without phase delay: one order, which serves phase delay too
+    std::vector<float> pulse(55, 0.5f);
+    for (int k = 1; k <= 6; k++) {
+        CHK(bcsim_set_excitation(s, pulse.data(), 55, 27, 50e6f, k * 1e6f));
+        REQUIRE(ranged(s));
+    }
+    REQUIRE(allocated() == 1);
+    CHK(bcsim_set_parameter(s, "phase_delay", "on"));
+    CHK(bcsim_set_excitation(s, pulse.data(), 55, 27, 50e6f, 1e6f));
+    REQUIRE(ranged(s) && allocated() == 0);
+    CHK(bcsim_set_parameter(s, "phase_delay", "off"));
+    for (float x : {0.001f, 0.002f, 0.003f}) REQUIRE(at(x));
+    REQUIRE(allocated() == 3);
+    // a fifth origin: from its second frame on, in the place of the first one
+    REQUIRE(!at(0.004f) && at(0.004f) && at(0.004f) && allocated() == 1);
+    REQUIRE(at(0.001f) && at(0.002f) && at(0.003f) && allocated() == 0);
+    // more origins by turns than orders: those that have one keep it, nothing is sorted again
+    for (int turn = 0; turn < 4; turn++) {
+        for (float x : {0.001f, 0.002f, 0.003f, 0.004f}) REQUIRE(at(x));
+        REQUIRE(!at(0.0f));
+    }
+    REQUIRE(allocated() == 0);
+    // an origin that wanders: nothing is sorted, the others keep their orders
+    for (int k = 0; k < 20; k++) REQUIRE(!at(0.01f + 0.0001f * k));
+    REQUIRE(at(0.001f) && at(0.002f) && at(0.003f) && at(0.004f) && allocated() == 0);
+    // a batch's tables name orders: they stay while it lives
+    bcsim_batch* b;
+    CHK(bcsim_batch_create(&b));
+    CHK(bcsim_batch_add(b, s, nullptr));  // at 0.004
+    size_t total = 0;
+    int jobs = 0;
+    CHK(bcsim_batch_get_layout(b, &total, &jobs, nullptr, nullptr, nullptr, 0));
+    void* out = nullptr;
+    REQUIRE(hipMalloc(&out, total * 8) == hipSuccess);
+    CHK(bcsim_batch_simulate_device(b, out, total));
+    (void)allocated();
+    REQUIRE(!at(0.02f) && at(0.02f) && !at(0.021f) && at(0.021f) && !at(0.022f) && at(0.022f) && allocated() == 3);
+    REQUIRE(!at(0.023f) && at(0.023f) && allocated() == 1);  // for 0.02's: 0.004's is the batch's
+    REQUIRE(at(0.004f) && allocated() == 0);
+    CHK(bcsim_batch_synchronize(b));
+    CHK(bcsim_batch_destroy(b));
+    CHK(bcsim_destroy(s));
+    hipFree(out);
+}
+
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     const std::vector<std::pair<std::string, void (*)()>> all = {
-        {"table_failures", table_failures}, {"optional_buffers", optional_buffers}, {"crowds", crowds}};
+        {"table_failures", table_failures}, {"optional_buffers", optional_buffers}, {"crowds", crowds}, {"origins", origins}};
     for (auto& e : all)
         if (e.first == what) {
             e.second();
