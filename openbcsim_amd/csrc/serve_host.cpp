@@ -164,7 +164,12 @@ struct Frame {
 struct bcsim_server {
     int device = -1;
     size_t budget = 0;       // device bytes for phantoms, frame buffers and outputs
-    size_t used = 0;         // accounted device bytes
+    size_t used = 0;         // accounted device bytes, but for the range orders
+    // the range orders that this server's frames sorted (36 bytes a point); where the budget has no
+    // room for one the frames run without, and they make room for what a request needs
+    std::shared_ptr<std::atomic<size_t>> orders = std::make_shared<std::atomic<size_t>>(0);
+    size_t out_growth = 0;  // bytes by which the frame being launched will grow its output
+    size_t in_use() const { return used + orders->load(); }
     size_t resident = 0;     // phantom datasets and LUTs (part of `used`)
     int max_jobs = 64;       // requests per batched frame
     bool autotune = true;
@@ -228,11 +233,12 @@ struct bcsim_server {
             if (!resident_sets.count(key) && added.insert(key).second) add += bytes;
         };
         if (s.lut) count(s.lut.get(), s.lut->bytes);
+        if (s.lut_rel) count(s.lut_rel.get(), s.lut_rel->bytes);
         for (auto& f : s.fixed) count(f.get(), f->pts.bytes + f->boxes.bytes);
         for (auto& sp : s.splines)
             count(sp.get(), sp->cx.bytes + sp->cy.bytes + sp->cz.bytes + sp->amp.bytes + sp->boxes.bytes +
                                 sp->iboxes.bytes);
-        if (used + add > budget) fail(BCSIM_ERR_OUT_OF_MEMORY, "phantom datasets exceed the server's memory budget");
+        if (in_use() + add > budget) fail(BCSIM_ERR_OUT_OF_MEMORY, "phantom datasets exceed the server's memory budget");
         resident_sets.insert(added.begin(), added.end());
         resident += add;
         used += add;
@@ -303,6 +309,11 @@ struct bcsim_server {
         auto s = std::make_unique<bcsim_sim>();
         s->configure_view_of(*phantoms[p]);
         const Geometry& gm = geom(gi);
+        s->order_account = orders;
+        s->order_room = [this](size_t bytes) {  // from launch(), which does not hold mu
+            std::lock_guard<std::mutex> g(mu);
+            return in_use() + out_growth + bytes <= budget;
+        };
         s->set_scan_sequence(gm.lines(), gm.o.data(), gm.d.data(), gm.lat.data(), gm.t.data(), gm.length, true);
         s->update_shape();
         return s;
@@ -427,13 +438,16 @@ struct bcsim_server {
         return nullptr;
     }
 
-    // Free idle slots, least recently used first, until `need` more bytes fit.
+    // Free idle slots, least recently used first, then range orders, until `need` more bytes fit.
     bool make_room(size_t need, const Slot* keep) {
-        while (used + need > budget) {
+        while (in_use() + need > budget) {
             Slot* lru = nullptr;
             for (auto& s : slots)
                 if (!s->busy && s.get() != keep && (!lru || s->last_used < lru->last_used)) lru = s.get();
-            if (!lru) return false;
+            if (!lru) {
+                if (!drop_order()) return false;
+                continue;
+            }
             used -= lru->bytes;
             for (size_t i = 0; i < slots.size(); i++)
                 if (slots[i].get() == lru) {
@@ -442,6 +456,17 @@ struct bcsim_server {
                 }
         }
         return true;
+    }
+
+    // Give back a range order that no frame in flight reads (mu held).
+    bool drop_order() {
+        if (orders->load() == 0) return false;
+        for (Frame& f : frames)
+            if (!f.busy) f.batch.orders.clear();  // its tables are rebuilt before its next frame
+        for (auto& p : phantoms)
+            for (auto& f : p->fixed)
+                if (f->by_range.release_one(orders)) return true;
+        return false;
     }
 
     // Is [p, p + bytes) inside one pinned block of bcsim_server_alloc_host? (mu held)
@@ -651,6 +676,9 @@ struct bcsim_server {
         b.device = -1;
         b.invalidate();
         for (Request* r : f->reqs) b.add(r->slot->sim.get());
+        size_t out_bytes = 0;
+        for (Request* r : f->reqs) out_bytes += (size_t)r->lines * r->samples * sizeof(float2);
+        out_growth = out_bytes > f->d_out.bytes ? std::max(out_bytes, f->d_out.bytes + f->d_out.bytes / 2) - f->out_accounted : 0;
         b.build();
         const size_t total = b.total_out;
         if (f->d_out.bytes < total * sizeof(float2)) {
@@ -755,8 +783,8 @@ struct bcsim_server {
         else if (key == "lines_completed") out = {lines_done};
         else if (key == "busy_span_ms") out = {t_first_submit >= 0 && t_last_done >= 0 ? t_last_done - t_first_submit : 0.0};
         else if (key == "budget_bytes") out = {(double)budget};
-        else if (key == "used_bytes") out = {(double)used};
-        else if (key == "resident_bytes") out = {(double)resident};
+        else if (key == "used_bytes") out = {(double)in_use()};
+        else if (key == "resident_bytes") out = {(double)(resident + orders->load())};
         else if (key == "idle_slots") {
             double n = 0;
             for (auto& s : slots) n += !s->busy;
@@ -790,7 +818,7 @@ BCSIM_API bcsim_status bcsim_server_set_parameter(bcsim_server* s, const char* k
         if (k == "memory_budget_bytes") {
             const long long v = std::stoll(value);
             if (v <= 0) fail(BCSIM_ERR_INVALID_ARGUMENT, "memory budget must be positive");
-            if ((size_t)v < s->used) fail(BCSIM_ERR_INVALID_ARGUMENT, "memory budget below the bytes already in use");
+            if ((size_t)v < s->in_use()) fail(BCSIM_ERR_INVALID_ARGUMENT, "memory budget below the bytes already in use");
             s->budget = (size_t)v;
         } else if (k == "max_jobs_per_frame") {
             const int v = parse_int(value);

@@ -11,6 +11,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <functional>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -230,7 +231,12 @@ struct RangeOrders {
         RangeRec* recs;
         int* start;
         uint64_t used;  // get()'s count when it was last asked for
+        std::shared_ptr<std::atomic<size_t>> account;  // a server's, whose bytes these are (or null)
+        ~Order() {
+            if (account) *account -= mem.bytes;
+        }
     };
+    static size_t bytes(size_t n) { return n * sizeof(RangeRec) + (2 * kRangeBins + 4 + n) * sizeof(int); }
     // Held while a frame is enqueued or a batch's tables name it; frames in flight are waited
     // for when it is freed.
     using Ref = std::shared_ptr<const Order>;
@@ -247,8 +253,10 @@ struct RangeOrders {
     // The order of `key`, or null.  `sort` fills a new order's buffers and waits for
     // them (other simulators may read them next, on streams of their own); null: only
     // an order built earlier.  Without memory for another copy there is no order.
+    // account: where a new order's bytes are counted, or null.
     template <class Sort>
-    Ref get(const Key& key, bool any_phase, size_t n, const Sort* sort) {
+    Ref get(const Key& key, bool any_phase, size_t n, const Sort* sort,
+            const std::shared_ptr<std::atomic<size_t>>& account = nullptr) {
         std::lock_guard<std::mutex> g(mu);
         asked++;
         for (auto& o : orders)
@@ -262,17 +270,44 @@ struct RangeOrders {
         o->used = asked;
         const bool fits = where_it_fits([&] {
             // one allocation (a new dataset's first frame waits for each)
-            o->mem.ensure(n * sizeof(RangeRec) + (2 * kRangeBins + 4 + n) * sizeof(int));
+            o->mem.ensure(bytes(n));
             o->recs = o->mem.as<RangeRec>();
             o->start = reinterpret_cast<int*>(o->recs + n);
             (*sort)(o->recs, o->start, o->start + kRangeBins + 4);
         });
         if (!fits) return nullptr;
+        if (account) *account += o->mem.bytes;
+        o->account = account;
         orders.push_back(o);
         return o;
     }
 
+    bool has(const Key& key, bool any_phase) {
+        std::lock_guard<std::mutex> g(mu);
+        for (auto& o : orders)
+            if (o->key.serves(key, any_phase)) return true;
+        return false;
+    }
+
+    // Gives back the order longest unused of those counted in `account` that nothing holds.
+    bool release_one(const std::shared_ptr<std::atomic<size_t>>& account) {
+        std::lock_guard<std::mutex> g(mu);
+        auto oldest = orders.end();
+        for (auto o = orders.begin(); o != orders.end(); ++o)
+            if (o->use_count() == 1 && (*o)->account == account && (oldest == orders.end() || (*o)->used < (*oldest)->used))
+                oldest = o;
+        if (oldest == orders.end()) return false;
+        release(oldest);
+        return true;
+    }
+
   private:
+    void release(std::vector<std::shared_ptr<Order>>::iterator o) {
+        std::atomic_thread_fence(std::memory_order_acquire);  // its last holder let go of it
+        hip_check(hipDeviceSynchronize(), "hipDeviceSynchronize");  // frames in flight may read it
+        orders.erase(o);
+    }
+
     // Gives back the order that `key` may take the place of, if there is one (mu held).
     bool replace(const Key& key, bool any_phase) {
         const auto known = std::find_if(refusals.begin(), refusals.end(),
@@ -288,9 +323,7 @@ struct RangeOrders {
                 oldest = o;
         if (oldest == orders.end()) return false;
         refusals.erase(known);
-        std::atomic_thread_fence(std::memory_order_acquire);  // its last holder let go of it
-        hip_check(hipDeviceSynchronize(), "hipDeviceSynchronize");  // frames in flight may read it
-        orders.erase(oldest);
+        release(oldest);
         return true;
     }
 };
@@ -622,6 +655,9 @@ struct bcsim_sim {
         RangeCrowd at;
     };
     std::vector<Crowd> crowds;
+    // a server's: whether a range order of so many bytes fits its budget, and where it is counted
+    std::function<bool(size_t)> order_room;
+    std::shared_ptr<std::atomic<size_t>> order_account;
     std::vector<RangeOrders::Ref> order_refs;  // what range_launch() handed out, for its caller to keep or drop
     bool dirty_patches = true;
     DevBuf d_stats;  // with store_kernel_details: per projection launch, weight evaluations and LDS additions
@@ -909,7 +945,8 @@ struct bcsim_sim {
 
     // Device bytes this simulator holds for its frames (not the shared datasets).
     size_t frame_bytes() const {
-        size_t b = d_lines.bytes + d_H.bytes + d_demod.bytes + d_tw.bytes + d_bins.bytes + d_iq.bytes + d_iq_turned.bytes;
+        size_t b = d_lines.bytes + d_H.bytes + d_demod.bytes + d_tw.bytes + d_bins.bytes + d_iq.bytes + d_iq_turned.bytes +
+                   d_patches.bytes;
         for (auto& sc : spline_scan) b += sc->basis.bytes + sc->rendered.bytes + sc->recs.bytes + sc->sort.bytes;
         return b;
     }
@@ -2195,7 +2232,9 @@ struct bcsim_sim {
             launch_target(t, g, bins);
             hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
         };
-        const RangeOrders::Ref o = t.fixed->by_range.get(key, !phase_delay, t.n, create ? &sort : nullptr);
+        RangeOrders& orders = t.fixed->by_range;
+        if (create && order_room && !orders.has(key, !phase_delay)) create = order_room(RangeOrders::bytes(t.n));
+        const RangeOrders::Ref o = orders.get(key, !phase_delay, t.n, create ? &sort : nullptr, order_account);
         if (!o) return R;
         order_refs.push_back(o);
         R.patches = d_patches.as<RangePatch>();

@@ -309,10 +309,71 @@ static void origins() {
     hipFree(out);
 }
 
+// A server counts the orders and the samples of its tables, sorts none that its budget has no
+// room for, and gives one back for a request that needs the room.
+static void server_budget() {
+    const size_t n = 40000, order = n * sizeof(RangeRec) + (2 * kRangeBins + 4 + n) * sizeof(int);
+    count_bytes = order;
+    const Scan small = sector(24), large = sector(320);
+    const auto stat = [](bcsim_server* v, const char* key) {
+        double x = 0;
+        size_t k = 0;
+        CHK(bcsim_server_get_stats(v, key, &x, 1, &k));
+        return x;
+    };
+    for (bool room : {false, true}) {
+        bcsim_sim* s = simulator(64, n);
+        bcsim_server* v;
+        CHK(bcsim_server_create(&v));
+        CHK(bcsim_server_set_parameter(v, "memory_budget_bytes", "1000000000"));
+        CHK(bcsim_server_add_phantom(v, s, nullptr));
+        int gs, gl, L, S;
+        CHK(bcsim_server_add_geometry(v, 24, small.o.data(), small.d.data(), small.l.data(), small.len, &gs));
+        CHK(bcsim_server_add_geometry(v, 320, large.o.data(), large.d.data(), large.l.data(), large.len, &gl));
+        CHK(bcsim_server_get_output_shape(v, 0, gl, &L, &S));
+        const double resident = stat(v, "resident_bytes");
+        const auto frame = [&](int lines) { return lines * (S * 4.0 + S * 8.0 + 64) + 4096 * 16.0 + S * 8.0; };
+        const double budget = resident + (room ? frame(320) + 200000 : frame(24) + 0.5 * order);
+        char text[32];
+        snprintf(text, sizeof text, "%.0f", budget);
+        CHK(bcsim_server_set_parameter(v, "memory_budget_bytes", text));
+        std::vector<float> out((size_t)L * S * 2);
+        const auto serve = [&](int g) {
+            uint64_t id;
+            CHK(bcsim_server_submit(v, 0, g, 0.0f, out.data(), out.size() / 2, &id));
+            CHK(bcsim_server_wait(v, id, -1, nullptr, nullptr, nullptr));
+        };
+        mallocs = 0;
+        serve(gs);
+        serve(gs);
+        REQUIRE(mallocs == (room ? 1 : 0));
+        REQUIRE(stat(v, "used_bytes") >= resident + (room ? order : 0) && stat(v, "used_bytes") <= budget);
+        if (room) {
+            REQUIRE(budget - resident < frame(320) + order);
+            serve(gl);  // the order gives way
+            REQUIRE(stat(v, "used_bytes") <= budget && stat(v, "resident_bytes") == resident);
+            serve(gs);
+        }
+        CHK(bcsim_server_destroy(v));
+        CHK(bcsim_destroy(s));
+    }
+    bcsim_sim* s = simulator(64, n);
+    bcsim_server* v;
+    CHK(bcsim_server_create(&v));
+    CHK(bcsim_server_add_phantom(v, s, nullptr));
+    const double plain = stat(v, "resident_bytes");
+    CHK(set_table(s, 16));
+    CHK(bcsim_server_add_phantom(v, s, nullptr));
+    REQUIRE(stat(v, "resident_bytes") - plain == 16 * 24 * 24 * (8 * 4 + 4));
+    CHK(bcsim_server_destroy(v));
+    CHK(bcsim_destroy(s));
+}
+
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     const std::vector<std::pair<std::string, void (*)()>> all = {
-        {"table_failures", table_failures}, {"optional_buffers", optional_buffers}, {"crowds", crowds}, {"origins", origins}};
+        {"table_failures", table_failures}, {"optional_buffers", optional_buffers}, {"crowds", crowds}, {"origins", origins},
+        {"server_budget", server_budget}};
     for (auto& e : all)
         if (e.first == what) {
             e.second();
