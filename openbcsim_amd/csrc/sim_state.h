@@ -1952,27 +1952,29 @@ struct bcsim_sim {
     }
 
     // FFT pass radix of this frame's convolution: set by the user, tuned per
-    // (FFT length, bin type, line count class), or the default.
+    // (FFT length, bin type, kernel, line count class), or the default.
     int plan_radix(bool tune_now) {
         if (radix) return radix;
         if (!tune_now || lines.empty()) return kDefaultRadix;
+        const uint32_t counter = noise_counter;  // neither this nor trials advance the noise stream
+        ConvParams p = conv_params(nullptr);
+        noise_counter = counter;
+        p.radix = 8;
+        const bool constant = conv_fixed(p);  // what 8 stands for: a noisy or deeper folded frame's is another kernel
         char key[96];
-        std::snprintf(key, sizeof key, "conv/F%d/%s/L2^%d", fft_len, phase_delay ? "complex" : "real",
-                      ceil_log2((long long)lines.size()));
+        std::snprintf(key, sizeof key, "conv/F%d/%s/%s/L2^%d", fft_len, phase_delay ? "complex" : "real",
+                      constant ? "constant" : "any", ceil_log2((long long)lines.size()));
         int r = 0;
         if (TuneCache::get().find_radix(key, r)) return r;
         DevBuf scratch;  // trial output, freed after the trials
         scratch.ensure(lines.size() * (size_t)n_out * sizeof(float2));
-        const uint32_t counter = noise_counter;  // trials do not advance the noise stream
-        ConvParams p = conv_params(scratch.as<float2>());
-        noise_counter = counter;
+        p.iq = scratch.as<float2>();
         std::string trials;
         double best_ms = 0.0;
-        p.radix = 8;
         // Alone a small frame's time is latency, where radix 4 can come out ahead; the constant
         // lengths issue about half the instructions (48 lines of 2^12 samples alone 8.9 us
         // against 8.3, 24 such frames in one batch 15 against 40).
-        const int first = conv_fixed(p) ? 8 : 4;
+        const int first = constant ? 8 : 4;
         for (int cand = first; cand <= 8; cand += 4) {
             p.radix = cand;
             const double ms =

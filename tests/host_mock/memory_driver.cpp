@@ -369,11 +369,29 @@ static void server_budget() {
     CHK(bcsim_destroy(s));
 }
 
+// Tuned choices are kept for the kernels that they were tried with.
+static void tuned_radix() {
+    int fours = 0;
+    for (int lines : {9, 17, 33, 65, 129, 257, 513}) {
+        bcsim_sim *noisy = simulator(lines, 500), *plain = simulator(lines, 500);
+        CHK(bcsim_set_parameter(noisy, "noise_amplitude", "0.5"));
+        for (bcsim_sim* s : {noisy, plain}) {
+            CHK(bcsim_set_parameter(s, "autotune", "on"));
+            (void)ranged(s);
+        }
+        fours += plan(noisy).find("radix=4") != std::string::npos;  // (by random times)
+        REQUIRE(plan(plain).find("radix=8") != std::string::npos);
+        CHK(bcsim_destroy(noisy));
+        CHK(bcsim_destroy(plain));
+    }
+    REQUIRE(fours > 0);
+}
+
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     const std::vector<std::pair<std::string, void (*)()>> all = {
         {"table_failures", table_failures}, {"optional_buffers", optional_buffers}, {"crowds", crowds}, {"origins", origins},
-        {"server_budget", server_budget}};
+        {"server_budget", server_budget}, {"tuned_radix", tuned_radix}};
     for (auto& e : all)
         if (e.first == what) {
             e.second();
