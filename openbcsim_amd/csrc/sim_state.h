@@ -1831,11 +1831,13 @@ struct bcsim_sim {
     }
 
     std::string shape_class(const char* kind, int nchunks, bool fixed_ok) const {
+        // points of one origin run a kernel of their own, with bins of their own
+        const bool shared = arc && std::strcmp(kind, "spline") != 0 && shared_origin();
         char buf[160];
         std::snprintf(buf, sizeof buf, "tile/%s/%s/%s/bins-%s/%s/L2^%d/C2^%d/F%d", kind,
                       profile == kProfileLut ? "lut" : "gauss", phase_delay ? "complex" : "real",
                       !fixed_ok ? "float-only" : bin_mode == 1 ? "fixed" : bin_mode == 2 ? "float" : "auto",
-                      arc ? "arc" : "noarc", ceil_log2((long long)lines.size()), ceil_log2(nchunks), fft_len);
+                      shared ? "arc-shared" : arc ? "arc" : "noarc", ceil_log2((long long)lines.size()), ceil_log2(nchunks), fft_len);
         return buf;
     }
 

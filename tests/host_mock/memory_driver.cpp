@@ -387,11 +387,45 @@ static void tuned_radix() {
     REQUIRE(fours > 0);
 }
 
+static std::string tuned(bcsim_sim* s) {
+    static char b[1 << 20];
+    CHK(bcsim_get_parameter(s, "autotune_report", b, sizeof b));
+    return b;
+}
+static int count(const std::string& text, const char* word) {
+    int n = 0;
+    for (size_t at = text.find(word); at != std::string::npos; at = text.find(word, at + 1)) n++;
+    return n;
+}
+static Scan parallel(int n) {
+    Scan s = sector(n);
+    for (int k = 0; k < n; k++) {
+        s.o[3 * k] = -0.01f + 0.02f * k / (n - 1);
+        for (int a = 0; a < 3; a++) s.d[3 * k + a] = a == 2, s.l[3 * k + a] = a == 0;
+    }
+    return s;
+}
+// Lines of one origin and others run different kernels: each class is tried.
+static void tuned_shapes_by_origin() {
+    bcsim_sim* s = simulator(12, 5000);
+    CHK(bcsim_set_parameter(s, "autotune", "on"));
+    (void)ranged(s);
+    REQUIRE(count(tuned(s), "tile/fixed/") == 1);
+    set_scan(s, parallel(12));
+    (void)ranged(s);
+    REQUIRE(count(tuned(s), "tile/fixed/") == 2);
+    set_scan(s, sector(12, 0.01f));
+    (void)ranged(s);
+    REQUIRE(count(tuned(s), "tile/fixed/") == 2);
+    CHK(bcsim_destroy(s));
+}
+
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     const std::vector<std::pair<std::string, void (*)()>> all = {
         {"table_failures", table_failures}, {"optional_buffers", optional_buffers}, {"crowds", crowds}, {"origins", origins},
-        {"server_budget", server_budget}, {"tuned_radix", tuned_radix}};
+        {"server_budget", server_budget}, {"tuned_radix", tuned_radix},
+        {"tuned_shapes_by_origin", tuned_shapes_by_origin}};
     for (auto& e : all)
         if (e.first == what) {
             e.second();
