@@ -19,6 +19,7 @@ namespace bcsim_hip {
 struct TileTune {
     int windows = 0, lines = 0, block = 0, slices = 0;
     int bins = 0;  // LDS bin accumulation (BinMode)
+    bool order = false;  // range order was faster than any shape
 };
 
 // kBinsWide: double, where a tile is one line of a lookup table's frame (else as float).
@@ -28,9 +29,9 @@ inline const char* bin_name(int m) {
 }
 
 inline std::string describe(const TileTune& t) {
-    char buf[112];
-    std::snprintf(buf, sizeof buf, "lines=%d block=%d slices=%d windows=%d bins=%s", t.lines, t.block, t.slices,
-                  t.windows, bin_name(t.bins));
+    char buf[128];
+    std::snprintf(buf, sizeof buf, "%slines=%d block=%d slices=%d windows=%d bins=%s", t.order ? "range order, else " : "",
+                  t.lines, t.block, t.slices, t.windows, bin_name(t.bins));
     return buf;
 }
 

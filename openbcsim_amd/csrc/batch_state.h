@@ -245,7 +245,10 @@ struct bcsim_batch {
                 // one accumulation mode for jobs of a kind, whose launch they share (trials of like
                 // shapes differ by less than they scatter: 24 spline jobs in two launches 122 us,
                 // in one 106)
-                J.g = s->plan_tile(t, tune_now, false);
+                TileTune tuned;
+                if (tune_now) tuned = s->tuned_tile(t, RangeLaunch{});
+                tuned.bins = kBinsAuto;
+                J.g = s->plan_tile(t, tuned);
                 if (tile_lines > 0) {
                     TileTune tt = s->tune;
                     tt.lines = tile_lines;

@@ -1845,10 +1845,11 @@ struct bcsim_sim {
     // coordinate search from the heuristic shape (bin accumulation and radial
     // windows, then lines per tile, then total workgroups, then block size), each
     // candidate timed on this frame's data.
+    // order: the target's launch in range order, tried beside the shapes, or none.
     // Writes the bins: call before they are cleared for the frame.
-    TileTune tuned_tile(const ProjTarget& t) {
+    TileTune tuned_tile(const ProjTarget& t, const RangeLaunch& order) {
         const bool fixed_ok = t.c.amp_scale > 0.0f;
-        const std::string key = shape_class(t.kind, t.nchunks, fixed_ok);
+        const std::string key = shape_class(t.kind, t.nchunks, fixed_ok) + (order.recs ? "/order" : "");
         TileTune best;
         if (TuneCache::get().find_tile(key, best)) return best;
         float* bins = d_bins.as<float>();
@@ -1862,12 +1863,12 @@ struct bcsim_sim {
             TileLaunch cfg = tile_launch(t.nchunks, tt, spl, target_bins(t, tt, tt.bins));
             const int blocks = tile_blocks(cfg);
             const bool ordered = tile_order && blocks >= kMinOrderedBlocks && blocks <= kMaxOrderedTiles;
-            DevBuf order;
+            DevBuf work;
             if (ordered) {
-                order.ensure(2 * (size_t)blocks * sizeof(int));
-                hip_check(launch_fill_zero(order.as<float>(), 2 * (size_t)blocks, stream), "fill kernel");
-                cfg.work = order.as<int>();
-                cfg.order = order.as<int>() + blocks;
+                work.ensure(2 * (size_t)blocks * sizeof(int));
+                hip_check(launch_fill_zero(work.as<float>(), 2 * (size_t)blocks, stream), "fill kernel");
+                cfg.work = work.as<int>();
+                cfg.order = work.as<int>() + blocks;
             }
             const double ms = time_launches(
                 stream,
@@ -1930,6 +1931,16 @@ struct bcsim_sim {
             const double ms = cost(c);
             if (ms < best_ms) best = c, best_ms = ms;
         }
+        if (order.recs) {
+            TileLaunch cfg = tile_launch(t.nchunks, tune, spl, target_bins(t, tune));
+            cfg.range = order;
+            cfg.atomic = 0;
+            const double ms = time_launches(stream, [&] { launch_target(t, cfg, bins); }, 3, 2);
+            char b[32];
+            std::snprintf(b, sizeof b, " [order]=%.3f", ms);
+            trials += b;
+            if (ms < best_ms) best.order = true, best_ms = ms;
+        }
         char head[64];
         std::snprintf(head, sizeof head, "%.3f ms with ", best_ms);
         TuneCache::get().put_tile(key, best,
@@ -1937,20 +1948,29 @@ struct bcsim_sim {
         return best;
     }
 
-    // Launch shape for a target: shape fields set by the user win, then the
-    // tuned shape (when tuning is on), then the heuristic.
-    // tuned_bins: a trial's accumulation mode too (else target_bins' rule).
-    TileLaunch plan_tile(const ProjTarget& t, bool tune_now, bool tuned_bins = true) {
+    // Launch shape for a target: shape fields set by the user win, then `tuned` (a
+    // trial's), then the heuristic.
+    TileLaunch plan_tile(const ProjTarget& t, const TileTune& tuned = TileTune{}) const {
         TileTune eff = tune;
+        if (!eff.windows) eff.windows = tuned.windows;
+        if (!eff.lines) eff.lines = tuned.lines;
+        if (!eff.block) eff.block = tuned.block;
+        if (!eff.slices) eff.slices = tuned.slices;
+        return tile_launch(t.nchunks, eff, std::strcmp(t.kind, "spline") == 0, target_bins(t, eff, tuned.bins));
+    }
+
+    // A target's launch in a frame of its own: in range order where range_launch's rule says
+    // so (and, with tuning on, a trial does not say otherwise), else of the tuned shape.
+    TileLaunch plan_target(const ProjTarget& t, float* bins, bool tune_now, bool create) {
+        TileLaunch g = plan_tile(t);
+        const RangeLaunch order = range_launch(t, g, bins, create);
+        TileTune tuned;
         if (tune_now) {
-            const TileTune tt = tuned_tile(t);
-            if (!eff.windows) eff.windows = tt.windows;
-            if (!eff.lines) eff.lines = tt.lines;
-            if (!eff.block) eff.block = tt.block;
-            if (!eff.slices) eff.slices = tt.slices;
-            if (tuned_bins) eff.bins = tt.bins;
+            tuned = tuned_tile(t, order);
+            g = plan_tile(t, tuned);
         }
-        return tile_launch(t.nchunks, eff, std::strcmp(t.kind, "spline") == 0, target_bins(t, eff, eff.bins));
+        if (order.recs && (!tune_now || tuned.order)) g.range = order;
+        return g;
     }
 
     // FFT pass radix of this frame's convolution: set by the user, tuned per
@@ -2284,9 +2304,8 @@ struct bcsim_sim {
             if (direct_mode) {
                 direct_plans.push_back(proj_launch(t.n));
             } else {
-                plans.push_back(plan_tile(t, autotune && !fm));
-                TileLaunch& g = plans.back();
-                g.range = range_launch(t, g, bins, fm == nullptr);
+                plans.push_back(plan_target(t, bins, autotune && !fm, fm == nullptr));
+                const TileLaunch& g = plans.back();
                 last_plan += std::string(t.kind) + (t.ss.iboxes ? " (interval boxes)" : "") +
                              ": lines=" + std::to_string(g.tile_lines) +
                              " block=" + std::to_string(g.block) + " slices=" + std::to_string(g.slices) +

@@ -146,8 +146,9 @@ static bool ranged(bcsim_sim* s) {
     std::vector<float> out((size_t)L * S * 2);
     const int before = range_launches;
     CHK(bcsim_simulate_lines(s, out.data(), (size_t)L * S, &L, &S));
-    REQUIRE((plan(s).find("range order") != std::string::npos) == (range_launches > before));
-    return range_launches > before;
+    const bool r = plan(s).find("range order") != std::string::npos;
+    REQUIRE(!r || range_launches > before);  // (trials launch it too)
+    return r;
 }
 
 // A table whose samples or quads do not fit, or whose copies fail, leaves the profile
@@ -420,12 +421,28 @@ static void tuned_shapes_by_origin() {
     CHK(bcsim_destroy(s));
 }
 
+// With tuning on, range order is tried beside the shapes, and what was faster runs.
+static void tuned_order() {
+    int in_order = 0, shapes = 0;
+    for (int lines : {17, 33, 65, 129, 257}) {
+        bcsim_sim* s = simulator(lines, 8000);
+        CHK(bcsim_set_parameter(s, "autotune", "on"));
+        const bool r = ranged(s);  // by random times
+        REQUIRE(count(tuned(s), "[order]=") == in_order + shapes + 1);
+        REQUIRE(count(tuned(s), "ms with range order") == in_order + (r ? 1 : 0));
+        REQUIRE(ranged(s) == r && count(tuned(s), "[order]=") == in_order + shapes + 1);
+        (r ? in_order : shapes)++;
+        CHK(bcsim_destroy(s));
+    }
+    REQUIRE(shapes > 0);
+}
+
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     const std::vector<std::pair<std::string, void (*)()>> all = {
         {"table_failures", table_failures}, {"optional_buffers", optional_buffers}, {"crowds", crowds}, {"origins", origins},
         {"server_budget", server_budget}, {"tuned_radix", tuned_radix},
-        {"tuned_shapes_by_origin", tuned_shapes_by_origin}};
+        {"tuned_shapes_by_origin", tuned_shapes_by_origin}, {"tuned_order", tuned_order}};
     for (auto& e : all)
         if (e.first == what) {
             e.second();
