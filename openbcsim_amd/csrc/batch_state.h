@@ -242,30 +242,34 @@ struct bcsim_batch {
                 J.ss = t.ss;
                 J.boxes = t.boxes;
                 J.bins = s->d_bins.as<float>();
-                // one accumulation mode for jobs of a kind, whose launch they share (trials of like
-                // shapes differ by less than they scatter: 24 spline jobs in two launches 122 us,
-                // in one 106)
-                TileTune tuned;
-                if (tune_now) tuned = s->tuned_tile(t, RangeLaunch{});
-                tuned.bins = kBinsAuto;
-                J.g = s->plan_tile(t, tuned);
+                // One dataset, a Gaussian beam: in range order where a frame of its own would be
+                // (48 jobs, half of them of about 25k points on 48 lines: these 85 -> 46 us).  Its
+                // items are those of the plain shape, about one a line, whatever a trial of the tile
+                // kernel would find.  A table's staged cells would tie an item's waves to one window
+                // of one job; crowded points would need the launch of their parts.
+                if (targets.size() == 1 && !lut && tile_lines <= 0 && std::strcmp(t.kind, "fixed") == 0) {
+                    J.g = s->plan_tile(t);
+                    const RangeLaunch order = s->range_launch(t, J.g, J.bins, true);
+                    if (order.recs && !order.split) {
+                        J.g.range = order;
+                        orders.insert(orders.end(), s->order_refs.begin(), s->order_refs.end());
+                    }
+                    s->order_refs.clear();
+                }
                 if (tile_lines > 0) {
                     TileTune tt = s->tune;
                     tt.lines = tile_lines;
                     J.g = s->tile_launch(t.nchunks, tt, is_spline, s->target_bins(t, tt));
+                } else if (!J.g.range.recs) {
+                    // one accumulation mode for jobs of a kind, whose launch they share (trials of like
+                    // shapes differ by less than they scatter: 24 spline jobs in two launches 122 us,
+                    // in one 106), and shapes tried with it
+                    J.g = s->plan_tile(t, tune_now ? s->tuned_tile(t, RangeLaunch{}, true) : TileTune{});
                 }
                 J.g.block = 1024;
                 J.g.chunks = t.chunk_order;
                 J.g.chunk_dist = t.chunk_dist;
                 J.nchunks = t.nchunks;
-                // One dataset, a Gaussian beam: in range order where a frame of its own would be
-                // (48 jobs, half of them of about 25k points on 48 lines: these 85 -> 46 us).
-                // A table's staged cells would tie an item's waves to one window of one job.
-                if (targets.size() == 1 && !lut && tile_lines <= 0 && std::strcmp(t.kind, "fixed") == 0)
-                    J.g.range = s->range_launch(t, J.g, J.bins, true);
-                if (J.g.range.split) J.g.range = RangeLaunch{};  // crowded points: no parts in a batch
-                if (J.g.range.recs) orders.insert(orders.end(), s->order_refs.begin(), s->order_refs.end());
-                s->order_refs.clear();
                 J.flags = (s->arc ? kJobArc : 0) | (cplx ? kJobPhase : 0) | (lut ? kJobLut : 0) |
                           (is_spline ? kJobSpline : 0) | (shared && !is_spline ? kJobShared : 0) |
                           (J.g.fixed ? kJobFixed : 0) | (J.g.wide ? kJobWide : 0) |

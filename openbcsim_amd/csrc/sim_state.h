@@ -1834,7 +1834,7 @@ struct bcsim_sim {
         // points of one origin run a kernel of their own, with bins of their own
         const bool shared = arc && std::strcmp(kind, "spline") != 0 && shared_origin();
         char buf[160];
-        std::snprintf(buf, sizeof buf, "tile/%s/%s/%s/bins-%s/%s/L2^%d/C2^%d/F%d", kind,
+        std::snprintf(buf, sizeof buf, "%s/%s/%s/bins-%s/%s/L2^%d/C2^%d/F%d", kind,
                       profile == kProfileLut ? "lut" : "gauss", phase_delay ? "complex" : "real",
                       !fixed_ok ? "float-only" : bin_mode == 1 ? "fixed" : bin_mode == 2 ? "float" : "auto",
                       shared ? "arc-shared" : arc ? "arc" : "noarc", ceil_log2((long long)lines.size()), ceil_log2(nchunks), fft_len);
@@ -1846,10 +1846,12 @@ struct bcsim_sim {
     // windows, then lines per tile, then total workgroups, then block size), each
     // candidate timed on this frame's data.
     // order: the target's launch in range order, tried beside the shapes, or none.
+    // one_mode: shapes for target_bins' default accumulation alone.
     // Writes the bins: call before they are cleared for the frame.
-    TileTune tuned_tile(const ProjTarget& t, const RangeLaunch& order) {
+    TileTune tuned_tile(const ProjTarget& t, const RangeLaunch& order, bool one_mode = false) {
         const bool fixed_ok = t.c.amp_scale > 0.0f;
-        const std::string key = shape_class(t.kind, t.nchunks, fixed_ok) + (order.recs ? "/order" : "");
+        const std::string key = (one_mode ? "tile=" : "tile/") + shape_class(t.kind, t.nchunks, fixed_ok) +
+                                (order.recs ? "/order" : "");
         TileTune best;
         if (TuneCache::get().find_tile(key, best)) return best;
         float* bins = d_bins.as<float>();
@@ -1893,7 +1895,7 @@ struct bcsim_sim {
         best.bins = target_bins(t, best);
         double best_ms = cost(best);
         std::vector<int> modes{best.bins};
-        if (!bin_mode)
+        if (!bin_mode && !one_mode)
             for (int b : {kBinsFixed, kBinsFloat})
                 if (b != best.bins && (b != kBinsFixed || (fixed_ok && best.bins != kBinsWide))) modes.push_back(b);
         for (int b : modes) {

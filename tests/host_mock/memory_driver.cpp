@@ -437,12 +437,46 @@ static void tuned_order() {
     REQUIRE(shapes > 0);
 }
 
+// A batch tries shapes only for jobs that run them, with the bins that they will have.
+static void batch_shapes() {
+    std::vector<bcsim_sim*> sims;
+    bcsim_batch* b;
+    CHK(bcsim_batch_create(&b));
+    for (int lines : {20, 40, 80}) {
+        sims.push_back(simulator(lines, 8000));  // range order
+        sims.push_back(simulator(lines, 8000));
+        set_scan(sims.back(), parallel(lines));
+        sims.push_back(simulator(lines, 8000));
+        set_scan(sims.back(), parallel(lines));
+        CHK(set_table(sims.back(), 16));
+    }
+    for (bcsim_sim* s : sims) CHK(bcsim_batch_add(b, s, nullptr));
+    size_t total = 0;
+    int jobs = 0;
+    CHK(bcsim_batch_get_layout(b, &total, &jobs, nullptr, nullptr, nullptr, 0));
+    void* out = nullptr;
+    REQUIRE(hipMalloc(&out, total * 8) == hipSuccess);
+    CHK(bcsim_batch_simulate_device(b, out, total));
+    CHK(bcsim_batch_synchronize(b));
+    const std::string report = tuned(sims[0]);
+    REQUIRE(count(report, "tile=fixed/") == 6 && count(report, "tile/") == 0 && count(report, "arc-shared") == 0);
+    for (size_t at = 0; at < report.size(); at = report.find('\n', at) + 1) {
+        const std::string line = report.substr(at, report.find('\n', at) - at);
+        if (line.find("tile=") != 0) continue;
+        REQUIRE(count(line, line.find("/gauss/") != std::string::npos ? ",float]=" : ",fixed]=") == 0);
+    }
+    CHK(bcsim_batch_destroy(b));
+    for (bcsim_sim* s : sims) CHK(bcsim_destroy(s));
+    hipFree(out);
+}
+
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     const std::vector<std::pair<std::string, void (*)()>> all = {
         {"table_failures", table_failures}, {"optional_buffers", optional_buffers}, {"crowds", crowds}, {"origins", origins},
         {"server_budget", server_budget}, {"tuned_radix", tuned_radix},
-        {"tuned_shapes_by_origin", tuned_shapes_by_origin}, {"tuned_order", tuned_order}};
+        {"tuned_shapes_by_origin", tuned_shapes_by_origin}, {"tuned_order", tuned_order},
+        {"batch_shapes", batch_shapes}};
     for (auto& e : all)
         if (e.first == what) {
             e.second();
