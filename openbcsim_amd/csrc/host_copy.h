@@ -11,10 +11,10 @@
 namespace bcsim_hip {
 
 // memcpy split over a few threads for large copies (page faults of a fresh
-// destination are taken in parallel too).
-inline void parallel_copy(void* dst, const void* src, size_t bytes) {
+// destination are taken in parallel too).  whole: the copy that this is a piece of.
+inline void parallel_copy(void* dst, const void* src, size_t bytes, size_t whole = 0) {
     constexpr size_t kChunk = (size_t)4 << 20;
-    const int parts = (int)std::min<size_t>(8, bytes / kChunk);
+    const int parts = (int)std::min<size_t>(8, std::max(bytes, whole) / kChunk);
     if (parts <= 1) {
         std::memcpy(dst, src, bytes);
         return;

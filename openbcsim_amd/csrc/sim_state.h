@@ -2524,11 +2524,13 @@ struct bcsim_sim {
     }
 
     // Frames copied into pageable host memory pass through pinned pieces: the DMA of the
-    // next pieces runs while the host moves one into the caller's buffer (the runtime's own
-    // path to pageable memory takes 0.33 ms for 1 MB and 0.18 for 3, this 0.06 and 0.13).
-    // Up to kStagePiece bytes are one pinned buffer in up to four pieces; more, two buffers
-    // of kStagePiece by turns, whose pieces several host threads move.
-    static constexpr size_t kStagedCopyMin = (size_t)128 << 10;
+    // next pieces runs while the host moves one into the caller's buffer.  Up to kStagePiece
+    // bytes are one pinned buffer in up to four pieces; more, two buffers of kStagePiece by
+    // turns.  Whole frames of 1 / 1.5 / 2 / 4 / 8 MB into memory used before: by the runtime's
+    // own path to pageable memory 82 / 119 / 142 / 261 / 482 us, by pieces 90 / 119 / 118 / 205 /
+    // 396; of 24 MB, one piece moved by several threads 882, four by one thread each 994, three by
+    // several 701 (into fresh memory 1259, 2033, 1148).
+    static constexpr size_t kStagedCopyMin = (size_t)1792 << 10;
     static constexpr size_t kStagePiece = (size_t)32 << 20;
     static constexpr int kStagePieces = 4;
     void* stage[2] = {nullptr, nullptr};
@@ -2558,8 +2560,10 @@ struct bcsim_sim {
         for (auto& e : stage_ev)
             if (!e) hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
         const bool small = bytes <= kStagePiece;
-        // pieces of about 768 KiB in one buffer, or whole buffers by turns
-        const size_t count = std::min<size_t>(kStagePieces, std::max<size_t>(1, bytes / ((size_t)768 << 10)));
+        // pieces of about 768 KiB in one buffer, from 8 MiB on (where several threads move each) of
+        // that, or whole buffers by turns
+        const size_t about = bytes < (size_t)8 << 20 ? (size_t)768 << 10 : (size_t)8 << 20;
+        const size_t count = std::min<size_t>(kStagePieces, std::max<size_t>(1, bytes / about));
         const size_t piece = small ? ((bytes + count - 1) / count + 255) & ~(size_t)255 : kStagePiece;
         const size_t pieces = (bytes + piece - 1) / piece;
         const int ahead = small ? (int)pieces : 2;  // pieces that may be under way
@@ -2577,7 +2581,7 @@ struct bcsim_sim {
             for (; issued < pieces && issued < c + ahead; issued++) issue(issued);
             if (issued == pieces) t.stop();
             hip_check(hipEventSynchronize(stage_ev[c % ahead]), "hipEventSynchronize");
-            parallel_copy((char*)dst + c * piece, staged(c), piece_len(c));
+            parallel_copy((char*)dst + c * piece, staged(c), piece_len(c), small ? bytes : 0);
         }
         hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
     }

@@ -72,7 +72,8 @@ def test_tuned_shapes_match_the_default():
 @pytest.mark.parametrize("lines,length,decimation", [(8, 0.028, 1), (8, 0.12, 1), (48, 0.12, 1), (340, 0.12, 1),
                                                      (640, 0.13, 1)])
 def test_host_copies(lines, length, decimation):
-    """0.1 MB: the runtime's copy; 0.5 MB: one pinned piece; 3 MB: four; 21 MB: four; 43 MB: two buffers by turns."""
+    """0.1 and 0.5 MB: the runtime's copy; 3 MB: pinned pieces, moved by one thread; 21 MB: by several; 43 MB: two
+    buffers by turns."""
     from openbcsim_amd.hip_rt import DeviceBuffer
     wl = W.fixed_sector_2d(3000, lines, seed=47, line_length=length, decimation=decimation)
     s = sim(wl, tile_order="off")
