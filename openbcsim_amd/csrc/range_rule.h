@@ -64,26 +64,33 @@ inline RangeCrowd range_crowd(const PointSample& s, int lo, int count, const flo
     const int finest = s.n > 512 ? 0 : 2;  // few points: cells of four blocks tell as much
     const int width = block << finest;
     int n = (num_rf + width - 1) / width;
-    std::vector<int> cell(n + 1, 0);
-    int seen = 0;
-    for (size_t i = 0; i < s.n; i++) {
-        float x = 0.f, y = 0.f, z = 0.f;
+    std::vector<int> cell(n + 1, 0);  // the last one takes what the scan does not see
+    const float to_cell = 1.0f / (float)width, none = (float)n;
+    // a few points at a time, in loops without branches
+    constexpr size_t kStep = 128;
+    float x[kStep], y[kStep], z[kStep], d[kStep], at[kStep];
+    for (size_t i0 = 0; i0 < s.n; i0 += kStep) {
+        const size_t m = std::min(kStep, s.n - i0);
+        for (size_t i = 0; i < m; i++) x[i] = -ox, y[i] = -oy, z[i] = -oz;
         for (int q = 0; q < count; q++) {
-            const size_t at = (size_t)(lo + q) * s.n + i;
-            x += s.x[at] * basis[q], y += s.y[at] * basis[q], z += s.z[at] * basis[q];
+            const size_t from = (size_t)(lo + q) * s.n + i0;
+            const float *px = &s.x[from], *py = &s.y[from], *pz = &s.z[from], w = basis[q];
+            for (size_t i = 0; i < m; i++) x[i] += px[i] * w, y[i] += py[i] * w, z[i] += pz[i] * w;
         }
-        x -= ox, y -= oy, z -= oz;
-        const float d = std::sqrt(x * x + y * y + z * z);
-        const float r = x * cone.r[0] + y * cone.r[1] + z * cone.r[2];
-        const float l = x * cone.l[0] + y * cone.l[1] + z * cone.l[2];
-        const float e = x * cone.e[0] + y * cone.e[1] + z * cone.e[2];
-        const float bin = d * bins_per_metre + 0.5f;
-        if (!(r > -d * cone.r[3] && std::fabs(l) < d * cone.l[3] + cone.beam_l &&
-              std::fabs(e) < d * cone.e[3] + cone.beam_e && bin < (float)num_rf))
-            continue;
-        cell[(int)bin / width]++;
-        seen++;
+        for (size_t i = 0; i < m; i++) d[i] = std::sqrt(x[i] * x[i] + y[i] * y[i] + z[i] * z[i]);
+        for (size_t i = 0; i < m; i++) {
+            const float r = x[i] * cone.r[0] + y[i] * cone.r[1] + z[i] * cone.r[2];
+            const float l = x[i] * cone.l[0] + y[i] * cone.l[1] + z[i] * cone.l[2];
+            const float e = x[i] * cone.e[0] + y[i] * cone.e[1] + z[i] * cone.e[2];
+            const float bin = d[i] * bins_per_metre + 0.5f;
+            const bool in = (r > -d[i] * cone.r[3]) & (std::fabs(l) < d[i] * cone.l[3] + cone.beam_l) &
+                            (std::fabs(e) < d[i] * cone.e[3] + cone.beam_e) & (bin < (float)num_rf);
+            at[i] = in ? bin * to_cell : none;
+        }
+        for (size_t i = 0; i < m; i++) cell[std::min((int)at[i], n)]++;
     }
+    const int seen = (int)s.n - cell[n];
+    cell[n] = 0;
     out.seen = seen * s.each;
     for (int k = finest; k < RangeCrowd::kLevels; k++) {
         int most = 0;

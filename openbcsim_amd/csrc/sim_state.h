@@ -254,6 +254,7 @@ struct RangeOrders {
     // them (other simulators may read them next, on streams of their own); null: only
     // an order built earlier.  Without memory for another copy there is no order.
     // account: where a new order's bytes are counted, or null.
+    // may_have() said yes.
     template <class Sort>
     Ref get(const Key& key, bool any_phase, size_t n, const Sort* sort,
             const std::shared_ptr<std::atomic<size_t>>& account = nullptr) {
@@ -280,6 +281,21 @@ struct RangeOrders {
         o->account = account;
         orders.push_back(o);
         return o;
+    }
+
+    // Is there an order of `key`, or (create) may there be one now?  What is refused is remembered.
+    bool may_have(const Key& key, bool any_phase, bool create) {
+        std::lock_guard<std::mutex> g(mu);
+        asked++;
+        for (auto& o : orders)
+            if (o->key.serves(key, any_phase)) return true;
+        if (!create) return false;
+        if (orders.size() < kMaxOrders) return true;
+        for (const Refusal& r : refusals)
+            if (r.key.serves(key, any_phase)) return true;
+        if (refusals.size() >= kMaxOrders) refusals.erase(refusals.begin());
+        refusals.push_back({key, asked});
+        return false;
     }
 
     bool has(const Key& key, bool any_phase) {
@@ -312,11 +328,7 @@ struct RangeOrders {
     bool replace(const Key& key, bool any_phase) {
         const auto known = std::find_if(refusals.begin(), refusals.end(),
                                         [&](const Refusal& r) { return r.key.serves(key, any_phase); });
-        if (known == refusals.end()) {
-            if (refusals.size() >= kMaxOrders) refusals.erase(refusals.begin());
-            refusals.push_back({key, asked});
-            return false;
-        }
+        if (known == refusals.end()) return false;
         auto oldest = orders.end();
         for (auto o = orders.begin(); o != orders.end(); ++o)
             if (o->use_count() == 1 && (*o)->used < known->at && (oldest == orders.end() || (*o)->used < (*oldest)->used))
@@ -645,6 +657,7 @@ struct bcsim_sim {
     std::shared_ptr<DevBuf> roots;  // conv_roots of roots_shape, or null
     ConvShape roots_shape{0, false, 0};
     DevBuf d_patches;  // RangePatch[n_patches] of the lines' directions
+    std::vector<RangePatch> patches;  // the same
     int n_patches = 0;
     float patch_dl = 0.0f, patch_de = 0.0f;  // means of their dl and de
     ScanCone cone{};                         // of all lines (its beam is set per frame)
@@ -2018,7 +2031,7 @@ struct bcsim_sim {
     void build_patches() {
         std::vector<int> order(lines.size());
         for (size_t i = 0; i < order.size(); i++) order[i] = (int)i;
-        std::vector<RangePatch> patches;
+        patches.clear();
         // mean of an axis of the lines [first, last), and how far theirs lie from it (rounded up)
         const auto bound = [&](const int* first, const int* last, float LineGeom::*x, float* axis) {
             const auto at = [&](int i) { return &(lines[i].*x); };
@@ -2073,10 +2086,11 @@ struct bcsim_sim {
             patches.push_back(q);
         };
         split(split, order.data(), order.data() + order.size());
-        quiesce();
+        // prepare() has waited for frames that read the old ones; the host does not wait for the copy
         d_patches.ensure(patches.size() * sizeof(RangePatch));
-        hip_check(hipMemcpy(d_patches.p, patches.data(), patches.size() * sizeof(RangePatch), hipMemcpyHostToDevice),
-                  "hipMemcpy");
+        hip_check(hipMemcpyAsync(d_patches.p, patches.data(), patches.size() * sizeof(RangePatch), hipMemcpyHostToDevice,
+                                 stream),
+                  "hipMemcpyAsync");
         n_patches = (int)patches.size();
         bound(order.data(), order.data() + order.size(), &LineGeom::rx, cone.r);
         bound(order.data(), order.data() + order.size(), &LineGeom::lx, cone.l);
@@ -2135,6 +2149,8 @@ struct bcsim_sim {
             if (!create || !where_it_fits([&] { build_patches(); })) return R;
         }
         R.n_patches = n_patches;
+        const RangeOrders::Key key{lines[0].ox, lines[0].oy, lines[0].oz, t.c.phase_per_sample, t.c.bin_scale, t.c.bin_denom};
+        if (!rendered && !t.fixed->by_range.may_have(key, !phase_delay, create)) return R;
         // A patch's waves visit every point that reaches any of its lines.  Where few of its 64
         // lanes have a line in reach of a point and each bin has many points, the tile kernel's
         // visits (a line, 64 points of a chunk) are fewer: 38 lines over 70 degrees against 405k
@@ -2245,7 +2261,6 @@ struct bcsim_sim {
             R.recs = t.scan->recs.as<RangeRec>();
             return R;
         }
-        const RangeOrders::Key key{lines[0].ox, lines[0].oy, lines[0].oz, t.c.phase_per_sample, t.c.bin_scale, t.c.bin_denom};
         const auto sort = [&](RangeRec* recs, int* start, int* scratch) {
             TileLaunch g = shape;
             g.range = R;
