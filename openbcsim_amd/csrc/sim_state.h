@@ -2219,7 +2219,7 @@ struct bcsim_sim {
             longest = frac * std::max(0.2 * run, (0.045 + 12.8 * R.group / R.block) * at.heaviest(R.window_bins, kRangeBlock));
             tile = 8.5 + 7.0 * few + 2.7 * mega_bins + (phase_delay ? 8.1 : 4.6) * pairs * reach + 0.14 * pairs;
         } else {
-            base = 5.5 + 2.3 * mega_bins + 6.7 * visits;
+            base = 5.5 + (phase_delay ? 2.0 : 3.6) * mega_bins + 6.7 * visits;  // (its stores are 32 or 16 bytes)
             longest = frac * 0.15 * run;
             tile = 8.4 + 4.7 * few + 2.6 * mega_bins + (phase_delay ? 3.8 : 2.4) * pairs * reach + 0.15 * pairs;
         }
@@ -2239,8 +2239,9 @@ struct bcsim_sim {
         // 2.9, which took 4.3 and 134 times as long before this rule and the parts.
         if (base + std::min(parts, longest) > 1.1 * tile + 60.0) return RangeLaunch{};
         // Few points do not earn the staging of a large table (1000 points, 48 lines, 256 x 64 x 64
-        // samples 21 us a frame, by the tile kernel 17; 10k points 22.9 and 24.6).
-        if (lut_profile && at.seen < 4000.0 && base > tile) return RangeLaunch{};
+        // samples 21 us a frame, by the tile kernel 17; 10k points 22.9 and 24.6), nor many lines'
+        // bins in stores of four (200 points, 2500 lines of 9740 samples: projection 94 and 65).
+        if (at.seen < 4000.0 && base > (lut_profile ? 1.0 : 1.15) * tile) return RangeLaunch{};
         if (rendered && R.split) return RangeLaunch{};  // their sort, too, counts a bin's points one by one
         if (rendered) {  // other points every frame: sorted by each, into this simulator's buffers
             const bool fits = where_it_fits([&] {
