@@ -248,6 +248,15 @@ static void crowds() {
         }
         CHK(bcsim_destroy(s));
     }
+    // few points on many long lines, whose bins are the frame
+    for (size_t n : {size_t(200), size_t(60000)}) {
+        bcsim_sim* s = simulator(2500, n);
+        Scan deep = sector(2500);
+        deep.len = 0.15f;
+        set_scan(s, deep);
+        REQUIRE(ranged(s) == (n > 200));
+        CHK(bcsim_destroy(s));
+    }
 }
 
 // Orders of a dataset: four, the one longest unused giving way to an origin that stays.

@@ -149,3 +149,27 @@ def test_batch_jobs_with_crowds_run_the_tile_kernel():
             assert np.abs(b).max() > 0 and rel_l2(a, b) < 1e-6
     for x in (batch, *sims):
         x.close()
+
+
+def test_steering_without_waiting():
+    """Frames of other directions enqueued one after another: each has its own patches."""
+    from openbcsim_amd.hip_rt import DeviceBuffer
+    from openbcsim_amd.pyrfsim import RfSimulator
+    wl = W.fixed_sector_2d(20000, 96, seed=9, line_length=0.05, phase_delay=True)
+    g = RfSimulator("gpu")
+    wl.apply(g)
+    L, S = g.output_shape()
+    outs, want = [], []
+    for k in range(6):
+        o, d, l, t, length = W.sector_scan(96, 0.6 + 0.12 * k, 0.05)
+        g.set_scan_sequence(o, d, length, l, t)
+        outs.append(DeviceBuffer(L * S * 8))
+        g.simulate_lines_device(outs[-1].address, L * S)
+        assert "range order" in g.get_parameter("launch_plan")
+    g.synchronize()
+    for k, out in enumerate(outs):
+        wl.scan = W.sector_scan(96, 0.6 + 0.12 * k, 0.05)
+        iq = np.empty((L, S), np.complex64)
+        out.to_host(iq)
+        assert rel_l2(iq, frame(wl, tile_lines="1")[0]) < 1e-6, k
+    g.close()
