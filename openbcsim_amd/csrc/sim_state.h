@@ -2223,21 +2223,28 @@ struct bcsim_sim {
             longest = frac * 0.15 * run;
             tile = 8.4 + 4.7 * few + 2.6 * mega_bins + (phase_delay ? 3.8 : 2.4) * pairs * reach + 0.15 * pairs;
         }
-        const double limit = 0.5 * base + 8.0;  // a walk this long hides behind the rest
-        double parts = INFINITY;
-        if (longest > limit && !(lut_profile && R.window_bins < kRangeBlock) &&
-            range_part_lds_bytes(phase_delay) + (lut_profile ? range_lds_bytes(R) : 0) <= (size_t)kLdsBytes - 512) {
-            const int waves = std::max(1, 8 / std::min(n_patches, kRangePartPatches));  // of a patch
-            const double walk = frac * std::max(std::min(512.0, block), block / kRangeParts) / waves;
-            const double items = std::ceil((double)n_patches / kRangePartPatches) * (at.seen / 512.0 + 2.0 * at.seen / block);
-            parts = limit + 6.0 + std::ceil(items / 512.0) * (lut_profile ? 20.0 + 0.2 * walk : 6.0 + 0.15 * walk);
-            if (parts < longest) R.split = (int)std::min(1e9, std::max(64.0, block * limit / longest));
+        // Only where a block of bins has six times its share: uniform points in a cone have two to
+        // three and a half times (in draws of these ranges, up to five among 15k points), their walks
+        // hide behind one another better than the estimate says, and parts gained on 24 such frames
+        // (350 -> 146 us) but lost on 7 (368 -> 472), the tile kernel likewise (98 -> 67, 163 -> 189).
+        if (block * num_rf > 6.0 * kRangeBlock * at.seen) {
+            const double limit = 0.5 * base + 8.0;  // a walk this long hides behind the rest
+            double parts = INFINITY;
+            if (longest > limit && !(lut_profile && R.window_bins < kRangeBlock) &&
+                range_part_lds_bytes(phase_delay) + (lut_profile ? range_lds_bytes(R) : 0) <= (size_t)kLdsBytes - 512) {
+                const int waves = std::max(1, 8 / std::min(n_patches, kRangePartPatches));  // of a patch
+                const double walk = frac * std::max(std::min(512.0, block), block / kRangeParts) / waves;
+                const double items =
+                    std::ceil((double)n_patches / kRangePartPatches) * (at.seen / 512.0 + 2.0 * at.seen / block);
+                parts = limit + 6.0 +
+                        std::ceil(items / 512.0) * (lut_profile ? 20.0 + 0.2 * walk : 6.0 + 0.15 * walk);
+                if (parts < longest) R.split = (int)std::min(1e9, std::max(64.0, block * limit / longest));
+            }
+            // The tile kernel where it clearly saves time: alone, walks are the frame's latency, but
+            // among other frames the chip works on those meanwhile.  Frames as above, crowded: 1.0
+            // to 2.9 of the tile kernel's time, 4.3 and 134 without this rule and the parts.
+            if (base + std::min(parts, longest) > 1.1 * tile + 60.0) return RangeLaunch{};
         }
-        // The tile kernel where it clearly saves time: alone, walks are the frame's latency, but among
-        // other frames the chip works on those meanwhile.  700 frames as above: uniform points
-        // 0.65 of the tile kernel's time (median) to 1.26 (95th percentile), crowded ones 1.0 to
-        // 2.9, which took 4.3 and 134 times as long before this rule and the parts.
-        if (base + std::min(parts, longest) > 1.1 * tile + 60.0) return RangeLaunch{};
         // Few points do not earn the staging of a large table (1000 points, 48 lines, 256 x 64 x 64
         // samples 21 us a frame, by the tile kernel 17; 10k points 22.9 and 24.6), nor many lines'
         // bins in stores of four (200 points, 2500 lines of 9740 samples: projection 94 and 65).

@@ -257,6 +257,24 @@ static void crowds() {
         REQUIRE(ranged(s) == (n > 200));
         CHK(bcsim_destroy(s));
     }
+    // many points on short lines, evenly over the sector's area: nothing crowds
+    for (int lines : {40, 400}) {
+        std::mt19937 rng(5);
+        std::uniform_real_distribution<float> u(0, 1);
+        std::vector<float> p;
+        for (int i = 0; i < 400000; i++) {
+            const float r = 0.025f * sqrtf(u(rng)), a = 1.2f * u(rng) - 0.6f;
+            p.insert(p.end(), {r * sinf(a), 0.01f * (u(rng) - 0.5f) * r, r * cosf(a), 1.0f});
+        }
+        bcsim_sim* s = simulator(lines, 0);
+        CHK(bcsim_add_fixed_scatterers(s, p.data(), p.size() / 4));
+        CHK(set_table(s, 24));
+        Scan shallow = sector(lines);
+        shallow.len = 0.025f;
+        set_scan(s, shallow);
+        REQUIRE(ranged(s) && plan(s).find("in parts") == std::string::npos);
+        CHK(bcsim_destroy(s));
+    }
 }
 
 // Orders of a dataset: four, the one longest unused giving way to an origin that stays.
