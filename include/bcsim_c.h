@@ -90,7 +90,10 @@ BCSIM_API bcsim_status bcsim_destroy(bcsim_sim* sim);
  * fewer than about 2048 lines).  With auto and no
  * tile_* shape set, arc projection of points onto lines of one origin runs in range
  * order instead of the tile kernel (points sorted by bin; register sums, double for
- * the Gaussian and float for a LUT), which launch_plan reports.  Datasets whose
+ * the Gaussian and float for a LUT), which launch_plan reports.  The order of a bin's points
+ * there is that of one sort, which another simulator's need not equal in the last
+ * bits; tile_slices 1 keeps the tile kernel, whose fixed-point bins are the same
+ * bits every time.  Datasets whose
  * amplitudes the grid cannot resolve (a non-finite amplitude, or a dynamic
  * range beyond ~2^39/n) use float bins whatever the setting.
  * Read-only keys of bcsim_get_parameter: launch_plan (shapes of the last frame)

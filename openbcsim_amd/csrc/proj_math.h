@@ -14,7 +14,9 @@ constexpr float kExpMinusMax = 80.0f;  // largest argument of exp_minus
 // Correctly rounded square root of a squared distance: the hardware root (within an
 // ulp) and the neighbour whose rounding interval holds x.  Residuals below 2^-96
 // (distances below 4e-15 m, bin 0 whatever their last bit) may be an ulp off; the
-// compiler's form rescales those, at twice the instructions.
+// compiler's form rescales those, at twice the instructions.  The steps are those of the AMD
+// compiler's own expansion of sqrtf, without its range handling (as the assembly of this
+// file's kernels shows it).
 __device__ __forceinline__ float sqrt_distance(float x) {
     const float s = __builtin_amdgcn_sqrtf(x);
     const float dn = __int_as_float(__float_as_int(s) - 1), up = __int_as_float(__float_as_int(s) + 1);
@@ -25,7 +27,8 @@ __device__ __forceinline__ float sqrt_distance(float x) {
 // exp(-x) for 0 <= x <= 80, where it neither under- nor overflows: 2^y, y = -x log2(e)
 // kept as a whole number n, a remainder and the rounding error of y, scaled by adding n
 // to the exponent: expf without its range checks, with the same error (8.2e-8 at most,
-// 2.6e-8 rms over [0, 80]).
+// 2.6e-8 rms over [0, 80]).  The split of log2(e) and the steps are the published expansion
+// that the AMD compiler gives expf, as the assembly of this file's kernels shows it.
 __device__ __forceinline__ float exp_minus(float x) {
     constexpr float c = -1.44269502f, c_lo = -1.92596303e-8f;  // -log2(e)
     const float y = x * c;

@@ -23,9 +23,11 @@
 //             radial difference: the eight corners of a lookup are four LDS reads.
 //
 // What bounds it: VALU issue.  A (point, patch) visit is about 50 instructions for 64
-// lines with a table and 30 with a Gaussian, at about 4.4 cycles a wave instruction
-// (1M points, 4096 lines, table 256 x 64 x 64: 7.3M visits, 46 % of the lanes' lines in
-// reach; the VALU busy for 0.95 of the kernel).  The tile kernel waits on the table
+// lines with a table and 30 with a Gaussian.  1M points, 4096 lines, table 256 x 64 x 64:
+// 7.3M visits, 46 % of the lanes' lines in reach, 448.8M wave instructions in 1.71M cycles on
+// 1024 SIMDs, one in 3.9 cycles, 0.69 of the rate at which fused multiply-adds issue on this
+// card (LDS waits are few).  A Gaussian sector (509 lines x 333k points), whose 7680 waves end
+// unevenly: one in 6.1 cycles, 0.43.  The tile kernel waits on the table
 // gathers' cache lines (one L1 miss a pair) and on float LDS atomics (a lane in three
 // cycles) instead.  Frame times, tile kernel -> range order, frames of three simulators
 // in flight with one convolution kernel: that volume 1.91 -> 0.83 ms (with that of
