@@ -46,6 +46,14 @@ inline void hip_check(hipError_t e, const char* what) {
     }
 }
 
+// Is a graph being captured on s?  (weak: the runtime may have no such query, as that of the host
+// tests)
+#pragma weak hipStreamIsCapturing
+inline bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing && hipStreamIsCapturing(s, &status) == hipSuccess && status != hipStreamCaptureStatusNone;
+}
+
 // Runs f, which allocates what a frame can do without; false without memory for it.
 template <typename F>
 bool where_it_fits(F&& f) {
@@ -214,7 +222,8 @@ struct ChunkOrders {
 // demodulation phase.  At most kMaxOrders; a further origin runs the tile kernel, and takes
 // the place of the order longest unused once it comes again and that one has not been used
 // in between: a scan that stays where it went gets its order, one that wanders, or more
-// scans by turns than there are orders, does not sort for every frame.
+// scans by turns than there are orders, does not sort for every frame.  What a frame under
+// graph capture uses stays as long as the dataset.
 struct RangeOrders {
     struct Key {
         float ox, oy, oz, phase;
@@ -231,6 +240,7 @@ struct RangeOrders {
         RangeRec* recs;
         int* start;
         uint64_t used;  // get()'s count when it was last asked for
+        mutable std::atomic<bool> kept{false};  // a captured frame names it: it stays with the dataset
         std::shared_ptr<std::atomic<size_t>> account;  // a server's, whose bytes these are (or null)
         ~Order() {
             if (account) *account -= mem.bytes;
@@ -310,18 +320,25 @@ struct RangeOrders {
         std::lock_guard<std::mutex> g(mu);
         auto oldest = orders.end();
         for (auto o = orders.begin(); o != orders.end(); ++o)
-            if (o->use_count() == 1 && (*o)->account == account && (oldest == orders.end() || (*o)->used < (*oldest)->used))
+            if (free(*o) && (*o)->account == account && (oldest == orders.end() || (*o)->used < (*oldest)->used))
                 oldest = o;
-        if (oldest == orders.end()) return false;
-        release(oldest);
-        return true;
+        return release(oldest);
     }
 
   private:
-    void release(std::vector<std::shared_ptr<Order>>::iterator o) {
+    static bool free(const std::shared_ptr<Order>& o) {
+        if (o.use_count() != 1) return false;
         std::atomic_thread_fence(std::memory_order_acquire);  // its last holder let go of it
-        hip_check(hipDeviceSynchronize(), "hipDeviceSynchronize");  // frames in flight may read it
+        return !o->kept;
+    }
+    bool release(std::vector<std::shared_ptr<Order>>::iterator o) {
+        if (o == orders.end()) return false;
+        if (hipDeviceSynchronize() != hipSuccess) {  // frames in flight may read it
+            (void)hipGetLastError();
+            return false;
+        }
         orders.erase(o);
+        return true;
     }
 
     // Gives back the order that `key` may take the place of, if there is one (mu held).
@@ -331,11 +348,9 @@ struct RangeOrders {
         if (known == refusals.end()) return false;
         auto oldest = orders.end();
         for (auto o = orders.begin(); o != orders.end(); ++o)
-            if (o->use_count() == 1 && (*o)->used < known->at && (oldest == orders.end() || (*o)->used < (*oldest)->used))
-                oldest = o;
-        if (oldest == orders.end()) return false;
+            if (free(*o) && (*o)->used < known->at && (oldest == orders.end() || (*o)->used < (*oldest)->used)) oldest = o;
+        if (!release(oldest)) return false;
         refusals.erase(known);
-        release(oldest);
         return true;
     }
 };
@@ -2287,9 +2302,12 @@ struct bcsim_sim {
             hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
         };
         RangeOrders& orders = t.fixed->by_range;
+        const bool captured = capturing(stream);  // a graph may replay this frame later: none is made or replaced
+        if (captured) create = false;
         if (create && order_room && !orders.has(key, !phase_delay)) create = order_room(RangeOrders::bytes(t.n));
         const RangeOrders::Ref o = orders.get(key, !phase_delay, t.n, create ? &sort : nullptr, order_account);
         if (!o) return R;
+        if (captured) o->kept = true;
         order_refs.push_back(o);
         R.patches = d_patches.as<RangePatch>();
         R.start = o->start;

@@ -56,12 +56,19 @@ extern "C" hipError_t hipMemcpy(void* dst, const void* src, size_t n, hipMemcpyK
     return mock_hipMemcpy(dst, src, n, kind);
 }
 
+static bool under_capture = false;
+extern "C" hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* status) {
+    *status = under_capture ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
+    return hipSuccess;
+}
+
 static bool live(const void* p) {
     hipPointerAttribute_t a;
     return p && hipPointerGetAttributes(&a, p) == hipSuccess;
 }
 
 static int range_launches = 0;  // projections in range order
+static const void* last_records = nullptr;  // of the last one
 static float table_value = 0.0f;  // what every sample of the profile's table is
 
 namespace bcsim_hip {
@@ -75,6 +82,7 @@ hipError_t launch_project_tile(const ProjCommon& c, const CullParams& cp, const 
         if (R.sort) REQUIRE(live(R.count) && live(R.rank));
         if (R.sort != 2) {
             range_launches++;
+            last_records = R.recs;
             REQUIRE(live(R.patches) && R.n_patches > 0);
             if (lut) {
                 REQUIRE(live(R.table));
@@ -337,6 +345,55 @@ static void origins() {
     hipFree(out);
 }
 
+// Orders that captured frames name: a graph of them can be replayed whatever scans came since.
+static void captured_frames() {
+    const size_t n = 20000;
+    for (bool noalloc : {true, false}) {
+        bcsim_sim* s = simulator(64, n);
+        count_bytes = n * sizeof(RangeRec) + (2 * kRangeBins + 4 + n) * sizeof(int);
+        const auto at = [&](float x) {
+            set_scan(s, sector(64, x));
+            return ranged(s);
+        };
+        int nl = 0, ns = 0;
+        CHK(bcsim_get_output_shape(s, &nl, &ns));
+        void *out = nullptr, *stream = nullptr;
+        REQUIRE(hipMalloc(&out, (size_t)nl * ns * 8) == hipSuccess);
+        CHK(bcsim_get_stream(s, &stream));
+        const hipStream_t st = static_cast<hipStream_t>(stream);
+        const auto capture = [&] {
+            hipGraph_t g = nullptr;
+            hipGraphExec_t e = nullptr;
+            under_capture = true;
+            REQUIRE(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal) == hipSuccess);
+            CHK((noalloc ? bcsim_simulate_lines_device_noalloc : bcsim_simulate_lines_device)(s, out, (size_t)nl * ns, &nl, &ns));
+            REQUIRE(hipStreamEndCapture(st, &g) == hipSuccess);
+            under_capture = false;
+            REQUIRE(hipGraphInstantiate(&e, g, nullptr, nullptr, 0) == hipSuccess);
+            REQUIRE(hipGraphDestroy(g) == hipSuccess);
+            return e;
+        };
+        REQUIRE(at(0.0f));
+        const hipGraphExec_t first = capture();
+        const void* records = last_records;
+        // four more origins that stay: three orders, then the one longest unused of those three
+        for (float x : {0.001f, 0.002f, 0.003f}) REQUIRE(at(x));
+        REQUIRE(!at(0.004f) && at(0.004f) && !at(0.005f) && at(0.005f) && !at(0.006f) && at(0.006f));
+        // one that is seen again under capture waits for nothing and allocates nothing
+        REQUIRE(!at(0.007f));
+        mallocs = range_launches = 0;
+        const hipGraphExec_t fifth = capture();
+        REQUIRE(mallocs == 0 && range_launches == 0);
+        // the captured one is there still, and the same
+        REQUIRE(live(records) && at(0.0f) && mallocs == 0 && last_records == records);
+        REQUIRE(hipGraphLaunch(first, st) == hipSuccess && hipGraphLaunch(fifth, st) == hipSuccess);
+        CHK(bcsim_synchronize(s));
+        REQUIRE(hipGraphExecDestroy(first) == hipSuccess && hipGraphExecDestroy(fifth) == hipSuccess);
+        CHK(bcsim_destroy(s));
+        hipFree(out);
+    }
+}
+
 // A server counts the orders and the samples of its tables, sorts none that its budget has no
 // room for, and gives one back for a request that needs the room.
 static void server_budget() {
@@ -501,6 +558,7 @@ int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     const std::vector<std::pair<std::string, void (*)()>> all = {
         {"table_failures", table_failures}, {"optional_buffers", optional_buffers}, {"crowds", crowds}, {"origins", origins},
+        {"captured_frames", captured_frames},
         {"server_budget", server_budget}, {"tuned_radix", tuned_radix},
         {"tuned_shapes_by_origin", tuned_shapes_by_origin}, {"tuned_order", tuned_order},
         {"batch_shapes", batch_shapes}};

@@ -33,8 +33,8 @@ def driver(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["table_failures", "optional_buffers", "crowds", "origins", "server_budget", "tuned_radix", "tuned_shapes_by_origin",
-                                      "tuned_order", "batch_shapes"])
+@pytest.mark.parametrize("scenario", ["table_failures", "optional_buffers", "crowds", "origins", "captured_frames",
+                                      "server_budget", "tuned_radix", "tuned_shapes_by_origin", "tuned_order", "batch_shapes"])
 def test_memory(driver, scenario):
     res = subprocess.run([driver, scenario], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=300,
                          env=dict(os.environ, MOCK_DELAY_US="20"))
